@@ -1,0 +1,673 @@
+// Matrix-core GEMM over operands that were split once into 16-bit planes: the
+// large f32 products of training (the policy's forward, data and weight
+// gradients, the linear head + cross-entropy, the MoE expert projections).
+//
+// f32-grade form. A row of op(A) (a column of op(B)) is scaled by a power of two
+// that puts its largest magnitude into [2^14, 2^15) and written as two f16
+// planes, x 2^s = hi + lo: 22 significant bits for every element within 2^-18
+// of its row's largest, and an absolute error of 2^-39 of that largest for
+// the rest. A product is lo.hi + hi.lo + hi.hi in f32 (v_mfma_f32_32x32x16_f16,
+// smallest first; lo.lo is below 2^-22), the scales are undone by one exact
+// ldexp per output. Three MFMAs per f32 product against the six of three
+// bf16 planes, and half as many f32 additions, which is where such a product's
+// error comes from: over K 512 to 32768 its distance to float64 is no larger
+// (measured beside each caller). Values of at most 11 bits (a 4-bit code times a
+// bf16 scale) need one plane: two MFMAs.
+// kBf16 form: bf16 operands, one MFMA.
+//
+// Layout of a split operand: per row, lines of 128 bytes: 64 k of one plane, or
+// 32 k of hi and then of lo. A stage of the K loop (one line of a pair) then
+// reads whole lines.
+//
+// gemm_pairs_kernel: a BM x BN tile per workgroup, 8 waves (4 for 128 x 128), 2
+// waves per SIMD; two LDS stages filled by global_load_lds (16 bytes a lane, no registers): the next
+// stage's copies are issued right after the barrier and land during the
+// current one's MFMAs. 16-byte chunk c of row r lies at c ^ f(r), f chosen so
+// that the 32-row fragment reads spread over all banks; the copy permutes its
+// global addresses instead, as its LDS side is always consecutive.
+#include "gemm_pairs.hpp"
+
+#include <algorithm>
+#include <type_traits>
+
+#include "common.hpp"
+
+namespace sm {
+namespace {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kCUs = 256;
+
+// The power of two that a row of largest magnitude `bits` is scaled by:
+// 2^(14 - floor(log2)); 1 for a zero row and for one with an infinity or a NaN
+// (whose outputs are NaN either way).
+__host__ __device__ inline int scale_shift(uint32_t bits) {
+  if (bits == 0 || bits >= 0x7f800000u) return 0;
+  const int e = (int)(bits >> 23);
+  if (e > 0) return 14 - (e - 127);
+  return 14 - (31 - __builtin_clz(bits) - 149);  // denormal: by its leading bit
+}
+
+// ------------------------------------------------------------------ split --
+
+// 8 consecutive values -> one 16-byte chunk per plane
+template <Split F>
+__device__ inline void split8(const float* v, int shift, u32x4& hi, u32x4& lo) {
+  if constexpr (F == Split::kBf16) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) hi[i] = pack_bf16x2(v[2 * i], v[2 * i + 1]);
+  } else {
+    h8 h, l;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float x = ldexpf(v[i], shift);
+      const _Float16 a = (_Float16)x;
+      h[i] = a;
+      l[i] = (_Float16)(x - (float)a);
+    }
+    hi = __builtin_bit_cast(u32x4, h);
+    lo = __builtin_bit_cast(u32x4, l);
+  }
+}
+
+// byte offset of the chunk of k (a multiple of 8) in a row
+template <Split F>
+__device__ inline int64_t chunk_offset(int64_t k) {
+  return F == Split::kPair ? (k / 32) * 128 + (k % 32) * 2 : k * 2;
+}
+
+template <Split F>
+__device__ inline void store8(char* row, int64_t k, const float* v, int shift) {
+  u32x4 hi, lo;
+  split8<F>(v, shift, hi, lo);
+  char* p = row + chunk_offset<F>(k);
+  *reinterpret_cast<u32x4*>(p) = hi;
+  if constexpr (F == Split::kPair) *reinterpret_cast<u32x4*>(p + 64) = lo;
+}
+
+// k contiguous: T threads per row (one wave, or the workgroup for long rows),
+// 8 k per thread and step; the first 4 steps stay in registers between the
+// row's maximum and its conversion, later ones are read twice. HBM-bound:
+// 4 bytes read and 2 per plane written a value.
+template <Split F, int T>
+__global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ X, int64_t ld,
+                                                         int64_t R, int64_t K, int64_t Kp,
+                                                         char* __restrict__ out,
+                                                         int64_t row_bytes,
+                                                         uint32_t* __restrict__ amax, int vec) {
+  constexpr int NR = 4;
+  __shared__ float red[256 / kWave];
+  const int64_t r = (int64_t)blockIdx.x * (256 / T) + threadIdx.x / T;
+  const int t = threadIdx.x % T;
+  const bool live = r < R;
+  const float* x = X + (live ? r : 0) * ld;
+  auto load8 = [&](int64_t k, float* v) {
+    if (vec && k + 8 <= K) {
+      const f32x4 a = *reinterpret_cast<const f32x4*>(x + k);
+      const f32x4 b = *reinterpret_cast<const f32x4*>(x + k + 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[e] = a[e];
+        v[4 + e] = b[e];
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = k + e < K ? x[k + e] : 0.f;
+    }
+  };
+  float v[NR][8];
+  int shift = 0;
+  if (live) {
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      const int64_t k = 8 * (t + (int64_t)T * i);
+      if (k < Kp) load8(k, v[i]);
+    }
+  }
+  if constexpr (F != Split::kBf16) {
+    uint32_t m = 0;  // magnitudes as bits: NaN above infinity above all finite
+    if (live) {
+#pragma unroll
+      for (int i = 0; i < NR; ++i)
+        if (8 * (t + (int64_t)T * i) < Kp)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) m = max(m, __float_as_uint(v[i][e]) & 0x7fffffffu);
+      for (int64_t k = 8 * (t + (int64_t)T * NR); k < Kp; k += 8 * T) {
+        float w[8];
+        load8(k, w);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) m = max(m, __float_as_uint(w[e]) & 0x7fffffffu);
+      }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o, kWave));
+    if constexpr (T > kWave) {
+      if (threadIdx.x % kWave == 0) red[threadIdx.x / kWave] = __uint_as_float(m);
+      __syncthreads();
+#pragma unroll
+      for (int w = 0; w < 256 / kWave; ++w) m = max(m, __float_as_uint(red[w]));
+    }
+    if (live && t == 0) amax[r] = m;
+    shift = scale_shift(m);
+  }
+  if (!live) return;
+  char* row = out + r * row_bytes;
+#pragma unroll
+  for (int i = 0; i < NR; ++i) {
+    const int64_t k = 8 * (t + (int64_t)T * i);
+    if (k < Kp) store8<F>(row, k, v[i], shift);
+  }
+  for (int64_t k = 8 * (t + (int64_t)T * NR); k < Kp; k += 8 * T) {
+    float w[8];
+    load8(k, w);
+    store8<F>(row, k, w, shift);
+  }
+}
+
+__global__ __launch_bounds__(256) void zero_u32_kernel(uint32_t* __restrict__ p, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) p[i] = 0;
+}
+
+// column maxima of X [K][ld] over 64-row slices; the atomic max of magnitude
+// bits does not depend on the order
+__global__ __launch_bounds__(256) void col_amax_kernel(const float* __restrict__ X, int64_t ld,
+                                                       int64_t R, int64_t K,
+                                                       uint32_t* __restrict__ amax) {
+  const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (r >= R) return;
+  const int64_t k0 = (int64_t)blockIdx.y * 64, k1 = min(k0 + 64, K);
+  uint32_t m = 0;
+#pragma unroll 8
+  for (int64_t k = k0; k < k1; ++k) m = max(m, __float_as_uint(X[k * ld + r]) & 0x7fffffffu);
+  if (m) atomicMax(amax + r, m);
+}
+
+// k across rows: 64 k x 64 r tiles through LDS; reads are 64 consecutive r a
+// wave, writes 8 consecutive chunks (whole lines) of a row. With runs, 64-k
+// block b of the output is the next 64 k of its run (zeros past its end).
+template <Split F>
+__global__ __launch_bounds__(256) void split_cols_kernel(const float* __restrict__ X, int64_t ld,
+                                                         int64_t R, int64_t K,
+                                                         char* __restrict__ out,
+                                                         int64_t row_bytes,
+                                                         const uint32_t* __restrict__ amax,
+                                                         int use_runs, Runs runs) {
+  __shared__ float t[64][65];  // [k][r]
+  const int64_t kb = blockIdx.x, r0 = (int64_t)blockIdx.y * 64;
+  int64_t k0 = kb * 64, k1 = K;
+  if (use_runs) {
+    int64_t b = kb;
+    int e = 0;
+    while (b >= (runs.cnt[e] + 63) / 64) b -= (runs.cnt[e++] + 63) / 64;
+    k0 = runs.off[e] + b * 64;
+    k1 = runs.off[e] + runs.cnt[e];
+  }
+  const int tx = threadIdx.x % 64, ty = threadIdx.x / 64;
+#pragma unroll 4
+  for (int i = ty; i < 64; i += 4) {
+    const int64_t k = k0 + i, r = r0 + tx;
+    t[i][tx] = (k < k1 && r < R) ? X[k * ld + r] : 0.f;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int c = (int)threadIdx.x + 256 * h, rl = c / 8, kl = (c % 8) * 8;
+    if (r0 + rl >= R) continue;
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = t[kl + e][rl];
+    const int shift = F == Split::kBf16 ? 0 : scale_shift(amax[r0 + rl]);
+    store8<F>(out + (r0 + rl) * row_bytes, kb * 64 + kl, v, shift);
+  }
+}
+
+// ------------------------------------------------------------------- GEMM --
+
+struct PairArgs {
+  const char *A, *B;
+  int64_t rowA, rowB;  // bytes
+  int rowsA;
+  const uint32_t *amax, *bmax;
+  float* C;
+  int64_t ldc;
+  int M, N, nst;  // nst: K stages
+  float alpha, beta;
+  const float* bias;
+  int ntm, ntn, splits;
+  float* part;     // [splits][M][N] when splits > 1
+  int64_t stride;  // run forms: B rows (kRows) or C floats (kKs) per run
+  Runs runs;
+};
+enum Mode { kPlain, kRows, kKs };
+
+// Tile order: workgroups go to the 8 XCDs in turn, each XCD gets a consecutive
+// range of tiles, and within it four tile rows are walked column by column, so
+// that the tiles an XCD works on at once share operand rows in its L2.
+__device__ inline void tile_of(int id, int total, int ntm, int ntn, int& tm, int& tn) {
+  const int per = total / 8, rem = total % 8, x = id % 8, i = id / 8;
+  const int t = x * per + min(x, rem) + i;
+  constexpr int G = 4;
+  const int band = t / (G * ntn), m0 = band * G, gm = min(G, ntm - m0), in = t - band * G * ntn;
+  tm = m0 + in % gm;
+  tn = in / gm;
+}
+
+template <bool F16>
+__device__ inline f32x16 mfma(u32x4 a, u32x4 b, f32x16 c) {
+  if constexpr (F16)
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8, a),
+                                                  __builtin_bit_cast(h8, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
+                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+template <bool F16, int PA, int PB, int BM, int BN, int BK, int WM, int WN, Mode MODE>
+__global__ __launch_bounds__(WM * WN * 64, 2) void gemm_pairs_kernel(PairArgs g) {
+  static_assert((PA == 1 || BK == 32) && (PB == 1 || BK == 32), "");
+  constexpr int NW = WM * WN;
+  constexpr int CR = BK / 8;                           // chunks per row, plane and stage
+  constexpr int SA = PA * BM * CR, SB = PB * BN * CR;  // chunks per stage
+  constexpr int NA = SA / (64 * NW), NB = SB / (64 * NW);  // copies per wave
+  static_assert(SA % (64 * NW) == 0 && SB % (64 * NW) == 0, "");
+  constexpr int MB = BM / WM / 32, NBk = BN / WN / 32;  // 32 x 32 blocks per wave
+  constexpr int kStage = (SA + SB) * 16;
+  __shared__ __attribute__((aligned(16))) char lds[2 * kStage];
+  const int lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int wm = wave / WN, wn = wave % WN;
+
+  int tm, tn, z = 0, M = g.M, s0 = 0, s1 = g.nst, arow0 = 0;
+  const char* Bp = g.B;
+  const uint32_t* bmax = g.bmax;
+  float* C = g.C;
+  if constexpr (MODE == kPlain) {
+    const int per = g.ntm * g.ntn;
+    z = blockIdx.x / per;
+    tile_of(blockIdx.x % per, per, g.ntm, g.ntn, tm, tn);
+    if (g.splits > 1) {
+      s0 = (int)((int64_t)g.nst * z / g.splits);
+      s1 = (int)((int64_t)g.nst * (z + 1) / g.splits);
+    }
+  } else if constexpr (MODE == kRows) {
+    int t = blockIdx.x / g.ntn, e = 0;
+    while (t >= (g.runs.cnt[e] + BM - 1) / BM) t -= (g.runs.cnt[e++] + BM - 1) / BM;
+    tm = t;
+    tn = blockIdx.x % g.ntn;
+    M = g.runs.cnt[e];
+    arow0 = g.runs.off[e];
+    Bp += (int64_t)e * g.stride * g.rowB;
+    if (F16) bmax += (int64_t)e * g.stride;
+    C += (int64_t)arow0 * g.ldc;
+  } else {
+    const int per = g.ntm * g.ntn, e = blockIdx.x / per;
+    tm = blockIdx.x % per / g.ntn;
+    tn = blockIdx.x % per % g.ntn;
+    for (int i = 0; i < e; ++i) s0 += (g.runs.cnt[i] + 63) / 64 * (64 / BK);
+    s1 = s0 + (g.runs.cnt[e] + 63) / 64 * (64 / BK);
+    C += (int64_t)e * g.stride;
+  }
+  const int m0 = tm * BM, n0 = tn * BN;
+
+  // copy j of this wave: chunks (NW j + wave) 64 + lane of the stage, at a fixed
+  // offset from the tile's first row; the rows' bases advance with the stages
+  uint32_t src[NA + NB];
+  auto swz = [](int r) { return CR == 4 ? (r >> 2) & 3 : (r >> 1) & 7; };
+#pragma unroll
+  for (int j = 0; j < NA + NB; ++j) {
+    const bool isA = j < NA;
+    const int c = (NW * (isA ? j : j - NA) + wave) * 64 + lane;
+    const int rows = isA ? BM : BN;
+    const int p = c / (rows * CR), r = c / CR % rows, k = (c % CR) ^ swz(r);
+    const int rr = min(r, isA ? g.rowsA - arow0 - m0 - 1 : g.N - n0 - 1);  // rows past the end
+    src[j] = (uint32_t)rr * (uint32_t)(isA ? g.rowA : g.rowB) + p * (BK * 2) + k * 16;
+  }
+  const char* at = g.A + (int64_t)(arow0 + m0) * g.rowA + (int64_t)s0 * (BK * 2 * PA);
+  const char* bt = Bp + (int64_t)n0 * g.rowB + (int64_t)s0 * (BK * 2 * PB);
+  auto fetch = [&](int buf) {
+#if defined(__HIP_DEVICE_COMPILE__)  // (the host pass does not emit the launch stub otherwise)
+#pragma unroll
+    for (int j = 0; j < NA + NB; ++j) {
+      const int to = buf * kStage + (j < NA ? 0 : SA * 16) +
+                     (NW * (j < NA ? j : j - NA) + wave) * 1024;
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) char*)(j < NA ? at : bt) + src[j],
+          (__attribute__((address_space(3))) char*)lds + to, 16, 0, 0);
+    }
+#endif
+    at += BK * 2 * PA;
+    bt += BK * 2 * PB;
+  };
+
+  f32x16 acc[MB][NBk];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NBk; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+  // fragment of lane l: row l % 32 of the block, chunk 2 ks + l / 32
+  const int fr = lane % 32, fs = swz(fr);  // blocks start at multiples of 32
+  const int fa = (wm * (BM / WM) + fr) * CR * 16, fb = (wn * (BN / WN) + fr) * CR * 16;
+
+  if (s0 < s1) fetch(0);
+  for (int s = s0; s < s1; ++s) {
+    const int buf = (s - s0) & 1;
+    // this wave's copies of stage s have landed, and behind the barrier every
+    // wave's; every wave has also read all it needs of the other buffer
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (s + 1 < s1) fetch(buf ^ 1);
+    const char* As = lds + buf * kStage;
+    const char* Bs = As + SA * 16;
+    // the fragments of the next 16 k are read between the MFMAs of these
+    u32x4 a[2][PA][MB], b[2][PB][NBk];
+    auto frags = [&](int ks) {
+      const int co = ((2 * ks + lane / 32) ^ fs) * 16;
+#pragma unroll
+      for (int p = 0; p < PA; ++p)
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+          a[ks & 1][p][i] =
+              *reinterpret_cast<const u32x4*>(As + (p * BM + i * 32) * CR * 16 + fa + co);
+#pragma unroll
+      for (int p = 0; p < PB; ++p)
+#pragma unroll
+        for (int i = 0; i < NBk; ++i)
+          b[ks & 1][p][i] =
+              *reinterpret_cast<const u32x4*>(Bs + (p * BN + i * 32) * CR * 16 + fb + co);
+    };
+    frags(0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ks = 0; ks < BK / 16; ++ks) {
+      if (ks + 1 < BK / 16) frags(ks + 1);
+      // lo.hi, hi.lo, hi.hi
+#pragma unroll
+      for (int q = 0; q < PA + PB - 1; ++q) {
+        const int pa = (PA == 2 && q == 0) ? 1 : 0;
+        const int pb = (PB == 2 && q == 1) ? 1 : 0;
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+          for (int j = 0; j < NBk; ++j)
+            acc[i][j] = mfma<F16>(a[ks & 1][pa][i], b[ks & 1][pb][j], acc[i][j]);
+      }
+      if (ks + 1 < BK / 16) {
+        constexpr int nr = PA * MB + PB * NBk, nm = (PA + PB - 1) * MB * NBk;
+#pragma unroll
+        for (int r = 0; r < nr; ++r) {
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one LDS read
+          __builtin_amdgcn_sched_group_barrier(0x008, nm / nr > 0 ? nm / nr : 1, 0);  // MFMAs
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, nm, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+
+  // acc[i][j][e]: row 8 (e / 4) + 4 (lane / 32) + e % 4, column lane % 32
+  auto emit = [&](auto whole) {  // whole: no row or column of the tile is past the end
+#pragma unroll
+    for (int i = 0; i < MB; ++i) {
+      const int rb = m0 + wm * (BM / WM) + i * 32 + 4 * (lane / 32);
+      int sa[16];
+      if constexpr (F16) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int row = rb + 8 * (e / 4) + e % 4;
+          sa[e] = scale_shift(g.amax[arow0 + (whole ? row : min(row, M - 1))]);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < NBk; ++j) {
+        const int col = n0 + wn * (BN / WN) + j * 32 + fr;
+        if (!whole && col >= g.N) continue;
+        const int sb = F16 ? scale_shift(bmax[col]) : 0;
+        const float bias = g.bias ? g.bias[col] : 0.f;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int row = rb + 8 * (e / 4) + e % 4;
+          if (!whole && row >= M) continue;
+          const float v = F16 ? ldexpf(acc[i][j][e], -(sa[e] + sb)) : acc[i][j][e];
+          if (MODE == kPlain && g.splits > 1) {
+            g.part[((int64_t)z * M + row) * g.N + col] = v;
+            continue;
+          }
+          float* o = C + (int64_t)row * g.ldc + col;
+          const float w = g.beta == 0.f ? g.alpha * v : fmaf(g.alpha, v, g.beta * *o);
+          *o = g.bias ? w + bias : w;
+        }
+      }
+    }
+  };
+  if (m0 + BM <= M && n0 + BN <= g.N) emit(std::true_type{});
+  else emit(std::false_type{});
+}
+
+// C = alpha sum_z part[z] + beta C (+ bias), z in order
+__global__ __launch_bounds__(256) void pairs_reduce_kernel(const float* __restrict__ part,
+                                                           int splits, int64_t M, int64_t N,
+                                                           float alpha, float beta,
+                                                           const float* __restrict__ bias,
+                                                           float* __restrict__ C, int64_t ldc) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= M * N) return;
+  float v = part[i];
+  for (int z = 1; z < splits; ++z) v += part[z * M * N + i];
+  float* o = C + i / N * ldc + i % N;
+  const float w = beta == 0.f ? alpha * v : fmaf(alpha, v, beta * *o);
+  *o = bias ? w + bias[i % N] : w;
+}
+
+// ---------------------------------------------------------------- dispatch --
+
+template <Mode MODE, int BM, int BN, int WM, int WN>
+int launch(const SplitOperand& A, const SplitOperand& B, PairArgs& g, int64_t wgs,
+           hipStream_t st) {
+  if (wgs == 0) return SM_OK;
+  SM_REQUIRE(wgs * 512 < ((int64_t)1 << 32) && pairs_fit(A.kp) && A.kp == B.kp,
+             "gemm_pairs: shape out of range");
+#define SM_GP(F16, PA, PB, BK) \
+  gemm_pairs_kernel<F16, PA, PB, BM, BN, BK, WM, WN, MODE>  \
+      <<<(unsigned)wgs, WM * WN * 64, 0, st>>>(g)
+  if (A.form == Split::kBf16) {
+    g.nst = (int)(A.kp / 64);
+    SM_GP(false, 1, 1, 64);
+  } else {
+    g.nst = (int)(A.kp / 32);
+    if (B.form == Split::kPair) SM_GP(true, 2, 2, 32);
+    else SM_GP(true, 2, 1, 32);
+  }
+#undef SM_GP
+  SM_LAUNCH_CHECK();
+  return SM_OK;
+}
+
+PairArgs pair_args(const SplitOperand& A, const SplitOperand& B) {
+  PairArgs g{};
+  g.A = A.data;
+  g.B = B.data;
+  g.rowA = A.row_bytes();
+  g.rowB = B.row_bytes();
+  g.rowsA = (int)A.rows;
+  g.amax = A.amax;
+  g.bmax = B.amax;
+  g.alpha = 1.f;
+  g.splits = 1;
+  return g;
+}
+
+// The tile and the K splits of an M x N x K product: rounds of workgroups over
+// the chip times the time of a round, ns per k measured at full rounds (`ns`;
+// 1.05-1.2 PF/s of MFMA work, set by power rather than by the tile), less where
+// a round leaves CUs idle (0.6 of it for the large tiles with few busy, half for
+// the 128 x 128 ones, two of which share a CU). A split writes and reads its
+// partial sums. Three products, us: 8192 x 8192 x 4096 256 x 256 1378, 128 x 256
+// 1493, 128 x 128 1558; 2048 x 2048 x 8184 500, 288, 208 (256 x 256 in 4 splits
+// 197); 1024 x 768 x 32768 128 x 256 in 10 splits 159, 256 x 256 in 8 259, in 21
+// 167. One bf16 product: 4096 x 2048 x 65536 1598, 1350, 1112.
+struct Tile {
+  int bm, bn, slots;  // slots: workgroups the chip runs at once
+  double ns[3];       // bf16, pair x f16, pair x pair
+};
+constexpr Tile kTiles[] = {{256, 256, kCUs, {34, 57, 85}},
+                           {128, 256, kCUs, {20, 30.5, 46}},
+                           {128, 128, 2 * kCUs, {18.5, 33, 47.5}}};
+struct Plan {
+  int tile, splits;
+};
+Plan pair_plan(Split a, Split b, int64_t M, int64_t N, int64_t K) {
+  const int form = a == Split::kBf16 ? 0 : b == Split::kF16 ? 1 : 2;
+  Plan best{0, 1};
+  double least = 0;
+  for (int i = 0; i < 3; ++i) {
+    const Tile& t = kTiles[i];
+    const int64_t tiles = ceil_div(M, t.bm) * ceil_div(N, t.bn);
+    for (int s = 1; s <= 32; ++s) {
+      // (bf16 operands: one accumulation chain per output)
+      if (s > 1 && (form == 0 || K / s < 512 || tiles * s > 4 * t.slots)) break;
+      const double rounds = (double)ceil_div(tiles * s, t.slots);
+      const double full = tiles * s / (rounds * t.slots);
+      const double part = t.slots > kCUs ? std::max(0.53, 0.1 + 0.9 * full) : 0.6 + 0.4 * full;
+      const double ns = rounds * ((double)K / s * t.ns[form] * part + 4000) +
+                        (s > 1 ? (double)s * M * N * 8 / 4000 + 5000 : 0);
+      if (least == 0 || ns < 0.98 * least) {
+        least = ns;
+        best = {i, s};
+      }
+    }
+  }
+  return best;
+}
+
+}  // namespace
+
+bool pairs_fit(int64_t K) { return K <= ((int64_t)1 << 21); }
+
+int64_t split_bytes(Split form, int64_t rows, int64_t K) {
+  const SplitOperand o = split_place(form, rows, K, nullptr);
+  const int64_t data = ceil_div(rows * o.row_bytes(), 256) * 256;
+  return data + (form == Split::kBf16 ? 0 : ceil_div(rows * 4, 256) * 256);
+}
+
+SplitOperand split_place(Split form, int64_t rows, int64_t K, void* buf) {
+  SplitOperand o{form, static_cast<char*>(buf), nullptr, rows, ceil_div(K, 64) * 64};
+  if (form != Split::kBf16)
+    o.amax = reinterpret_cast<uint32_t*>(o.data + ceil_div(rows * o.row_bytes(), 256) * 256);
+  return o;
+}
+
+int64_t runs_kp(const Runs& r) {
+  int64_t n = 0;
+  for (int i = 0; i < r.n; ++i) n += (r.cnt[i] + 63) / 64 * 64;
+  return n;
+}
+
+namespace {
+template <Split F>
+int split_fill(const SplitOperand& o, const float* X, int64_t ld, bool kc, int64_t K,
+               hipStream_t st, const Runs* runs) {
+  const int64_t R = o.rows, rb = o.row_bytes();
+  if (kc) {
+    const int vec = ld % 4 == 0 && reinterpret_cast<uintptr_t>(X) % 16 == 0;
+    if (o.kp <= 2048)
+      split_rows_kernel<F, 64><<<(unsigned)ceil_div(R, 4), 256, 0, st>>>(X, ld, R, K, o.kp,
+                                                                         o.data, rb, o.amax, vec);
+    else
+      split_rows_kernel<F, 256><<<(unsigned)R, 256, 0, st>>>(X, ld, R, K, o.kp, o.data, rb,
+                                                             o.amax, vec);
+  } else {
+    if (F != Split::kBf16) {
+      zero_u32_kernel<<<(unsigned)ceil_div(R, 256), 256, 0, st>>>(o.amax, R);
+      const dim3 grid((unsigned)ceil_div(R, 256), (unsigned)ceil_div(K, 64));
+      col_amax_kernel<<<grid, 256, 0, st>>>(X, ld, R, K, o.amax);
+    }
+    const dim3 grid((unsigned)(o.kp / 64), (unsigned)ceil_div(R, 64));
+    split_cols_kernel<F><<<grid, 256, 0, st>>>(X, ld, R, K, o.data, rb, o.amax,
+                                               runs ? 1 : 0, runs ? *runs : Runs{});
+  }
+  SM_LAUNCH_CHECK();
+  return SM_OK;
+}
+}  // namespace
+
+int split_operand(const SplitOperand& o, const float* X, int64_t ld, bool kc, int64_t K,
+                  hipStream_t st, const Runs* runs) {
+  if (o.rows == 0 || o.kp == 0) return SM_OK;
+  switch (o.form) {
+    case Split::kBf16: return split_fill<Split::kBf16>(o, X, ld, kc, K, st, runs);
+    case Split::kF16: return split_fill<Split::kF16>(o, X, ld, kc, K, st, runs);
+    default: return split_fill<Split::kPair>(o, X, ld, kc, K, st, runs);
+  }
+}
+
+int64_t gemm_pairs_part_floats(Split a, Split b, int64_t M, int64_t N, int64_t K) {
+  const Plan p = pair_plan(a, b, M, N, ceil_div(K, 64) * 64);  // as gemm_pairs sees it
+  return p.splits == 1 ? 0 : p.splits * M * N;
+}
+
+int gemm_pairs(const SplitOperand& A, const SplitOperand& B, int64_t M, int64_t N, float alpha,
+               float beta, const float* bias, float* C, int64_t ldc, float* part,
+               int64_t part_floats, hipStream_t st) {
+  if (M == 0 || N == 0) return SM_OK;
+  PairArgs g = pair_args(A, B);
+  Plan p = pair_plan(A.form, B.form, M, N, A.kp);
+  if (!part || p.splits * M * N > part_floats) p.splits = 1;
+  g.C = C;
+  g.ldc = ldc;
+  g.M = (int)M;
+  g.N = (int)N;
+  g.alpha = alpha;
+  g.beta = beta;
+  g.bias = bias;
+  g.splits = p.splits;
+  g.part = part;
+  g.ntm = (int)ceil_div(M, kTiles[p.tile].bm);
+  g.ntn = (int)ceil_div(N, kTiles[p.tile].bn);
+  const int64_t wgs = (int64_t)g.ntm * g.ntn * p.splits;
+  if (p.tile == 0) SM_TRY((launch<kPlain, 256, 256, 2, 4>(A, B, g, wgs, st)));
+  else if (p.tile == 1) SM_TRY((launch<kPlain, 128, 256, 2, 4>(A, B, g, wgs, st)));
+  else SM_TRY((launch<kPlain, 128, 128, 2, 2>(A, B, g, wgs, st)));
+  if (p.splits > 1) {
+    pairs_reduce_kernel<<<(unsigned)ceil_div(M * N, 256), 256, 0, st>>>(part, p.splits, M, N, alpha,
+                                                                        beta, bias, C, ldc);
+    SM_LAUNCH_CHECK();
+  }
+  return SM_OK;
+}
+
+int gemm_pairs_rows(const SplitOperand& A, const SplitOperand& B, int64_t bstride, int64_t N,
+                    const Runs& runs, float* C, int64_t ldc, hipStream_t st) {
+  PairArgs g = pair_args(A, B);
+  g.C = C;
+  g.ldc = ldc;
+  g.N = (int)N;
+  g.stride = bstride;
+  g.runs = runs;
+  g.ntn = (int)ceil_div(N, 256);
+  int64_t tiles = 0;
+  for (int i = 0; i < runs.n; ++i) tiles += ceil_div(runs.cnt[i], 128);
+  return launch<kRows, 128, 256, 2, 4>(A, B, g, tiles * g.ntn, st);
+}
+
+int gemm_pairs_ks(const SplitOperand& A, const SplitOperand& B, int64_t M, int64_t N,
+                  const Runs& runs, float* C, int64_t ldc, int64_t cstride, hipStream_t st) {
+  PairArgs g = pair_args(A, B);
+  g.C = C;
+  g.ldc = ldc;
+  g.M = (int)M;
+  g.N = (int)N;
+  g.stride = cstride;
+  g.runs = runs;
+  g.ntm = (int)ceil_div(M, 128);
+  g.ntn = (int)ceil_div(N, 256);
+  return launch<kKs, 128, 256, 2, 4>(A, B, g, (int64_t)runs.n * g.ntm * g.ntn, st);
+}
+
+}  // namespace sm

@@ -1,0 +1,68 @@
+// Internal interface of the pre-split matrix-core GEMM (gemm_pairs.hip).
+#pragma once
+
+#include <cstddef>
+#include <cstdint>
+
+#include <hip/hip_runtime.h>
+
+namespace sm {
+
+// How a split operand holds its values.
+// kBf16: rounded to bf16, one plane (the one-plane policy's operands).
+// kF16: one f16 plane of x 2^s, s from the row's largest magnitude: exact for
+//   values of at most 11 significant bits (a 4-bit code times a bf16 scale).
+// kPair: x 2^s = hi + lo, two f16 planes, about 22 significant bits.
+enum class Split { kBf16, kF16, kPair };
+
+// Consecutive runs of the grouped forms: run i covers `cnt[i]` rows (or k)
+// from `off[i]` of the dense operand.
+constexpr int kMaxRuns = 64;
+struct Runs {
+  int n;
+  int off[kMaxRuns], cnt[kMaxRuns];
+};
+
+// op(X) of `rows` rows and K columns in split form, k padded with zeros to whole
+// 64s. `data` and the row maxima live in the caller's buffer of split_bytes()
+// (16-byte aligned).
+struct SplitOperand {
+  Split form;
+  char* data;
+  uint32_t* amax;  // bits of each row's largest |x| (not kBf16)
+  int64_t rows, kp;
+  int64_t row_bytes() const { return kp * (form == Split::kPair ? 4 : 2); }
+};
+int64_t split_bytes(Split form, int64_t rows, int64_t K);
+SplitOperand split_place(Split form, int64_t rows, int64_t K, void* buf);
+
+// Whether K is in the kernel's range (a tile's rows lie within 4 GB).
+bool pairs_fit(int64_t K);
+
+// Fills `o` from X: element (r, k) at X[r * ld + k] (kc) or X[k * ld + r]. With
+// `runs` (not kc), run i's k go to the columns from runs_kp() on, each run
+// padded with zeros to whole 64-k blocks.
+int split_operand(const SplitOperand& o, const float* X, int64_t ld, bool kc, int64_t K,
+                  hipStream_t st, const Runs* runs = nullptr);
+// Columns a run-padded operand needs: the sum of cnt rounded up to 64.
+int64_t runs_kp(const Runs& r);
+
+// C = alpha A B^T + beta C (+ bias along n) from split operands; A and B are
+// both kBf16, or A is kPair and B kPair or kF16.
+// part (nullable): room for split-K partial sums, part_floats floats; without
+// it, or where it is too small, K is not split.
+int gemm_pairs(const SplitOperand& A, const SplitOperand& B, int64_t M, int64_t N, float alpha,
+               float beta, const float* bias, float* C, int64_t ldc, float* part,
+               int64_t part_floats, hipStream_t st);
+// Floats of `part` that let gemm_pairs split K as it would choose to.
+int64_t gemm_pairs_part_floats(Split a, Split b, int64_t M, int64_t N, int64_t K);
+// Rows of A in runs, run e against B[e] (`bstride` rows of B apart, N used):
+// C rows off[e] .. = A rows off[e] .. times B_e^T.
+int gemm_pairs_rows(const SplitOperand& A, const SplitOperand& B, int64_t bstride, int64_t N,
+                    const Runs& runs, float* C, int64_t ldc, hipStream_t st);
+// k in runs: C_e (`cstride` floats apart) = A[:, run e] B[:, run e]^T, zero for
+// an empty run.
+int gemm_pairs_ks(const SplitOperand& A, const SplitOperand& B, int64_t M, int64_t N,
+                  const Runs& runs, float* C, int64_t ldc, int64_t cstride, hipStream_t st);
+
+}  // namespace sm

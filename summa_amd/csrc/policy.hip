@@ -83,6 +83,8 @@ int gemm_ex_planes(int planes, int trans_a, int trans_b, int64_t M, int64_t N, i
                    float alpha, const float* A, int64_t lda, const float* B, int64_t ldb,
                    float beta, float* C, int64_t ldc, void* stream, float* scratch = nullptr,
                    int64_t scratch_floats = 0, int b_planes = 3);  // train.hip
+int64_t gemm_presplit_scratch_floats(int planes, bool weight_b, int64_t M, int64_t N,
+                                     int64_t K);  // gemm_mfma.hip
 int64_t gemm_planes_scratch_floats(bool ta, bool tb, int64_t M, int64_t N,
                                    int64_t K);  // gemm_mfma.hip
 int64_t rmsnorm_dgamma_chunks(int64_t rows);                          // train.hip
@@ -572,9 +574,9 @@ int policy_prepare(sm_policy* p, sm_model* reference, const float* ref_lp_in,
   hipStream_t st = as_stream(stream);
   const int64_t d = c.d_model, H = c.heads, KVH = c.kv_heads, hd = c.head_dim, F = c.ffn;
   const int64_t V = c.vocab, qn = p->qn, qdim = p->qdim;
-  // the prepare's GEMMs on the policy's plane count, with room for their
-  // transposed operands (tps: the largest need of the backward's (1, 0) and
-  // (0, 0) products below)
+  // the prepare's GEMMs on the policy's plane count, with room for their split
+  // (two planes: transposed) operands (tps: the largest need of the products
+  // below)
   float* tps = nullptr;
   int64_t tps_floats = 0;
   auto pgemm = [&](int ta, int tb, int64_t m, int64_t n, int64_t k, float alpha, const float* A,
@@ -584,8 +586,8 @@ int policy_prepare(sm_policy* p, sm_model* reference, const float* ref_lp_in,
                           tps, tps_floats, 3);
   };
   // the same with B a weight the forward uses: a quantized policy's are its
-  // fake-quantized copies (a bf16 scale times a 4-bit code), exact in two bf16
-  // planes, so three-plane products skip B's zero third plane (same bits)
+  // fake-quantized copies (a bf16 scale times a 4-bit code), exact in one f16
+  // plane, so f32-grade products skip B's second one
   const int wb_planes = c.quantized ? 2 : 3;
   auto wgemm = [&](int ta, int tb, int64_t m, int64_t n, int64_t k, float alpha, const float* A,
                    int64_t lda, const float* B, int64_t ldb, float beta, float* C, int64_t ldc,
@@ -605,18 +607,20 @@ int policy_prepare(sm_policy* p, sm_model* reference, const float* ref_lp_in,
   const int64_t ffn_fixed = moe ? RT * d /*dyr*/ + 2 * M /*gw*/ + RT * Fe /*dar*/ +
                                       RT * 2 * Fe /*dur*/ + RT * d /*drt*/ + M * E /*dlog*/ + 1
                                 : M * 2 * F /*du*/ + M * F /*da*/;
-  // transposed operands of the backward's weight (1, 0) and data (0, 0) GEMMs
-  auto tneed = [](bool ta, bool tb, int64_t m, int64_t n, int64_t k) {
-    return gemm_planes_scratch_floats(ta, tb, m, n, k);
+  // forward (0, 1), data-gradient (0, 0) and weight-gradient (1, 0) products of
+  // a projection of m rows, `out` x `in`
+  auto tneed = [&](int64_t m, int64_t out, int64_t in) {
+    if (p->planes == 2)
+      return std::max(gemm_planes_scratch_floats(true, false, out, in, m),
+                      gemm_planes_scratch_floats(false, false, m, in, out));
+    return std::max({gemm_presplit_scratch_floats(p->planes, c.quantized, m, out, in),
+                     gemm_presplit_scratch_floats(p->planes, c.quantized, m, in, out),
+                     gemm_presplit_scratch_floats(p->planes, false, out, in, m)});
   };
-  int64_t tp_need = std::max(tneed(true, false, V, d, R), tneed(false, false, R, d, V));
+  int64_t tp_need = tneed(R, V, d);
   const int64_t lin[4][2] = {{qn, d}, {d, qdim}, {2 * F, d}, {d, F}};  // {out, in}
-  for (int i = 0; i < (moe ? 2 : 4); ++i)
-    tp_need = std::max({tp_need, tneed(true, false, lin[i][0], lin[i][1], M),
-                        tneed(false, false, M, lin[i][1], lin[i][0])});
-  if (moe)
-    tp_need = std::max({tp_need, tneed(true, false, d, Fe, RT), tneed(false, false, RT, Fe, d),
-                        tneed(true, false, 2 * Fe, d, RT), tneed(false, false, RT, d, 2 * Fe)});
+  for (int i = 0; i < (moe ? 2 : 4); ++i) tp_need = std::max(tp_need, tneed(M, lin[i][0], lin[i][1]));
+  if (moe) tp_need = std::max({tp_need, tneed(RT, d, Fe), tneed(RT, 2 * Fe, d)});
   const int64_t per_layer =
       M * (d + d + qn + qdim + 2 * p->kvdim + qdim + H + d + d) + ffn_layer;
   const int64_t fixed = M * d /*x*/ + M * d /*hf*/ + R * d /*hr*/ + R * V /*logits*/ +
