@@ -335,44 +335,18 @@ int64_t gemm_planes_scratch_floats(bool ta, bool tb, int64_t M, int64_t N, int64
 }
 
 namespace {
-// operand forms of a product at `planes` (3: f32 grade, 1: bf16 operands)
-Split a_form(int planes) { return planes == 1 ? Split::kBf16 : Split::kPair; }
-Split b_form(int planes, bool weight_b) {
-  return planes == 3 && weight_b ? Split::kF16 : a_form(planes);
+// operand forms of a product of `planes` bf16 planes (b_planes 2: B exact in two)
+Split a_form(int planes) {
+  return planes == 1 ? Split::kBf16 : planes == 2 ? Split::kBf16x2 : Split::kBf16x3;
+}
+Split b_form(int planes, int b_planes) {
+  return planes == 3 && b_planes == 2 ? Split::kBf16x2 : a_form(planes);
 }
 }  // namespace
 
-// Floats of scratch with which gemm_presplit runs a product at its best.
-int64_t gemm_presplit_scratch_floats(int planes, bool weight_b, int64_t M, int64_t N, int64_t K) {
-  const Split fa = a_form(planes), fb = b_form(planes, weight_b);
-  return (split_bytes(fa, M, K) + split_bytes(fb, N, K)) / 4 +
-         gemm_pairs_part_floats(fa, fb, M, N, K);
-}
-
-// gemm_planes for a caller that takes any f32-grade (planes 3) or
-// bf16-operand (planes 1) product, whatever its summation order: operands split
-// once (gemm_pairs.hip), K split where the tiles are few and the scratch has room.
-// weight_b: B's values have at most 11 significant bits. Returns false, with
-// nothing launched, when the scratch cannot hold the operands or planes is 2
-// (whose products are defined by the plane arithmetic).
-bool gemm_presplit(int planes, bool weight_b, bool ta, bool tb, int64_t M, int64_t N, int64_t K,
-                   float alpha, const float* A, int64_t lda, const float* B, int64_t ldb,
-                   float beta, float* C, int64_t ldc, hipStream_t st, float* scratch,
-                   int64_t scratch_floats, int* status) {
-  if (planes == 2 || !pairs_fit(K) || !scratch || reinterpret_cast<uintptr_t>(scratch) % 16 != 0)
-    return false;
-  const Split fa = a_form(planes), fb = b_form(planes, weight_b);
-  const int64_t na = split_bytes(fa, M, K), nb = split_bytes(fb, N, K);
-  if (na + nb > scratch_floats * 4) return false;
-  char* at = reinterpret_cast<char*>(scratch);
-  const SplitOperand a = split_place(fa, M, K, at), b = split_place(fb, N, K, at + na);
-  int s = split_operand(a, A, lda, !ta, K, st);
-  if (s == SM_OK) s = split_operand(b, B, ldb, tb, K, st);
-  if (s == SM_OK)
-    s = gemm_pairs(a, b, M, N, alpha, beta, nullptr, C, ldc,
-                   reinterpret_cast<float*>(at + na + nb), scratch_floats - (na + nb) / 4, st);
-  *status = s;
-  return true;
+// Bytes of scratch with which gemm_planes splits the operands first.
+int64_t gemm_presplit_scratch_bytes(int planes, int b_planes, int64_t M, int64_t N, int64_t K) {
+  return split_bytes(a_form(planes), M, K) + split_bytes(b_form(planes, b_planes), N, K);
 }
 
 int gemm_planes(int planes, bool ta, bool tb, int64_t M, int64_t N, int64_t K, float alpha,
@@ -380,18 +354,20 @@ int gemm_planes(int planes, bool ta, bool tb, int64_t M, int64_t N, int64_t K, f
                 int64_t ldc, hipStream_t st, float* scratch, int64_t scratch_floats,
                 int b_planes) {
   const bool al16 = scratch && reinterpret_cast<uintptr_t>(scratch) % 16 == 0;
-  // One plane, with room for both operands' bf16 copies: each is converted
-  // once (transposed on the way where its k is not contiguous) and the K loop
-  // only copies them into LDS: the same values and, unsplit, the same MFMA
-  // order, so the same bits. FFN-in forward (8184 x 11264 x 2048) 780 us with the
-  // in-loop conversion, 435 with 128 x 128 tiles staged through registers, 414
-  // with gemm_pairs' tiles; LM head data gradient (4096 x 2048 x 65536) 3.9 -> 1.27
-  // -> 1.11 ms.
-  if (planes == 1 && al16 && pairs_fit(K) && split_scratch_floats(M, N, K) <= scratch_floats) {
-    const SplitOperand a = split_place(Split::kBf16, M, K, scratch);
-    const SplitOperand b = split_place(Split::kBf16, N, K,
-                                       reinterpret_cast<char*>(scratch) +
-                                           split_bytes(Split::kBf16, M, K));
+  // With room for both operands in split form each is converted once
+  // (transposed on the way where its k is not contiguous) and the K loop only
+  // copies the planes into LDS: the same values and MFMA order, so the same
+  // bits. One plane: FFN-in forward (8184 x 11264 x 2048) 780 us with the in-loop
+  // conversion, 435 with 128 x 128 tiles staged through registers, 414 with
+  // gemm_pairs' tiles; LM head data gradient (4096 x 2048 x 65536) 3.9 -> 1.27 ->
+  // 1.11 ms. Three planes (B exact in two): LM head forward (4096 x 65536 x 2048)
+  // 5.25 -> 4.10 ms, 8184 x 11264 x 2048 1.56 -> 1.37.
+  const int64_t split = gemm_presplit_scratch_bytes(planes, b_planes, M, N, K);
+  if (al16 && pairs_fit(K) && split <= scratch_floats * 4) {
+    const Split fa = a_form(planes), fb = b_form(planes, b_planes);
+    const SplitOperand a = split_place(fa, M, K, scratch);
+    const SplitOperand b = split_place(fb, N, K,
+                                       reinterpret_cast<char*>(scratch) + split_bytes(fa, M, K));
     SM_TRY(split_operand(a, A, lda, !ta, K, st));
     SM_TRY(split_operand(b, B, ldb, tb, K, st));
     return gemm_pairs(a, b, M, N, alpha, beta, nullptr, C, ldc, nullptr, 0, st);

@@ -13,11 +13,13 @@
 // error comes from: over K 512 to 32768 its distance to float64 is no larger
 // (measured beside each caller). Values of at most 11 bits (a 4-bit code times a
 // bf16 scale) need one plane: two MFMAs.
-// kBf16 form: bf16 operands, one MFMA.
+// bf16 forms: one, two or three unscaled bf16 planes, the plane products of
+// gemm_mfma.hip in its order (the same bits) with the split taken out of the K
+// loop.
 //
-// Layout of a split operand: per row, lines of 128 bytes: 64 k of one plane, or
-// 32 k of hi and then of lo. A stage of the K loop (one line of a pair) then
-// reads whole lines.
+// Layout of a split operand: per row, one plane: its k in order; more: per 32 k
+// the planes' 64 bytes one after the other. A stage of the K loop then reads
+// whole lines.
 //
 // gemm_pairs_kernel: a BM x BN tile per workgroup, 8 waves (4 for 128 x 128), 2
 // waves per SIMD; two LDS stages filled by global_load_lds (16 bytes a lane, no registers): the next
@@ -53,39 +55,36 @@ __host__ __device__ inline int scale_shift(uint32_t bits) {
 
 // ------------------------------------------------------------------ split --
 
-// 8 consecutive values -> one 16-byte chunk per plane
+// 8 consecutive values of a row at k (a multiple of 8) -> 16 bytes per plane
 template <Split F>
-__device__ inline void split8(const float* v, int shift, u32x4& hi, u32x4& lo) {
-  if constexpr (F == Split::kBf16) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) hi[i] = pack_bf16x2(v[2 * i], v[2 * i + 1]);
-  } else {
+__device__ inline void store8(char* row, int64_t k, const float* v, int shift) {
+  constexpr int P = F == Split::kBf16x3 ? 3 : F == Split::kPair || F == Split::kBf16x2 ? 2 : 1;
+  u32x4 w[P];
+  if constexpr (F == Split::kF16 || F == Split::kPair) {
     h8 h, l;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const float x = ldexpf(v[i], shift);
-      const _Float16 a = (_Float16)x;
-      h[i] = a;
-      l[i] = (_Float16)(x - (float)a);
+      h[i] = (_Float16)x;
+      l[i] = (_Float16)(x - (float)h[i]);
     }
-    hi = __builtin_bit_cast(u32x4, h);
-    lo = __builtin_bit_cast(u32x4, l);
+    w[0] = __builtin_bit_cast(u32x4, h);
+    if constexpr (P > 1) w[1] = __builtin_bit_cast(u32x4, l);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float a = v[2 * i], b = v[2 * i + 1];
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        w[p][i] = pack_bf16x2(a, b);
+        a -= bf16lo(w[p][i]);
+        b -= bf16hi(w[p][i]);
+      }
+    }
   }
-}
-
-// byte offset of the chunk of k (a multiple of 8) in a row
-template <Split F>
-__device__ inline int64_t chunk_offset(int64_t k) {
-  return F == Split::kPair ? (k / 32) * 128 + (k % 32) * 2 : k * 2;
-}
-
-template <Split F>
-__device__ inline void store8(char* row, int64_t k, const float* v, int shift) {
-  u32x4 hi, lo;
-  split8<F>(v, shift, hi, lo);
-  char* p = row + chunk_offset<F>(k);
-  *reinterpret_cast<u32x4*>(p) = hi;
-  if constexpr (F == Split::kPair) *reinterpret_cast<u32x4*>(p + 64) = lo;
+  char* o = row + (P == 1 ? k * 2 : k / 32 * (64 * P) + k % 32 * 2);
+#pragma unroll
+  for (int p = 0; p < P; ++p) *reinterpret_cast<u32x4*>(o + 64 * p) = w[p];
 }
 
 // k contiguous: T threads per row (one wave, or the workgroup for long rows),
@@ -127,7 +126,7 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict
       if (k < Kp) load8(k, v[i]);
     }
   }
-  if constexpr (F != Split::kBf16) {
+  if constexpr (F == Split::kF16 || F == Split::kPair) {
     uint32_t m = 0;  // magnitudes as bits: NaN above infinity above all finite
     if (live) {
 #pragma unroll
@@ -220,7 +219,7 @@ __global__ __launch_bounds__(256) void split_cols_kernel(const float* __restrict
     float v[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = t[kl + e][rl];
-    const int shift = F == Split::kBf16 ? 0 : scale_shift(amax[r0 + rl]);
+    const int shift = (F == Split::kF16 || F == Split::kPair) ? scale_shift(amax[r0 + rl]) : 0;
     store8<F>(out + (r0 + rl) * row_bytes, kb * 64 + kl, v, shift);
   }
 }
@@ -255,6 +254,20 @@ __device__ inline void tile_of(int id, int total, int ntm, int ntn, int& tm, int
   tm = m0 + in % gm;
   tn = in / gm;
 }
+
+// plane pairs (a, b) of each product, smallest weight first
+template <int PA, int PB> struct Products;
+template <> struct Products<3, 3> {
+  static constexpr int n = 6, a[6] = {2, 1, 0, 1, 0, 0}, b[6] = {0, 1, 2, 0, 1, 0};
+};
+template <> struct Products<3, 2> {
+  static constexpr int n = 5, a[5] = {2, 1, 1, 0, 0}, b[5] = {0, 1, 0, 1, 0};
+};
+template <> struct Products<2, 2> {
+  static constexpr int n = 3, a[3] = {1, 0, 0}, b[3] = {0, 1, 0};
+};
+template <> struct Products<2, 1> { static constexpr int n = 2, a[2] = {1, 0}, b[2] = {0, 0}; };
+template <> struct Products<1, 1> { static constexpr int n = 1, a[1] = {0}, b[1] = {0}; };
 
 template <bool F16>
 __device__ inline f32x16 mfma(u32x4 a, u32x4 b, f32x16 c) {
@@ -387,19 +400,16 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_pairs_kernel(PairArgs g)
 #pragma unroll
     for (int ks = 0; ks < BK / 16; ++ks) {
       if (ks + 1 < BK / 16) frags(ks + 1);
-      // lo.hi, hi.lo, hi.hi
+      using Pr = Products<PA, PB>;
 #pragma unroll
-      for (int q = 0; q < PA + PB - 1; ++q) {
-        const int pa = (PA == 2 && q == 0) ? 1 : 0;
-        const int pb = (PB == 2 && q == 1) ? 1 : 0;
+      for (int q = 0; q < Pr::n; ++q)
 #pragma unroll
         for (int i = 0; i < MB; ++i)
 #pragma unroll
           for (int j = 0; j < NBk; ++j)
-            acc[i][j] = mfma<F16>(a[ks & 1][pa][i], b[ks & 1][pb][j], acc[i][j]);
-      }
+            acc[i][j] = mfma<F16>(a[ks & 1][Pr::a[q]][i], b[ks & 1][Pr::b[q]][j], acc[i][j]);
       if (ks + 1 < BK / 16) {
-        constexpr int nr = PA * MB + PB * NBk, nm = (PA + PB - 1) * MB * NBk;
+        constexpr int nr = PA * MB + PB * NBk, nm = Pr::n * MB * NBk;
 #pragma unroll
         for (int r = 0; r < nr; ++r) {
           __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one LDS read
@@ -467,6 +477,7 @@ __global__ __launch_bounds__(256) void pairs_reduce_kernel(const float* __restri
 
 // ---------------------------------------------------------------- dispatch --
 
+// (the grouped modes take f16 pairs only)
 template <Mode MODE, int BM, int BN, int WM, int WN>
 int launch(const SplitOperand& A, const SplitOperand& B, PairArgs& g, int64_t wgs,
            hipStream_t st) {
@@ -476,14 +487,17 @@ int launch(const SplitOperand& A, const SplitOperand& B, PairArgs& g, int64_t wg
 #define SM_GP(F16, PA, PB, BK) \
   gemm_pairs_kernel<F16, PA, PB, BM, BN, BK, WM, WN, MODE>  \
       <<<(unsigned)wgs, WM * WN * 64, 0, st>>>(g)
-  if (A.form == Split::kBf16) {
-    g.nst = (int)(A.kp / 64);
-    SM_GP(false, 1, 1, 64);
-  } else {
-    g.nst = (int)(A.kp / 32);
-    if (B.form == Split::kPair) SM_GP(true, 2, 2, 32);
-    else SM_GP(true, 2, 1, 32);
+  g.nst = (int)(A.kp / (A.form == Split::kBf16 ? 64 : 32));
+  if constexpr (BM * BN <= 256 * 128) {  // (three planes of a larger tile overflow LDS)
+    if (A.form == Split::kBf16x3) {
+      if (B.form == Split::kBf16x3) SM_GP(false, 3, 3, 32);
+      else SM_GP(false, 3, 2, 32);
+    }
   }
+  if (A.form == Split::kBf16x2) SM_GP(false, 2, 2, 32);
+  else if (A.form == Split::kBf16) SM_GP(false, 1, 1, 64);
+  else if (A.form == Split::kPair && B.form == Split::kPair) SM_GP(true, 2, 2, 32);
+  else if (A.form == Split::kPair) SM_GP(true, 2, 1, 32);
 #undef SM_GP
   SM_LAUNCH_CHECK();
   return SM_OK;
@@ -514,7 +528,7 @@ PairArgs pair_args(const SplitOperand& A, const SplitOperand& B) {
 // 167. One bf16 product: 4096 x 2048 x 65536 1598, 1350, 1112.
 struct Tile {
   int bm, bn, slots;  // slots: workgroups the chip runs at once
-  double ns[3];       // bf16, pair x f16, pair x pair
+  double ns[3];       // 1, 2 and 3 products; more in proportion
 };
 constexpr Tile kTiles[] = {{256, 256, kCUs, {34, 57, 85}},
                            {128, 256, kCUs, {20, 30.5, 46}},
@@ -523,19 +537,23 @@ struct Plan {
   int tile, splits;
 };
 Plan pair_plan(Split a, Split b, int64_t M, int64_t N, int64_t K) {
+  const bool three = a == Split::kBf16x3;
   const int form = a == Split::kBf16 ? 0 : b == Split::kF16 ? 1 : 2;
+  const double products = !three ? 1.0 : b == Split::kBf16x3 ? 2.0 : 5.0 / 3.0;
   Plan best{0, 1};
   double least = 0;
-  for (int i = 0; i < 3; ++i) {
+  for (int i = three ? 1 : 0; i < 3; ++i) {
     const Tile& t = kTiles[i];
     const int64_t tiles = ceil_div(M, t.bm) * ceil_div(N, t.bn);
+    const int slots = three ? kCUs : t.slots;  // (three planes: one workgroup's LDS per CU)
+    const double half = t.slots / slots;
     for (int s = 1; s <= 32; ++s) {
-      // (bf16 operands: one accumulation chain per output)
-      if (s > 1 && (form == 0 || K / s < 512 || tiles * s > 4 * t.slots)) break;
-      const double rounds = (double)ceil_div(tiles * s, t.slots);
-      const double full = tiles * s / (rounds * t.slots);
-      const double part = t.slots > kCUs ? std::max(0.53, 0.1 + 0.9 * full) : 0.6 + 0.4 * full;
-      const double ns = rounds * ((double)K / s * t.ns[form] * part + 4000) +
+      // (bf16 planes: one accumulation chain per output, as in gemm_mfma.hip)
+      if (s > 1 && (!scaled(a) || K / s < 512 || tiles * s > 4 * slots)) break;
+      const double rounds = (double)ceil_div(tiles * s, slots);
+      const double full = tiles * s / (rounds * slots);
+      const double part = slots > kCUs ? std::max(0.53, 0.1 + 0.9 * full) : 0.6 + 0.4 * full;
+      const double ns = rounds * ((double)K / s * t.ns[form] * products / half * part + 4000) +
                         (s > 1 ? (double)s * M * N * 8 / 4000 + 5000 : 0);
       if (least == 0 || ns < 0.98 * least) {
         least = ns;
@@ -553,12 +571,12 @@ bool pairs_fit(int64_t K) { return K <= ((int64_t)1 << 21); }
 int64_t split_bytes(Split form, int64_t rows, int64_t K) {
   const SplitOperand o = split_place(form, rows, K, nullptr);
   const int64_t data = ceil_div(rows * o.row_bytes(), 256) * 256;
-  return data + (form == Split::kBf16 ? 0 : ceil_div(rows * 4, 256) * 256);
+  return data + (scaled(form) ? ceil_div(rows * 4, 256) * 256 : 0);
 }
 
 SplitOperand split_place(Split form, int64_t rows, int64_t K, void* buf) {
   SplitOperand o{form, static_cast<char*>(buf), nullptr, rows, ceil_div(K, 64) * 64};
-  if (form != Split::kBf16)
+  if (scaled(form))
     o.amax = reinterpret_cast<uint32_t*>(o.data + ceil_div(rows * o.row_bytes(), 256) * 256);
   return o;
 }
@@ -583,7 +601,7 @@ int split_fill(const SplitOperand& o, const float* X, int64_t ld, bool kc, int64
       split_rows_kernel<F, 256><<<(unsigned)R, 256, 0, st>>>(X, ld, R, K, o.kp, o.data, rb,
                                                              o.amax, vec);
   } else {
-    if (F != Split::kBf16) {
+    if (scaled(F)) {
       zero_u32_kernel<<<(unsigned)ceil_div(R, 256), 256, 0, st>>>(o.amax, R);
       const dim3 grid((unsigned)ceil_div(R, 256), (unsigned)ceil_div(K, 64));
       col_amax_kernel<<<grid, 256, 0, st>>>(X, ld, R, K, o.amax);
@@ -603,6 +621,8 @@ int split_operand(const SplitOperand& o, const float* X, int64_t ld, bool kc, in
   switch (o.form) {
     case Split::kBf16: return split_fill<Split::kBf16>(o, X, ld, kc, K, st, runs);
     case Split::kF16: return split_fill<Split::kF16>(o, X, ld, kc, K, st, runs);
+    case Split::kBf16x2: return split_fill<Split::kBf16x2>(o, X, ld, kc, K, st, runs);
+    case Split::kBf16x3: return split_fill<Split::kBf16x3>(o, X, ld, kc, K, st, runs);
     default: return split_fill<Split::kPair>(o, X, ld, kc, K, st, runs);
   }
 }

@@ -13,7 +13,12 @@ namespace sm {
 // kF16: one f16 plane of x 2^s, s from the row's largest magnitude: exact for
 //   values of at most 11 significant bits (a 4-bit code times a bf16 scale).
 // kPair: x 2^s = hi + lo, two f16 planes, about 22 significant bits.
-enum class Split { kBf16, kF16, kPair };
+// kBf16x2, kBf16x3: the leading two or three bf16 planes of x (three: exact).
+enum class Split { kBf16, kF16, kPair, kBf16x2, kBf16x3 };
+inline int planes_of(Split f) {
+  return f == Split::kBf16x3 ? 3 : f == Split::kPair || f == Split::kBf16x2 ? 2 : 1;
+}
+inline bool scaled(Split f) { return f == Split::kF16 || f == Split::kPair; }
 
 // Consecutive runs of the grouped forms: run i covers `cnt[i]` rows (or k)
 // from `off[i]` of the dense operand.
@@ -29,9 +34,9 @@ struct Runs {
 struct SplitOperand {
   Split form;
   char* data;
-  uint32_t* amax;  // bits of each row's largest |x| (not kBf16)
+  uint32_t* amax;  // bits of each row's largest |x| (the scaled forms)
   int64_t rows, kp;
-  int64_t row_bytes() const { return kp * (form == Split::kPair ? 4 : 2); }
+  int64_t row_bytes() const { return kp * 2 * planes_of(form); }
 };
 int64_t split_bytes(Split form, int64_t rows, int64_t K);
 SplitOperand split_place(Split form, int64_t rows, int64_t K, void* buf);
@@ -47,8 +52,8 @@ int split_operand(const SplitOperand& o, const float* X, int64_t ld, bool kc, in
 // Columns a run-padded operand needs: the sum of cnt rounded up to 64.
 int64_t runs_kp(const Runs& r);
 
-// C = alpha A B^T + beta C (+ bias along n) from split operands; A and B are
-// both kBf16, or A is kPair and B kPair or kF16.
+// C = alpha A B^T + beta C (+ bias along n) from split operands: kPair with kPair
+// or kF16, kBf16 with itself, kBf16x2 with itself, kBf16x3 with itself or kBf16x2.
 // part (nullable): room for split-K partial sums, part_floats floats; without
 // it, or where it is too small, K is not split.
 int gemm_pairs(const SplitOperand& A, const SplitOperand& B, int64_t M, int64_t N, float alpha,

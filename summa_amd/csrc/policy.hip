@@ -83,10 +83,8 @@ int gemm_ex_planes(int planes, int trans_a, int trans_b, int64_t M, int64_t N, i
                    float alpha, const float* A, int64_t lda, const float* B, int64_t ldb,
                    float beta, float* C, int64_t ldc, void* stream, float* scratch = nullptr,
                    int64_t scratch_floats = 0, int b_planes = 3);  // train.hip
-int64_t gemm_presplit_scratch_floats(int planes, bool weight_b, int64_t M, int64_t N,
-                                     int64_t K);  // gemm_mfma.hip
-int64_t gemm_planes_scratch_floats(bool ta, bool tb, int64_t M, int64_t N,
-                                   int64_t K);  // gemm_mfma.hip
+int64_t gemm_presplit_scratch_bytes(int planes, int b_planes, int64_t M, int64_t N,
+                                    int64_t K);  // gemm_mfma.hip
 int64_t rmsnorm_dgamma_chunks(int64_t rows);                          // train.hip
 int rmsnorm_backward_parts(const float* x, const float* gamma, const float* dy, int64_t rows,
                            int64_t d, float eps, int accumulate, float* dx, float* dgamma,
@@ -574,9 +572,8 @@ int policy_prepare(sm_policy* p, sm_model* reference, const float* ref_lp_in,
   hipStream_t st = as_stream(stream);
   const int64_t d = c.d_model, H = c.heads, KVH = c.kv_heads, hd = c.head_dim, F = c.ffn;
   const int64_t V = c.vocab, qn = p->qn, qdim = p->qdim;
-  // the prepare's GEMMs on the policy's plane count, with room for their split
-  // (two planes: transposed) operands (tps: the largest need of the products
-  // below)
+  // the prepare's GEMMs on the policy's plane count, with room for their operands
+  // in split form (tps: the largest need of the products below)
   float* tps = nullptr;
   int64_t tps_floats = 0;
   auto pgemm = [&](int ta, int tb, int64_t m, int64_t n, int64_t k, float alpha, const float* A,
@@ -586,8 +583,8 @@ int policy_prepare(sm_policy* p, sm_model* reference, const float* ref_lp_in,
                           tps, tps_floats, 3);
   };
   // the same with B a weight the forward uses: a quantized policy's are its
-  // fake-quantized copies (a bf16 scale times a 4-bit code), exact in one f16
-  // plane, so f32-grade products skip B's second one
+  // fake-quantized copies (a bf16 scale times a 4-bit code), exact in two bf16
+  // planes, so three-plane products skip B's zero third plane (same bits)
   const int wb_planes = c.quantized ? 2 : 3;
   auto wgemm = [&](int ta, int tb, int64_t m, int64_t n, int64_t k, float alpha, const float* A,
                    int64_t lda, const float* B, int64_t ldb, float beta, float* C, int64_t ldc,
@@ -610,12 +607,9 @@ int policy_prepare(sm_policy* p, sm_model* reference, const float* ref_lp_in,
   // forward (0, 1), data-gradient (0, 0) and weight-gradient (1, 0) products of
   // a projection of m rows, `out` x `in`
   auto tneed = [&](int64_t m, int64_t out, int64_t in) {
-    if (p->planes == 2)
-      return std::max(gemm_planes_scratch_floats(true, false, out, in, m),
-                      gemm_planes_scratch_floats(false, false, m, in, out));
-    return std::max({gemm_presplit_scratch_floats(p->planes, c.quantized, m, out, in),
-                     gemm_presplit_scratch_floats(p->planes, c.quantized, m, in, out),
-                     gemm_presplit_scratch_floats(p->planes, false, out, in, m)});
+    return std::max({gemm_presplit_scratch_bytes(p->planes, wb_planes, m, out, in),
+                     gemm_presplit_scratch_bytes(p->planes, wb_planes, m, in, out),
+                     gemm_presplit_scratch_bytes(p->planes, 3, out, in, m)}) / 4 + 1;
   };
   int64_t tp_need = tneed(R, V, d);
   const int64_t lin[4][2] = {{qn, d}, {d, qdim}, {2 * F, d}, {d, F}};  // {out, in}

@@ -605,18 +605,12 @@ int gemm_planes(int planes, bool ta, bool tb, int64_t M, int64_t N, int64_t K, f
                 const float* A, int64_t lda, const float* B, int64_t ldb, float beta, float* C,
                 int64_t ldc, hipStream_t st, float* scratch = nullptr,
                 int64_t scratch_floats = 0, int b_planes = 3);  // gemm_mfma.hip
-bool gemm_presplit(int planes, bool weight_b, bool ta, bool tb, int64_t M, int64_t N, int64_t K,
-                   float alpha, const float* A, int64_t lda, const float* B, int64_t ldb,
-                   float beta, float* C, int64_t ldc, hipStream_t st, float* scratch,
-                   int64_t scratch_floats, int* status);  // gemm_mfma.hip
-
-// sm_gemm_ex with the matrix-core launches at `planes` bf16 planes per operand
+// sm_gemm_ex with the matrix-core launches on `planes` bf16 planes per operand
 // (3: f32-grade; 2: 16-bit operands; 1: bf16 operands); the small problems
 // stay on the f32 FMA kernel. scratch (optional, 16-byte aligned): room for
-// the operands in split form (gemm_presplit_scratch_floats; products at 3 planes
-// then run on f16 pairs) or transposed (gemm_planes_scratch_floats).
-// b_planes 2: B is a fake-quantized weight, a bf16 scale times a 4-bit code:
-// exact in one f16 plane, and in two bf16 planes.
+// the matrix-core launch's operands in split form (gemm_presplit_scratch_bytes).
+// b_planes 2: B's values are exact in two bf16 planes (fake-quantized
+// weights), so three-plane products skip the zero third plane of B.
 int gemm_ex_planes(int planes, int trans_a, int trans_b, int64_t M, int64_t N, int64_t K,
                    float alpha, const float* A, int64_t lda, const float* B, int64_t ldb,
                    float beta, float* C, int64_t ldc, void* stream, float* scratch,
@@ -631,14 +625,9 @@ int gemm_ex_planes(int planes, int trans_a, int trans_b, int64_t M, int64_t N, i
   hipStream_t st = as_stream(stream);
   // large problems on the matrix cores (bf16 plane products, gemm_mfma.hip);
   // small ones, where a launch has few 128 x 128 tiles, here
-  if (K >= 32 && M * N >= (int64_t)128 * 128 * 16 && M * N * K >= ((int64_t)1 << 27)) {
-    int status = SM_OK;
-    if (gemm_presplit(planes, b_planes == 2, trans_a != 0, trans_b != 0, M, N, K, alpha, A, lda, B,
-                      ldb, beta, C, ldc, st, scratch, scratch_floats, &status))
-      return status;
+  if (K >= 32 && M * N >= (int64_t)128 * 128 * 16 && M * N * K >= ((int64_t)1 << 27))
     return gemm_planes(planes, trans_a != 0, trans_b != 0, M, N, K, alpha, A, lda, B, ldb, beta,
                        C, ldc, st, scratch, scratch_floats, b_planes);
-  }
   const dim3 grid((unsigned)ceil_div(N, 64), (unsigned)ceil_div(M, 64));
 #define SM_GX(TA, TB)                                                                        \
   gemm_ex_kernel<TA, TB><<<grid, 256, 0, st>>>(A, lda, B, ldb, C, ldc, (int)M, (int)N, (int)K, \
