@@ -519,7 +519,10 @@ int sm_swiglu_backward(const void* gate_value, const void* grad, int dtype, int6
  * Float-weight grouped expert projections and the route permutation at the
  * reference's dispatch seam (GroupedLinearBackend, grouped_linear.rs:23-60;
  * RowPermutationBackend, row_permute.rs:33-41). All f32, f32-grade products
- * (sm_gemm_ex per expert with rows, in expert order; no allocation).
+ * (sm_gemm_ex per expert with rows, in expert order; no allocation). The _ws
+ * forms take a 16-byte aligned workspace of the queried bytes (0: none is used)
+ * and run each projection as one launch over all experts; with a smaller one
+ * they are the plain forms.
  * counts: HOST array [experts] of the rows per expert, as
  *   grouped_linear_inner takes them (Vec<usize>); they must sum to routes.
  * sm_row_permute: out[i] = input[order[i]] over rows of `cols` elements
@@ -541,6 +544,31 @@ int sm_swiglu_backward(const void* gate_value, const void* grad, int dtype, int6
  *   (grouped_swiglu_mlp_backward, :801-826); scratch: routes * 3 * I floats. */
 int sm_row_permute(const void* input, int dtype, int64_t rows, int64_t cols,
                    const int32_t* order, void* out, void* stream);
+int64_t sm_grouped_linear_workspace_bytes(int64_t experts, int64_t routes, int64_t d_in,
+                                          int64_t d_out, int backward);
+int64_t sm_grouped_swiglu_mlp_workspace_bytes(int64_t experts, int64_t routes, int64_t d,
+                                              int64_t intermediate, int64_t d_out, int backward);
+int sm_grouped_linear_ws(const float* input, const float* weight, const int64_t* counts,
+                         int64_t experts, int64_t routes, int64_t d_in, int64_t d_out, float* out,
+                         void* workspace, int64_t workspace_bytes, void* stream);
+int sm_grouped_linear_backward_ws(const float* input, const float* weight, const float* grad,
+                                  const int64_t* counts, int64_t experts, int64_t routes,
+                                  int64_t d_in, int64_t d_out, float* grad_input,
+                                  float* grad_weight, void* workspace, int64_t workspace_bytes,
+                                  void* stream);
+int sm_grouped_swiglu_mlp_ws(const float* input, const float* in_weight,
+                             const float* down_weight, const int64_t* counts, int64_t experts,
+                             int64_t routes, int64_t d, int64_t intermediate, int64_t d_out,
+                             float* out, float* projected, float* hidden, void* workspace,
+                             int64_t workspace_bytes, void* stream);
+int sm_grouped_swiglu_mlp_backward_ws(const float* input, const float* in_weight,
+                                      const float* down_weight, const int64_t* counts,
+                                      int64_t experts, int64_t routes, int64_t d,
+                                      int64_t intermediate, int64_t d_out, const float* projected,
+                                      const float* hidden, const float* grad, float* grad_input,
+                                      float* grad_in_weight, float* grad_down_weight,
+                                      float* scratch, void* workspace, int64_t workspace_bytes,
+                                      void* stream);
 int sm_grouped_linear(const float* input, const float* weight, const int64_t* counts,
                       int64_t experts, int64_t routes, int64_t d_in, int64_t d_out, float* out,
                       void* stream);

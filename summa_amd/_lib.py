@@ -132,6 +132,15 @@ SIGNATURES: dict[str, tuple] = {
     "sm_rl_prepare": (i32, [vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, f64, f64, f64, i64,
                             vp, vp, vp, vp, vp, vp]),
     "sm_row_permute": (i32, [vp, i32, i64, i64, vp, vp, vp]),
+    "sm_grouped_linear_workspace_bytes": (i64, [i64, i64, i64, i64, i32]),
+    "sm_grouped_swiglu_mlp_workspace_bytes": (i64, [i64, i64, i64, i64, i64, i32]),
+    "sm_grouped_linear_ws": (i32, [vp, vp, vp, i64, i64, i64, i64, vp, vp, i64, vp]),
+    "sm_grouped_linear_backward_ws": (i32, [vp, vp, vp, vp, i64, i64, i64, i64, vp, vp, vp, i64,
+                                            vp]),
+    "sm_grouped_swiglu_mlp_ws": (i32, [vp, vp, vp, vp, i64, i64, i64, i64, i64, vp, vp, vp, vp,
+                                       i64, vp]),
+    "sm_grouped_swiglu_mlp_backward_ws": (i32, [vp, vp, vp, vp, i64, i64, i64, i64, i64, vp, vp,
+                                                vp, vp, vp, vp, vp, vp, i64, vp]),
     "sm_grouped_linear": (i32, [vp, vp, vp, i64, i64, i64, i64, vp, vp]),
     "sm_grouped_linear_backward": (i32, [vp, vp, vp, vp, i64, i64, i64, i64, vp, vp, vp]),
     "sm_grouped_swiglu_mlp": (i32, [vp, vp, vp, vp, i64, i64, i64, i64, i64, vp, vp, vp, vp]),

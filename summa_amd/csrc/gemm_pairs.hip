@@ -178,6 +178,8 @@ __global__ __launch_bounds__(256) void col_amax_kernel(const float* __restrict__
                                                        uint32_t* __restrict__ amax) {
   const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (r >= R) return;
+  X += blockIdx.z * K * ld;
+  amax += blockIdx.z * R;
   const int64_t k0 = (int64_t)blockIdx.y * 64, k1 = min(k0 + 64, K);
   uint32_t m = 0;
 #pragma unroll 8
@@ -197,6 +199,9 @@ __global__ __launch_bounds__(256) void split_cols_kernel(const float* __restrict
                                                          int use_runs, Runs runs) {
   __shared__ float t[64][65];  // [k][r]
   const int64_t kb = blockIdx.x, r0 = (int64_t)blockIdx.y * 64;
+  X += blockIdx.z * K * ld;
+  out += blockIdx.z * R * row_bytes;
+  amax += blockIdx.z * R;
   int64_t k0 = kb * 64, k1 = K;
   if (use_runs) {
     int64_t b = kb;
@@ -488,16 +493,20 @@ int launch(const SplitOperand& A, const SplitOperand& B, PairArgs& g, int64_t wg
   gemm_pairs_kernel<F16, PA, PB, BM, BN, BK, WM, WN, MODE>  \
       <<<(unsigned)wgs, WM * WN * 64, 0, st>>>(g)
   g.nst = (int)(A.kp / (A.form == Split::kBf16 ? 64 : 32));
-  if constexpr (BM * BN <= 256 * 128) {  // (three planes of a larger tile overflow LDS)
+  if constexpr (MODE != kPlain) {
+    SM_GP(true, 2, 2, 32);
+  } else if constexpr (BM * BN <= 256 * 128) {  // (three planes of a larger tile overflow LDS)
     if (A.form == Split::kBf16x3) {
       if (B.form == Split::kBf16x3) SM_GP(false, 3, 3, 32);
       else SM_GP(false, 3, 2, 32);
     }
   }
-  if (A.form == Split::kBf16x2) SM_GP(false, 2, 2, 32);
-  else if (A.form == Split::kBf16) SM_GP(false, 1, 1, 64);
-  else if (A.form == Split::kPair && B.form == Split::kPair) SM_GP(true, 2, 2, 32);
-  else if (A.form == Split::kPair) SM_GP(true, 2, 1, 32);
+  if constexpr (MODE == kPlain) {
+    if (A.form == Split::kBf16x2) SM_GP(false, 2, 2, 32);
+    else if (A.form == Split::kBf16) SM_GP(false, 1, 1, 64);
+    else if (A.form == Split::kPair && B.form == Split::kPair) SM_GP(true, 2, 2, 32);
+    else if (A.form == Split::kPair) SM_GP(true, 2, 1, 32);
+  }
 #undef SM_GP
   SM_LAUNCH_CHECK();
   return SM_OK;
@@ -581,17 +590,11 @@ SplitOperand split_place(Split form, int64_t rows, int64_t K, void* buf) {
   return o;
 }
 
-int64_t runs_kp(const Runs& r) {
-  int64_t n = 0;
-  for (int i = 0; i < r.n; ++i) n += (r.cnt[i] + 63) / 64 * 64;
-  return n;
-}
-
 namespace {
 template <Split F>
 int split_fill(const SplitOperand& o, const float* X, int64_t ld, bool kc, int64_t K,
-               hipStream_t st, const Runs* runs) {
-  const int64_t R = o.rows, rb = o.row_bytes();
+               hipStream_t st, const Runs* runs, int64_t batch) {
+  const int64_t R = o.rows / batch, rb = o.row_bytes();
   if (kc) {
     const int vec = ld % 4 == 0 && reinterpret_cast<uintptr_t>(X) % 16 == 0;
     if (o.kp <= 2048)
@@ -602,11 +605,11 @@ int split_fill(const SplitOperand& o, const float* X, int64_t ld, bool kc, int64
                                                              o.amax, vec);
   } else {
     if (scaled(F)) {
-      zero_u32_kernel<<<(unsigned)ceil_div(R, 256), 256, 0, st>>>(o.amax, R);
-      const dim3 grid((unsigned)ceil_div(R, 256), (unsigned)ceil_div(K, 64));
+      zero_u32_kernel<<<(unsigned)ceil_div(o.rows, 256), 256, 0, st>>>(o.amax, o.rows);
+      const dim3 grid((unsigned)ceil_div(R, 256), (unsigned)ceil_div(K, 64), (unsigned)batch);
       col_amax_kernel<<<grid, 256, 0, st>>>(X, ld, R, K, o.amax);
     }
-    const dim3 grid((unsigned)(o.kp / 64), (unsigned)ceil_div(R, 64));
+    const dim3 grid((unsigned)(o.kp / 64), (unsigned)ceil_div(R, 64), (unsigned)batch);
     split_cols_kernel<F><<<grid, 256, 0, st>>>(X, ld, R, K, o.data, rb, o.amax,
                                                runs ? 1 : 0, runs ? *runs : Runs{});
   }
@@ -616,14 +619,14 @@ int split_fill(const SplitOperand& o, const float* X, int64_t ld, bool kc, int64
 }  // namespace
 
 int split_operand(const SplitOperand& o, const float* X, int64_t ld, bool kc, int64_t K,
-                  hipStream_t st, const Runs* runs) {
+                  hipStream_t st, const Runs* runs, int64_t batch) {
   if (o.rows == 0 || o.kp == 0) return SM_OK;
   switch (o.form) {
-    case Split::kBf16: return split_fill<Split::kBf16>(o, X, ld, kc, K, st, runs);
-    case Split::kF16: return split_fill<Split::kF16>(o, X, ld, kc, K, st, runs);
-    case Split::kBf16x2: return split_fill<Split::kBf16x2>(o, X, ld, kc, K, st, runs);
-    case Split::kBf16x3: return split_fill<Split::kBf16x3>(o, X, ld, kc, K, st, runs);
-    default: return split_fill<Split::kPair>(o, X, ld, kc, K, st, runs);
+    case Split::kBf16: return split_fill<Split::kBf16>(o, X, ld, kc, K, st, runs, batch);
+    case Split::kF16: return split_fill<Split::kF16>(o, X, ld, kc, K, st, runs, batch);
+    case Split::kBf16x2: return split_fill<Split::kBf16x2>(o, X, ld, kc, K, st, runs, batch);
+    case Split::kBf16x3: return split_fill<Split::kBf16x3>(o, X, ld, kc, K, st, runs, batch);
+    default: return split_fill<Split::kPair>(o, X, ld, kc, K, st, runs, batch);
   }
 }
 
@@ -662,6 +665,11 @@ int gemm_pairs(const SplitOperand& A, const SplitOperand& B, int64_t M, int64_t 
   return SM_OK;
 }
 
+namespace {
+// The grouped forms' column tile: 256 from two rounds of workgroups on.
+bool wide_tiles(int64_t tm, int64_t N) { return tm * ceil_div(N, 256) >= 2 * kCUs; }
+}  // namespace
+
 int gemm_pairs_rows(const SplitOperand& A, const SplitOperand& B, int64_t bstride, int64_t N,
                     const Runs& runs, float* C, int64_t ldc, hipStream_t st) {
   PairArgs g = pair_args(A, B);
@@ -670,10 +678,12 @@ int gemm_pairs_rows(const SplitOperand& A, const SplitOperand& B, int64_t bstrid
   g.N = (int)N;
   g.stride = bstride;
   g.runs = runs;
-  g.ntn = (int)ceil_div(N, 256);
-  int64_t tiles = 0;
-  for (int i = 0; i < runs.n; ++i) tiles += ceil_div(runs.cnt[i], 128);
-  return launch<kRows, 128, 256, 2, 4>(A, B, g, tiles * g.ntn, st);
+  int64_t tm = 0;
+  for (int i = 0; i < runs.n; ++i) tm += ceil_div(runs.cnt[i], 128);
+  const bool wide = wide_tiles(tm, N);
+  g.ntn = (int)ceil_div(N, wide ? 256 : 128);
+  if (wide) return launch<kRows, 128, 256, 2, 4>(A, B, g, tm * g.ntn, st);
+  return launch<kRows, 128, 128, 2, 2>(A, B, g, tm * g.ntn, st);
 }
 
 int gemm_pairs_ks(const SplitOperand& A, const SplitOperand& B, int64_t M, int64_t N,
@@ -686,8 +696,11 @@ int gemm_pairs_ks(const SplitOperand& A, const SplitOperand& B, int64_t M, int64
   g.stride = cstride;
   g.runs = runs;
   g.ntm = (int)ceil_div(M, 128);
-  g.ntn = (int)ceil_div(N, 256);
-  return launch<kKs, 128, 256, 2, 4>(A, B, g, (int64_t)runs.n * g.ntm * g.ntn, st);
+  const bool wide = wide_tiles(g.ntm * runs.n, N);
+  g.ntn = (int)ceil_div(N, wide ? 256 : 128);
+  const int64_t wgs = (int64_t)runs.n * g.ntm * g.ntn;
+  if (wide) return launch<kKs, 128, 256, 2, 4>(A, B, g, wgs, st);
+  return launch<kKs, 128, 128, 2, 2>(A, B, g, wgs, st);
 }
 
 }  // namespace sm

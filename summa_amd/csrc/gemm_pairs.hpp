@@ -45,12 +45,11 @@ SplitOperand split_place(Split form, int64_t rows, int64_t K, void* buf);
 bool pairs_fit(int64_t K);
 
 // Fills `o` from X: element (r, k) at X[r * ld + k] (kc) or X[k * ld + r]. With
-// `runs` (not kc), run i's k go to the columns from runs_kp() on, each run
-// padded with zeros to whole 64-k blocks.
+// `runs` (not kc), the runs' k follow each other, each padded with zeros to whole
+// 64s (K: their sum). With `batch` > 1 (not kc), X holds that many matrices,
+// K * ld apart, whose rows / batch rows each follow each other.
 int split_operand(const SplitOperand& o, const float* X, int64_t ld, bool kc, int64_t K,
-                  hipStream_t st, const Runs* runs = nullptr);
-// Columns a run-padded operand needs: the sum of cnt rounded up to 64.
-int64_t runs_kp(const Runs& r);
+                  hipStream_t st, const Runs* runs = nullptr, int64_t batch = 1);
 
 // C = alpha A B^T + beta C (+ bias along n) from split operands: kPair with kPair
 // or kF16, kBf16 with itself, kBf16x2 with itself, kBf16x3 with itself or kBf16x2.

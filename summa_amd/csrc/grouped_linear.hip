@@ -17,10 +17,19 @@
 //     selection by the inverse permutation).
 // The counts are host values, as grouped_linear_inner takes them (Vec<usize>;
 // the CUDA path reads device counts back to the host before its grouped GEMM,
-// grouped_linear.rs:787). Each expert with rows is one f32-grade GEMM
-// (sm_gemm_ex: the three-plane bf16 matrix-core kernel from 2^27
-// multiply-adds, the f32 FMA kernel below), in expert order on the stream.
+// grouped_linear.rs:787).
+//
+// With a workspace (the _ws entries) a projection is one f32-grade launch over
+// all experts on operands split once into scaled f16 pairs (gemm_pairs.hip): a
+// launch per expert left the chip with one expert's few tiles at a time (24 to
+// 100 workgroups on 256 CUs; the weight gradients, K = an expert's rows, ran on
+// 24-48). 8192 tokens, top-2 of 8 experts, d 512, width 768, forward and
+// backward: 4.81 -> 0.96 ms. Without one, or for products under 2^25 multiply-adds
+// in all, each expert with rows is one sm_gemm_ex, in expert order.
+#include <algorithm>
+
 #include "common.hpp"
+#include "gemm_pairs.hpp"
 
 extern "C" {
 int sm_gemm_ex(int, int, int64_t, int64_t, int64_t, float, const float*, int64_t, const float*,
@@ -65,9 +74,77 @@ int check_counts(const int64_t* counts, int64_t experts, int64_t routes, const c
   return SM_OK;
 }
 
+// The workspace of a projection: the rows, the weights and, in the backward, the
+// two run-padded transposes, all as f16 pairs.
+struct GroupedWs {
+  void* p;
+  int64_t bytes;
+};
+
+bool grouped_split_sizes(int64_t routes, int64_t d_in, int64_t d_out, int64_t experts) {
+  return std::min(d_in, d_out) >= 32 && routes * d_in * d_out >= ((int64_t)1 << 25) &&
+         pairs_fit(d_in) && pairs_fit(d_out) && pairs_fit(routes + 64 * experts) &&
+         experts * std::max(d_in, d_out) < (1 << 30) && experts < (1 << 16);
+}
+
+int64_t forward_bytes(int64_t experts, int64_t routes, int64_t d_in, int64_t d_out) {
+  if (!grouped_split_sizes(routes, d_in, d_out, experts)) return 0;
+  return split_bytes(Split::kPair, routes, d_in) + split_bytes(Split::kPair, experts * d_out, d_in);
+}
+
+int64_t backward_bytes(int64_t experts, int64_t routes, int64_t d_in, int64_t d_out) {
+  if (!grouped_split_sizes(routes, d_in, d_out, experts)) return 0;
+  const int64_t kp = routes + 64 * experts;  // every run padded to whole 64s
+  return std::max(split_bytes(Split::kPair, routes, d_out) +
+                      split_bytes(Split::kPair, experts * d_in, d_out),
+                  split_bytes(Split::kPair, d_in, kp) + split_bytes(Split::kPair, d_out, kp));
+}
+
+bool use_split(const GroupedWs& ws, int64_t need) {
+  return ws.p && need > 0 && need <= ws.bytes && reinterpret_cast<uintptr_t>(ws.p) % 16 == 0;
+}
+
+// Experts e0 .. e0 + kMaxRuns - 1 as runs of the grouped rows.
+Runs runs_of(const int64_t* counts, int64_t experts, int64_t e0, int64_t off) {
+  Runs r{};
+  r.n = (int)std::min<int64_t>(kMaxRuns, experts - e0);
+  for (int i = 0; i < r.n; ++i) {
+    r.off[i] = (int)off;
+    r.cnt[i] = (int)counts[e0 + i];
+    off += counts[e0 + i];
+  }
+  return r;
+}
+
+// y = x B_e^T per expert, from split rows x and weights [E][n] split along k
+int grouped_rows(const SplitOperand& x, const SplitOperand& w, const int64_t* counts,
+                 int64_t experts, int64_t n, float* y, hipStream_t st) {
+  int64_t off = 0;
+  for (int64_t e0 = 0; e0 < experts; e0 += kMaxRuns) {
+    const Runs r = runs_of(counts, experts, e0, off);
+    SplitOperand b = w;
+    b.data += e0 * n * w.row_bytes();
+    b.amax += e0 * n;
+    SM_TRY(gemm_pairs_rows(x, b, n, n, r, y, n, st));
+    off = r.off[r.n - 1] + r.cnt[r.n - 1];
+  }
+  return SM_OK;
+}
+
 // y = x W_e per expert (x rows grouped by expert, W [E, d_in, d_out])
 int grouped_forward(const float* x, const float* w, const int64_t* counts, int64_t experts,
-                    int64_t d_in, int64_t d_out, float* y, void* stream) {
+                    int64_t routes, int64_t d_in, int64_t d_out, float* y, const GroupedWs& ws,
+                    void* stream) {
+  if (use_split(ws, forward_bytes(experts, routes, d_in, d_out))) {
+    hipStream_t st = as_stream(stream);
+    const SplitOperand a = split_place(Split::kPair, routes, d_in, ws.p);
+    const SplitOperand b =
+        split_place(Split::kPair, experts * d_out, d_in,
+                    static_cast<char*>(ws.p) + split_bytes(Split::kPair, routes, d_in));
+    SM_TRY(split_operand(a, x, d_in, true, d_in, st));
+    SM_TRY(split_operand(b, w, d_out, false, d_in, st, nullptr, experts));
+    return grouped_rows(a, b, counts, experts, d_out, y, st);
+  }
   int64_t off = 0;
   for (int64_t e = 0; e < experts; ++e) {
     const int64_t c = counts[e];
@@ -79,11 +156,52 @@ int grouped_forward(const float* x, const float* w, const int64_t* counts, int64
   return SM_OK;
 }
 
+// The same two gradients as one launch each.
+int grouped_backward_split(const float* x, const float* w, const float* grad,
+                           const int64_t* counts, int64_t experts, int64_t routes, int64_t d_in,
+                           int64_t d_out, float* grad_x, float* grad_w, void* ws,
+                           hipStream_t st) {
+  char* at = static_cast<char*>(ws);
+  if (grad_x) {
+    const SplitOperand g = split_place(Split::kPair, routes, d_out, at);
+    const SplitOperand b = split_place(Split::kPair, experts * d_in, d_out,
+                                       at + split_bytes(Split::kPair, routes, d_out));
+    SM_TRY(split_operand(g, grad, d_out, true, d_out, st));
+    SM_TRY(split_operand(b, w, d_out, true, d_out, st));
+    SM_TRY(grouped_rows(g, b, counts, experts, d_in, grad_x, st));
+  }
+  if (grad_w) {
+    int64_t off = 0;
+    for (int64_t e0 = 0; e0 < experts; e0 += kMaxRuns) {
+      const Runs r = runs_of(counts, experts, e0, off);
+      int64_t kp = 0;
+      for (int i = 0; i < r.n; ++i) kp += ceil_div(r.cnt[i], 64) * 64;
+      const SplitOperand a = split_place(Split::kPair, d_in, kp, at);
+      const SplitOperand b =
+          split_place(Split::kPair, d_out, kp, at + split_bytes(Split::kPair, d_in, kp));
+      // (the runs are consecutive rows of x: their maxima are taken over rows
+      // r.off[0] on, which the shifted base and K give)
+      const int64_t rows = r.off[r.n - 1] + r.cnt[r.n - 1] - r.off[0];
+      Runs local = r;
+      for (int i = 0; i < r.n; ++i) local.off[i] -= r.off[0];
+      SM_TRY(split_operand(a, x + off * d_in, d_in, false, rows, st, &local));
+      SM_TRY(split_operand(b, grad + off * d_out, d_out, false, rows, st, &local));
+      SM_TRY(gemm_pairs_ks(a, b, d_in, d_out, r, grad_w + e0 * d_in * d_out, d_out,
+                           d_in * d_out, st));
+      off += rows;
+    }
+  }
+  return SM_OK;
+}
+
 // grad_x = grad W_e^T; grad_w[e] = x_e^T grad_e (zero without rows)
 int grouped_backward(const float* x, const float* w, const float* grad, const int64_t* counts,
-                     int64_t experts, int64_t d_in, int64_t d_out, float* grad_x, float* grad_w,
-                     void* stream) {
+                     int64_t experts, int64_t routes, int64_t d_in, int64_t d_out, float* grad_x,
+                     float* grad_w, const GroupedWs& ws, void* stream) {
   hipStream_t st = as_stream(stream);
+  if (use_split(ws, backward_bytes(experts, routes, d_in, d_out)))
+    return grouped_backward_split(x, w, grad, counts, experts, routes, d_in, d_out, grad_x, grad_w,
+                                  ws.p, st);
   int64_t off = 0;
   for (int64_t e = 0; e < experts; ++e) {
     const int64_t c = counts[e];
@@ -140,13 +258,55 @@ extern "C" int sm_row_permute(const void* input, int dtype, int64_t rows, int64_
   return SM_OK;
 }
 
-extern "C" int sm_grouped_linear(const float* input, const float* weight, const int64_t* counts,
-                                 int64_t experts, int64_t routes, int64_t d_in, int64_t d_out,
-                                 float* out, void* stream) {
+extern "C" int64_t sm_grouped_linear_workspace_bytes(int64_t experts, int64_t routes,
+                                                     int64_t d_in, int64_t d_out, int backward) {
+  if (experts <= 0 || routes < 0 || d_in <= 0 || d_out <= 0) return -1;
+  return backward ? backward_bytes(experts, routes, d_in, d_out)
+                  : forward_bytes(experts, routes, d_in, d_out);
+}
+
+extern "C" int64_t sm_grouped_swiglu_mlp_workspace_bytes(int64_t experts, int64_t routes,
+                                                         int64_t d, int64_t intermediate,
+                                                         int64_t d_out, int backward) {
+  if (experts <= 0 || routes < 0 || d <= 0 || intermediate <= 0 || d_out <= 0) return -1;
+  if (backward)
+    return std::max(backward_bytes(experts, routes, intermediate, d_out),
+                    backward_bytes(experts, routes, d, 2 * intermediate));
+  return std::max(forward_bytes(experts, routes, d, 2 * intermediate),
+                  forward_bytes(experts, routes, intermediate, d_out));
+}
+
+extern "C" int sm_grouped_linear_ws(const float* input, const float* weight,
+                                    const int64_t* counts, int64_t experts, int64_t routes,
+                                    int64_t d_in, int64_t d_out, float* out, void* workspace,
+                                    int64_t workspace_bytes, void* stream) {
   SM_REQUIRE(input && weight && out, "sm_grouped_linear: null buffer");
   SM_REQUIRE(experts > 0 && routes >= 0 && d_in > 0 && d_out > 0, "sm_grouped_linear: bad shape");
   SM_TRY(check_counts(counts, experts, routes, "sm_grouped_linear"));
-  return grouped_forward(input, weight, counts, experts, d_in, d_out, out, stream);
+  return grouped_forward(input, weight, counts, experts, routes, d_in, d_out, out,
+                         {workspace, workspace_bytes}, stream);
+}
+
+extern "C" int sm_grouped_linear(const float* input, const float* weight, const int64_t* counts,
+                                 int64_t experts, int64_t routes, int64_t d_in, int64_t d_out,
+                                 float* out, void* stream) {
+  return sm_grouped_linear_ws(input, weight, counts, experts, routes, d_in, d_out, out, nullptr, 0,
+                              stream);
+}
+
+extern "C" int sm_grouped_linear_backward_ws(const float* input, const float* weight,
+                                             const float* grad, const int64_t* counts,
+                                             int64_t experts, int64_t routes, int64_t d_in,
+                                             int64_t d_out, float* grad_input,
+                                             float* grad_weight, void* workspace,
+                                             int64_t workspace_bytes, void* stream) {
+  SM_REQUIRE(input && weight && grad && (grad_input || grad_weight),
+             "sm_grouped_linear_backward: null buffer");
+  SM_REQUIRE(experts > 0 && routes >= 0 && d_in > 0 && d_out > 0,
+             "sm_grouped_linear_backward: bad shape");
+  SM_TRY(check_counts(counts, experts, routes, "sm_grouped_linear_backward"));
+  return grouped_backward(input, weight, grad, counts, experts, routes, d_in, d_out, grad_input,
+                          grad_weight, {workspace, workspace_bytes}, stream);
 }
 
 extern "C" int sm_grouped_linear_backward(const float* input, const float* weight,
@@ -154,13 +314,28 @@ extern "C" int sm_grouped_linear_backward(const float* input, const float* weigh
                                           int64_t experts, int64_t routes, int64_t d_in,
                                           int64_t d_out, float* grad_input, float* grad_weight,
                                           void* stream) {
-  SM_REQUIRE(input && weight && grad && (grad_input || grad_weight),
-             "sm_grouped_linear_backward: null buffer");
-  SM_REQUIRE(experts > 0 && routes >= 0 && d_in > 0 && d_out > 0,
-             "sm_grouped_linear_backward: bad shape");
-  SM_TRY(check_counts(counts, experts, routes, "sm_grouped_linear_backward"));
-  return grouped_backward(input, weight, grad, counts, experts, d_in, d_out, grad_input,
-                          grad_weight, stream);
+  return sm_grouped_linear_backward_ws(input, weight, grad, counts, experts, routes, d_in, d_out,
+                                       grad_input, grad_weight, nullptr, 0, stream);
+}
+
+extern "C" int sm_grouped_swiglu_mlp_ws(const float* input, const float* in_weight,
+                                        const float* down_weight, const int64_t* counts,
+                                        int64_t experts, int64_t routes, int64_t d,
+                                        int64_t intermediate, int64_t d_out, float* out,
+                                        float* projected, float* hidden, void* workspace,
+                                        int64_t workspace_bytes, void* stream) {
+  SM_REQUIRE(input && in_weight && down_weight && out && projected && hidden,
+             "sm_grouped_swiglu_mlp: null buffer");
+  SM_REQUIRE(experts > 0 && routes >= 0 && d > 0 && intermediate > 0 && d_out > 0,
+             "sm_grouped_swiglu_mlp: bad shape");
+  SM_TRY(check_counts(counts, experts, routes, "sm_grouped_swiglu_mlp"));
+  if (routes == 0) return SM_OK;
+  const GroupedWs ws{workspace, workspace_bytes};
+  SM_TRY(grouped_forward(input, in_weight, counts, experts, routes, d, 2 * intermediate, projected,
+                         ws, stream));
+  SM_TRY(sm_swiglu(projected, SM_F32, routes, intermediate, hidden, stream));
+  return grouped_forward(hidden, down_weight, counts, experts, routes, intermediate, d_out, out, ws,
+                         stream);
 }
 
 extern "C" int sm_grouped_swiglu_mlp(const float* input, const float* in_weight,
@@ -168,16 +343,33 @@ extern "C" int sm_grouped_swiglu_mlp(const float* input, const float* in_weight,
                                      int64_t experts, int64_t routes, int64_t d,
                                      int64_t intermediate, int64_t d_out, float* out,
                                      float* projected, float* hidden, void* stream) {
-  SM_REQUIRE(input && in_weight && down_weight && out && projected && hidden,
-             "sm_grouped_swiglu_mlp: null buffer");
+  return sm_grouped_swiglu_mlp_ws(input, in_weight, down_weight, counts, experts, routes, d,
+                                  intermediate, d_out, out, projected, hidden, nullptr, 0, stream);
+}
+
+extern "C" int sm_grouped_swiglu_mlp_backward_ws(
+    const float* input, const float* in_weight, const float* down_weight, const int64_t* counts,
+    int64_t experts, int64_t routes, int64_t d, int64_t intermediate, int64_t d_out,
+    const float* projected, const float* hidden, const float* grad, float* grad_input,
+    float* grad_in_weight, float* grad_down_weight, float* scratch, void* workspace,
+    int64_t workspace_bytes, void* stream) {
+  SM_REQUIRE(input && in_weight && down_weight && projected && hidden && grad && grad_input &&
+                 grad_in_weight && grad_down_weight && scratch,
+             "sm_grouped_swiglu_mlp_backward: null buffer");
   SM_REQUIRE(experts > 0 && routes >= 0 && d > 0 && intermediate > 0 && d_out > 0,
-             "sm_grouped_swiglu_mlp: bad shape");
-  SM_TRY(check_counts(counts, experts, routes, "sm_grouped_swiglu_mlp"));
-  if (routes == 0) return SM_OK;
-  SM_TRY(grouped_forward(input, in_weight, counts, experts, d, 2 * intermediate, projected,
-                         stream));
-  SM_TRY(sm_swiglu(projected, SM_F32, routes, intermediate, hidden, stream));
-  return grouped_forward(hidden, down_weight, counts, experts, intermediate, d_out, out, stream);
+             "sm_grouped_swiglu_mlp_backward: bad shape");
+  SM_TRY(check_counts(counts, experts, routes, "sm_grouped_swiglu_mlp_backward"));
+  const GroupedWs ws{workspace, workspace_bytes};
+  // scratch: grad_hidden [routes, I] then grad_projected [routes, 2I]
+  float* grad_hidden = scratch;
+  float* grad_projected = scratch + routes * intermediate;
+  SM_TRY(grouped_backward(hidden, down_weight, grad, counts, experts, routes, intermediate, d_out,
+                          grad_hidden, grad_down_weight, ws, stream));
+  if (routes > 0)
+    SM_TRY(sm_swiglu_backward(projected, grad_hidden, SM_F32, routes, intermediate,
+                              grad_projected, stream));
+  return grouped_backward(input, in_weight, grad_projected, counts, experts, routes, d,
+                          2 * intermediate, grad_input, grad_in_weight, ws, stream);
 }
 
 extern "C" int sm_grouped_swiglu_mlp_backward(const float* input, const float* in_weight,
@@ -188,20 +380,8 @@ extern "C" int sm_grouped_swiglu_mlp_backward(const float* input, const float* i
                                               const float* grad, float* grad_input,
                                               float* grad_in_weight, float* grad_down_weight,
                                               float* scratch, void* stream) {
-  SM_REQUIRE(input && in_weight && down_weight && projected && hidden && grad && grad_input &&
-                 grad_in_weight && grad_down_weight && scratch,
-             "sm_grouped_swiglu_mlp_backward: null buffer");
-  SM_REQUIRE(experts > 0 && routes >= 0 && d > 0 && intermediate > 0 && d_out > 0,
-             "sm_grouped_swiglu_mlp_backward: bad shape");
-  SM_TRY(check_counts(counts, experts, routes, "sm_grouped_swiglu_mlp_backward"));
-  // scratch: grad_hidden [routes, I] then grad_projected [routes, 2I]
-  float* grad_hidden = scratch;
-  float* grad_projected = scratch + routes * intermediate;
-  SM_TRY(grouped_backward(hidden, down_weight, grad, counts, experts, intermediate, d_out,
-                          grad_hidden, grad_down_weight, stream));
-  if (routes > 0)
-    SM_TRY(sm_swiglu_backward(projected, grad_hidden, SM_F32, routes, intermediate,
-                              grad_projected, stream));
-  return grouped_backward(input, in_weight, grad_projected, counts, experts, d,
-                          2 * intermediate, grad_input, grad_in_weight, stream);
+  return sm_grouped_swiglu_mlp_backward_ws(input, in_weight, down_weight, counts, experts, routes,
+                                           d, intermediate, d_out, projected, hidden, grad,
+                                           grad_input, grad_in_weight, grad_down_weight, scratch,
+                                           nullptr, 0, stream);
 }

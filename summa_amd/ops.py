@@ -602,6 +602,15 @@ def _f32_dev(t: torch.Tensor, name: str) -> torch.Tensor:
     return t.contiguous()
 
 
+def _grouped_ws(query: str, device, *sizes):
+    """(tensor, pointer, bytes) of the workspace that ``query`` asks for."""
+    nbytes = int(getattr(_lib.lib(), query)(*sizes))
+    if nbytes <= 0:
+        return None, None, 0
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    return ws, ws.data_ptr(), nbytes
+
+
 def grouped_linear(input: torch.Tensor, weight: torch.Tensor, counts) -> torch.Tensor:
     """GroupedLinearBackend::grouped_linear_inner (grouped_linear.rs:23-28,
     65-86): input [routes, d_in] with counts[e] consecutive rows per expert,
@@ -613,8 +622,9 @@ def grouped_linear(input: torch.Tensor, weight: torch.Tensor, counts) -> torch.T
         raise ValueError("grouped linear input width mismatch")
     c = _host_counts(counts, E, R)
     out = torch.empty(R, dout, dtype=torch.float32, device=x.device)
-    call("sm_grouped_linear", x.data_ptr(), w.data_ptr(), c.ctypes.data, E, R, din, dout,
-         out.data_ptr(), _stream())
+    ws, base, nbytes = _grouped_ws("sm_grouped_linear_workspace_bytes", x.device, E, R, din, dout, 0)
+    call("sm_grouped_linear_ws", x.data_ptr(), w.data_ptr(), c.ctypes.data, E, R, din, dout,
+         out.data_ptr(), base, nbytes, _stream())
     return out
 
 
@@ -627,8 +637,9 @@ def grouped_linear_backward(input: torch.Tensor, weight: torch.Tensor, grad: tor
     E, _, dout = w.shape
     c = _host_counts(counts, E, R)
     gx, gw = torch.empty_like(x), torch.empty_like(w)
-    call("sm_grouped_linear_backward", x.data_ptr(), w.data_ptr(), g.data_ptr(), c.ctypes.data,
-         E, R, din, dout, gx.data_ptr(), gw.data_ptr(), _stream())
+    ws, base, nbytes = _grouped_ws("sm_grouped_linear_workspace_bytes", x.device, E, R, din, dout, 1)
+    call("sm_grouped_linear_backward_ws", x.data_ptr(), w.data_ptr(), g.data_ptr(), c.ctypes.data,
+         E, R, din, dout, gx.data_ptr(), gw.data_ptr(), base, nbytes, _stream())
     return gx, gw
 
 
@@ -648,8 +659,11 @@ def grouped_swiglu_mlp(input: torch.Tensor, in_weight: torch.Tensor, down_weight
     out = torch.empty(R, dout, dtype=torch.float32, device=x.device)
     proj = torch.empty(R, 2 * intermediate, dtype=torch.float32, device=x.device)
     hid = torch.empty(R, intermediate, dtype=torch.float32, device=x.device)
-    call("sm_grouped_swiglu_mlp", x.data_ptr(), wi.data_ptr(), wd.data_ptr(), c.ctypes.data, E, R,
-         d, intermediate, dout, out.data_ptr(), proj.data_ptr(), hid.data_ptr(), _stream())
+    ws, base, nbytes = _grouped_ws("sm_grouped_swiglu_mlp_workspace_bytes", x.device, E, R, d,
+                                   intermediate, dout, 0)
+    call("sm_grouped_swiglu_mlp_ws", x.data_ptr(), wi.data_ptr(), wd.data_ptr(), c.ctypes.data, E,
+         R, d, intermediate, dout, out.data_ptr(), proj.data_ptr(), hid.data_ptr(), base, nbytes,
+         _stream())
     return out, proj, hid
 
 
@@ -666,9 +680,12 @@ def grouped_swiglu_mlp_backward(input, in_weight, down_weight, counts, projected
     c = _host_counts(counts, E, R)
     gx, gwi, gwd = torch.empty_like(x), torch.empty_like(wi), torch.empty_like(wd)
     scratch = torch.empty(max(R, 1) * 3 * intermediate, dtype=torch.float32, device=x.device)
-    call("sm_grouped_swiglu_mlp_backward", x.data_ptr(), wi.data_ptr(), wd.data_ptr(),
+    ws, base, nbytes = _grouped_ws("sm_grouped_swiglu_mlp_workspace_bytes", x.device, E, R, d,
+                                   intermediate, dout, 1)
+    call("sm_grouped_swiglu_mlp_backward_ws", x.data_ptr(), wi.data_ptr(), wd.data_ptr(),
          c.ctypes.data, E, R, d, intermediate, dout, p.data_ptr(), h.data_ptr(), g.data_ptr(),
-         gx.data_ptr(), gwi.data_ptr(), gwd.data_ptr(), scratch.data_ptr(), _stream())
+         gx.data_ptr(), gwi.data_ptr(), gwd.data_ptr(), scratch.data_ptr(), base, nbytes,
+         _stream())
     return gx, gwi, gwd
 
 

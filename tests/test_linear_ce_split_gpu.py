@@ -42,7 +42,7 @@ def test_split_linear_ce_matches_f64(dev, T, d, V, logical, chunk, bias):
     el = _bound(d) * float((h.double().abs() @ w.double().abs().T).amax()) + 1e-6
     G = (torch.softmax(logits, 1).detach() * 3.0 / T)
     G = G + F.one_hot(t.long(), logical) * 3.0 / T
-    assert abs(float(loss) - float(ref)) <= 2 * el
+    assert abs(float(loss) - float(ref.detach())) <= 2 * el
     for name, got, want, mag, K in (
             ("hidden", gh, h64.grad, G @ w64[:logical].abs(), V),
             ("weight", gw[:logical], w64.grad[:logical], G.T @ h64.abs(), T)):
