@@ -15,70 +15,14 @@
 // All f32 with f32 accumulation: the precision of the reference CPU path.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "attn_common.hpp"
 #include "common.hpp"
+#include "gemm_wave.hpp"
 
 namespace sm {
 namespace {
-
-// ------------------------------------------------------------------ GEMM ---
-// 64 x 64 output tile per 256-thread workgroup, 4 x 4 outputs per thread, K in
-// steps of 16 through LDS; op(A) is [M, K] (A stored [M, K] or, transposed,
-// [K, M]), op(B) is [K, N] (B stored [K, N] or [N, K]).
-template <bool TA, bool TB>
-__global__ __launch_bounds__(256) void gemm_ex_kernel(const float* __restrict__ A, int64_t lda,
-                                                      const float* __restrict__ B, int64_t ldb,
-                                                      float* __restrict__ C, int64_t ldc, int M,
-                                                      int N, int K, float alpha, float beta) {
-  __shared__ float as[16][64 + 4];
-  __shared__ float bs[16][64 + 4];
-  const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
-  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-  float acc[4][4] = {};
-  for (int k0 = 0; k0 < K; k0 += 16) {
-    for (int e = threadIdx.x; e < 64 * 16; e += 256) {
-      // consecutive threads walk the contiguous dimension of each operand
-      int r, kk;
-      if (TA) { kk = e / 64; r = e % 64; } else { r = e / 16; kk = e % 16; }
-      const int gm = m0 + r, gk = k0 + kk;
-      as[kk][r] = (gm < M && gk < K) ? (TA ? A[(size_t)gk * lda + gm] : A[(size_t)gm * lda + gk])
-                                     : 0.f;
-      int c, kb;
-      if (TB) { c = e / 16; kb = e % 16; } else { kb = e / 64; c = e % 64; }
-      const int gn = n0 + c, gkb = k0 + kb;
-      bs[kb][c] = (gn < N && gkb < K) ? (TB ? B[(size_t)gn * ldb + gkb] : B[(size_t)gkb * ldb + gn])
-                                      : 0.f;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < 16; ++kk) {
-      float a[4], b[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        a[i] = as[kk][ty * 4 + i];
-        b[i] = bs[kk][tx * 4 + i];
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int gm = m0 + ty * 4 + i;
-    if (gm >= M) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int gn = n0 + tx * 4 + j;
-      if (gn >= N) continue;
-      float* cp = C + (size_t)gm * ldc + gn;
-      *cp = alpha * acc[i][j] + (beta != 0.f ? beta * *cp : 0.f);
-    }
-  }
-}
 
 // --------------------------------------------------------------- RMSNorm ---
 // y = x r gamma with r = 1 / sqrt(mean(x^2) + eps):
@@ -624,19 +568,20 @@ int gemm_ex_planes(int planes, int trans_a, int trans_b, int64_t M, int64_t N, i
   SM_REQUIRE(ceil_div(M, 64) <= 65535, "sm_gemm_ex: M above 65535 x 64 rows");
   hipStream_t st = as_stream(stream);
   // large problems on the matrix cores (bf16 plane products, gemm_mfma.hip);
-  // small ones, where a launch has few 128 x 128 tiles, here
+  // small ones on the FMA units (gemm_wave.hpp)
   if (K >= 32 && M * N >= (int64_t)128 * 128 * 16 && M * N * K >= ((int64_t)1 << 27))
     return gemm_planes(planes, trans_a != 0, trans_b != 0, M, N, K, alpha, A, lda, B, ldb, beta,
                        C, ldc, st, scratch, scratch_floats, b_planes);
-  const dim3 grid((unsigned)ceil_div(N, 64), (unsigned)ceil_div(M, 64));
-#define SM_GX(TA, TB)                                                                        \
-  gemm_ex_kernel<TA, TB><<<grid, 256, 0, st>>>(A, lda, B, ldb, C, ldc, (int)M, (int)N, (int)K, \
-                                               alpha, beta)
-  if (trans_a && trans_b) SM_GX(true, true);
-  else if (trans_a) SM_GX(true, false);
-  else if (trans_b) SM_GX(false, true);
-  else SM_GX(false, false);
-#undef SM_GX
+  auto run = [&](auto ta, auto tb) {
+    gemm_wave<decltype(ta)::value, decltype(tb)::value>(A, lda, B, ldb, C, ldc, M, N, K, alpha,
+                                                        beta, st);
+  };
+  using T = std::true_type;
+  using F = std::false_type;
+  if (trans_a && trans_b) run(T{}, T{});
+  else if (trans_a) run(T{}, F{});
+  else if (trans_b) run(F{}, T{});
+  else run(F{}, F{});
   SM_LAUNCH_CHECK();
   return SM_OK;
 }

@@ -39,3 +39,28 @@ def test_gemm_f32_matches_f64(dev, M, N, K, pad, epilogue):
     # K + 1 roundings of at most 2^-24 of the running magnitude
     assert (np.abs(got[:, :N] - want) <= (K + 1) * 2.0 ** -24 * mag).all()
     assert (got[:, N:] == 7.0).all()
+
+
+# sm_gemm_ex's small products, each transpose pair: ragged tiles of every size
+# (one, two and four 8-row blocks a wave), odd leading dimensions, and a long k.
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K,pad", [(1, 1, 1, 0), (13, 9, 131, 1), (64, 64, 128, 0),
+                                       (20, 36, 4100, 4), (515, 520, 67, 0), (1030, 1027, 33, 0)])
+def test_small_gemm_ex_matches_f64(dev, ta, tb, M, N, K, pad):
+    print(f"case small gemm_ex ta={ta} tb={tb} M={M} N={N} K={K} pad={pad}", flush=True)
+    rng = np.random.default_rng(M + N + K + 2 * ta + tb)
+    a, b = rng.normal(0, 1, (M, K)).astype(np.float32), rng.normal(0, 1, (K, N)).astype(np.float32)
+    c0 = rng.normal(0, 1, (M, N)).astype(np.float32)
+
+    def padded(x):
+        t = torch.full((x.shape[0], x.shape[1] + pad), float("nan"), device=dev)
+        t[:, :x.shape[1]] = torch.from_numpy(np.ascontiguousarray(x)).to(dev)
+        return t
+    A, B, C = padded(a.T if ta else a), padded(b.T if tb else b), padded(c0)
+    call("sm_gemm_ex", ta, tb, M, N, K, 0.5, A.data_ptr(), A.stride(0), B.data_ptr(), B.stride(0),
+         2.0, C.data_ptr(), C.stride(0), torch.cuda.current_stream().cuda_stream)
+    got = C[:, :N].cpu().numpy().astype(np.float64)
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    want = 0.5 * (a64 @ b64) + 2.0 * c0
+    mag = 0.5 * (np.abs(a64) @ np.abs(b64)) + 2.0 * np.abs(c0)
+    assert (np.abs(got - want) <= (K + 3) * 2.0 ** -24 * mag).all()
