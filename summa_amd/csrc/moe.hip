@@ -11,8 +11,8 @@
 //   out[t] = sum_j w[t,j] * routed[inverse[t*k+j]] (route_combine_forward,
 //     moe_dispatch.rs:290-312), added to the residual stream.
 //
-// MI355X design: no host round trip anywhere. The route plan (one workgroup,
-// deterministic stable counting sort) also emits two device tile lists
+// MI355X design: no host round trip anywhere. The route plan (a deterministic
+// stable counting sort) also emits two device tile lists
 // (16-row and 128-row tiles per expert), which the grouped Q4 matmuls consume
 // directly: the small-M kernel for decode (q4.hip) and the LDS kernel for
 // prefill / recompute (q4_gemm_bl.hip). The token gather is folded into the
@@ -49,6 +49,7 @@ namespace {
 
 constexpr int kRouterThreads = 512;  // 8 waves: four experts each at E = 32
 constexpr int kRouterLds = 64 * 1024;  // dynamic LDS budget (h rows + logits)
+constexpr int kRouterMaxE = 64;
 
 // One workgroup per TT tokens: their h rows go to LDS (f32), then each of the
 // 8 waves takes experts e = wave, wave + 8, ...: its lanes stream W_r[e] once
@@ -174,6 +175,98 @@ __global__ __launch_bounds__(kRouterThreads) void router_top2_kernel(
   }
 }
 
+// The same for many tokens (d = 64 CH): 32 tokens per workgroup, each wave's four
+// rows held in registers (lane: columns 64 u + lane) and every expert's weights
+// staged through LDS once for all of them, two experts deep. With the rows in LDS
+// each FMA needed its own LDS read, and every four tokens re-read all the
+// router weights from L2: 32 experts, 8192 tokens 109 -> 54 us, 65536 861 -> 380. The
+// sums are those of the kernel above, bit for bit.
+constexpr int kRouterRows = 32;
+template <typename TH, bool PAIR, int CH>
+__global__ __launch_bounds__(kRouterThreads) void router_rows_kernel(
+    const TH* __restrict__ h, const float* __restrict__ wr, int64_t tokens, int E,
+    float* __restrict__ logits_out, int32_t* __restrict__ top_idx, float* __restrict__ top_w) {
+  constexpr int D = CH * kWave, TT = 4, NV = (D / 4 + kRouterThreads - 1) / kRouterThreads;
+  __shared__ __attribute__((aligned(16))) float ws[2][D];
+  __shared__ float lg[kRouterRows][kRouterMaxE + 1];
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  const int64_t t0 = (int64_t)blockIdx.x * kRouterRows;
+  float hv[TT][CH];
+#pragma unroll
+  for (int t = 0; t < TT; ++t) {
+    const int64_t r = min<int64_t>(t0 + wave * TT + t, tokens - 1);
+    const TH* row = h + r * (PAIR ? 2 * D : D) + lane;
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      float v = (float)row[u * kWave];
+      if constexpr (PAIR) v += (float)row[D + u * kWave];
+      hv[t][u] = v;
+    }
+  }
+  float4 next[NV];
+  auto fetch = [&](int e) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = threadIdx.x + i * kRouterThreads;
+      if (c < D / 4) next[i] = reinterpret_cast<const float4*>(wr + (size_t)e * D)[c];
+    }
+  };
+  auto stage = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = threadIdx.x + i * kRouterThreads;
+      if (c < D / 4) reinterpret_cast<float4*>(ws[buf])[c] = next[i];
+    }
+  };
+  fetch(0);
+  stage(0);
+  __syncthreads();
+  for (int e = 0; e < E; ++e) {
+    if (e + 1 < E) fetch(e + 1);
+    float acc[TT] = {};
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      const float w = ws[e & 1][u * kWave + lane];
+#pragma unroll
+      for (int t = 0; t < TT; ++t) acc[t] = fmaf(hv[t][u], w, acc[t]);
+    }
+#pragma unroll
+    for (int t = 0; t < TT; ++t) {
+      const float v = wave_sum(acc[t]);
+      if (lane == 0) lg[wave * TT + t][e] = v;
+    }
+    if (e + 1 < E) stage((e + 1) & 1);  // last read before the previous barrier
+    __syncthreads();
+  }
+  const int n = (int)min<int64_t>(kRouterRows, tokens - t0);
+  if ((int)threadIdx.x < n && top_idx) {
+    const int64_t r = t0 + threadIdx.x;
+    int i0, i1;
+    float w0, w1;
+    top2_of(lg[threadIdx.x], E, i0, i1, w0, w1);
+    top_idx[r * 2] = i0;
+    top_idx[r * 2 + 1] = i1;
+    top_w[r * 2] = w0;
+    top_w[r * 2 + 1] = w1;
+  }
+  if (logits_out)
+    for (int i = threadIdx.x; i < n * E; i += kRouterThreads)
+      logits_out[t0 * E + i] = lg[i / E][i % E];
+}
+
+// Runs router_rows_kernel where it is the faster one: rows that fill its registers
+// and enough tokens for half the chip (one workgroup takes 32 tokens through
+// every expert, 41 us however few there are: 3072 tokens 39 us with the kernel
+// above, 4096 56). At d 1024 it gains nothing (8192 tokens 35 -> 32, 4000 14 -> 18).
+template <typename TH, bool PAIR>
+bool launch_router_rows(const void* h, const float* wr, int64_t tokens, int d, int E, float* lo,
+                        int32_t* idx, float* w, hipStream_t st) {
+  if (tokens < 4096 || d != 32 * kWave || reinterpret_cast<uintptr_t>(wr) % 16 != 0) return false;
+  router_rows_kernel<TH, PAIR, 32><<<(unsigned)ceil_div(tokens, kRouterRows), kRouterThreads, 0,
+                                     st>>>(static_cast<const TH*>(h), wr, tokens, E, lo, idx, w);
+  return true;
+}
+
 template <typename TH, bool PAIR, int TT>
 void launch_router(const void* h, const float* wr, int64_t tokens, int d, int E, float* lo,
                    int32_t* idx, float* w, hipStream_t st) {
@@ -198,6 +291,7 @@ void launch_router(const void* h, const float* wr, int64_t tokens, int d, int E,
 template <typename TH, bool PAIR>
 void launch_router_tt(const void* h, const float* wr, int64_t tokens, int d, int E, float* lo,
                       int32_t* idx, float* w, hipStream_t st) {
+  if (launch_router_rows<TH, PAIR>(h, wr, tokens, d, E, lo, idx, w, st)) return;
   // tokens per workgroup: the largest of 8 / 4 / 2 / 1 whose rows fit the LDS budget
   const int64_t row = (int64_t)(d + E) * sizeof(float);
   if (8 * row <= kRouterLds) launch_router<TH, PAIR, 8>(h, wr, tokens, d, E, lo, idx, w, st);
@@ -206,84 +300,175 @@ void launch_router_tt(const void* h, const float* wr, int64_t tokens, int d, int
   else launch_router<TH, PAIR, 1>(h, wr, tokens, d, E, lo, idx, w, st);
 }
 
-// Stable counting sort of the routes by expert in one workgroup. Thread i owns
-// the contiguous route chunk [i*C, (i+1)*C); per-(thread, expert) counts live in
-// LDS, an exclusive scan over threads per expert gives each thread's write
-// base, and each thread then places its routes in order: the result equals the
-// reference's host plan (experts ascending, route ids ascending within one).
-constexpr int kPlanThreads = 128;
+// The route plan is a stable counting sort of the routes by expert: the result
+// equals the reference's host plan (experts ascending, route ids ascending
+// within one), with the 16- and 128-row tile lists beside it.
 constexpr int kMaxExperts = 64;
+static_assert(kRouterMaxE == kMaxExperts, "");
+constexpr int kPlanSmall = 1024;  // routes per workgroup pass
 
-__global__ __launch_bounds__(kPlanThreads) void route_plan_kernel(const int32_t* __restrict__ idx,
-                                                                  int routes, int k, int E,
-                                                                  PlanView pv, int max16,
-                                                                  int max128,
-                                                                  int32_t* __restrict__ error) {
-  __shared__ int32_t cnt[kPlanThreads][kMaxExperts + 1];
-  __shared__ int32_t offs[kMaxExperts + 1];
-  const int t = threadIdx.x;
-  const int C = (routes + kPlanThreads - 1) / kPlanThreads;
-  const int r0 = min(t * C, routes), r1 = min(r0 + C, routes);
-  for (int e = 0; e < E; ++e) cnt[t][e] = 0;
-  int bad = 0;
-  for (int r = r0; r < r1; ++r) {
+// Rank of this thread's route among its wave's routes of the same expert (lanes,
+// like waves, are in route order), and the wave's count of every expert.
+__device__ inline int expert_rank(int e, int E, int32_t* wave_counts) {
+  const int lane = threadIdx.x % kWave;
+  const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  int rank = 0;
+  for (int x = 0; x < E; ++x) {
+    const uint64_t m = __ballot(e == x);
+    if (e == x) rank = __popcll(m & below);
+    if (lane == 0) wave_counts[x] = __popcll(m);
+  }
+  return rank;
+}
+
+// Routes of workgroup b out of nb: kPlanSmall each, the last one the remainder
+// too (up to twice as many).
+__device__ inline void plan_range(int routes, int& r0, int& r1) {
+  r0 = (int)blockIdx.x * kPlanSmall;
+  r1 = blockIdx.x == gridDim.x - 1 ? routes : r0 + kPlanSmall;
+}
+
+// More than kPlanSmall routes, in three launches. 1: each workgroup counts its
+// routes per expert, into the first words of its own part of `inverse` (nothing
+// else is there yet). 2: one workgroup turns the counts into each workgroup's
+// first position per expert, and writes the offsets and tile lists. 3: each
+// workgroup ranks its routes again and writes their positions. (One workgroup
+// walking everything serially took 126 us at 16384 routes and 956 at 131072; now
+// 16 us at both, the launches themselves.)
+__global__ __launch_bounds__(kPlanSmall) void route_count_kernel(const int32_t* __restrict__ idx,
+                                                                 int routes, int E, PlanView pv,
+                                                                 int32_t* __restrict__ error) {
+  __shared__ int32_t cnt[kMaxExperts];
+  if (threadIdx.x < kMaxExperts) cnt[threadIdx.x] = 0;
+  __syncthreads();
+  int r0, r1;
+  plan_range(routes, r0, r1);
+  for (int r = r0 + threadIdx.x; r < r1; r += kPlanSmall) {
     const int e = idx[r];
-    if (e < 0 || e >= E) { bad = 1; continue; }
-    cnt[t][e] += 1;
-  }
-  if (bad) atomicOr(error, 1);
-  __syncthreads();
-  // per expert: exclusive scan over threads (thread e does expert e)
-  if (t < E) {
-    int run = 0;
-    for (int i = 0; i < kPlanThreads; ++i) {
-      const int c = cnt[i][t];
-      cnt[i][t] = run;
-      run += c;
-    }
-    pv.counts[t] = run;
-    offs[t] = run;  // total per expert, turned into offsets below
+    if (e < 0 || e >= E) atomicOr(error, 1);
+    else atomicAdd(&cnt[e], 1);
   }
   __syncthreads();
-  if (t == 0) {
-    int acc = 0;
-    for (int e = 0; e < E; ++e) {
-      const int c = offs[e];
-      offs[e] = acc;
-      pv.offsets[e] = acc;
-      acc += c;
+  if ((int)threadIdx.x < E) pv.inverse[r0 + threadIdx.x] = cnt[threadIdx.x];
+}
+
+__global__ __launch_bounds__(kPlanSmall) void route_scan_kernel(int nb, int E, PlanView pv,
+                                                                int max16, int max128) {
+  constexpr int NP = kPlanSmall / kMaxExperts;  // parts of the workgroup list
+  __shared__ int32_t part[NP][kMaxExperts];
+  __shared__ int32_t s16[kMaxExperts + 1], s128[kMaxExperts + 1];
+  const int e = threadIdx.x % kMaxExperts, p = threadIdx.x / kMaxExperts;
+  const int b0 = (int)((int64_t)nb * p / NP), b1 = (int)((int64_t)nb * (p + 1) / NP);
+  int sum = 0;
+  if (e < E)
+#pragma unroll 4
+    for (int b = b0; b < b1; ++b) sum += pv.inverse[(int64_t)b * kPlanSmall + e];
+  part[p][e] = sum;
+  __syncthreads();
+  if (threadIdx.x < kWave) {  // lane e: totals, then exclusive scans over the experts
+    int tot = 0;
+    for (int i = 0; i < NP; ++i) {
+      const int c = part[i][e];
+      part[i][e] = tot;
+      tot += c;
     }
-    offs[E] = acc;
-    pv.offsets[E] = acc;
-    // tile lists: (expert, first row) for 16- and 128-row tiles
-    int n16 = 0, n128 = 0;
-    for (int e = 0; e < E; ++e) {
-      const int c = offs[e + 1] - offs[e];
-      for (int r = 0; r < c && n16 < max16; r += 16, ++n16) {
-        pv.tiles16[2 * n16] = e;
-        pv.tiles16[2 * n16 + 1] = r;
+    const int t16 = (tot + 15) / 16, t128 = (tot + 127) / 128;
+    int a = tot, a16 = t16, a128 = t128;  // inclusive scans
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const int x = __shfl_up(a, o, kWave), x16 = __shfl_up(a16, o, kWave),
+                x128 = __shfl_up(a128, o, kWave);
+      if (e >= o) { a += x; a16 += x16; a128 += x128; }
+    }
+    s16[e + 1] = a16;
+    s128[e + 1] = a128;
+    if (e == 0) s16[0] = s128[0] = 0;
+    if (e < E) {
+      pv.counts[e] = tot;
+      pv.offsets[e] = a - tot;
+      if (e == E - 1) {
+        pv.offsets[E] = a;
+        pv.ntiles16[0] = min(a16, max16);
+        pv.ntiles128[0] = min(a128, max128);
       }
-      for (int r = 0; r < c && n128 < max128; r += 128, ++n128) {
-        pv.tiles128[2 * n128] = e;
-        pv.tiles128[2 * n128 + 1] = r;
-      }
     }
-    pv.ntiles16[0] = n16;
-    pv.ntiles128[0] = n128;
   }
   __syncthreads();
-  for (int r = r0; r < r1; ++r) {
-    const int e = idx[r];
-    if (e < 0 || e >= E) {
-      pv.inverse[r] = -1;  // flagged route: combine skips it
-      continue;
+  if (e < E) {
+    int run = part[p][e];
+    for (int b = b0; b < b1; ++b) {
+      int32_t* c = pv.inverse + (int64_t)b * kPlanSmall + e;
+      const int n = *c;
+      *c = run;
+      run += n;
     }
-    const int pos = offs[e] + cnt[t][e];
-    cnt[t][e] += 1;
-    pv.order[pos] = r;
-    pv.inverse[r] = pos;
-    pv.src_rows[pos] = r / k;
   }
+  auto tiles = [&](const int32_t* first, int max_tiles, int rows, int32_t* out) {
+    const int n = min(first[E], max_tiles);
+    for (int i = threadIdx.x; i < n; i += kPlanSmall) {
+      int lo = 0, hi = E - 1;  // the expert whose tiles hold i
+      while (lo < hi) {
+        const int mid = (lo + hi) / 2;
+        if (i < first[mid + 1]) hi = mid;
+        else lo = mid + 1;
+      }
+      out[2 * i] = lo;
+      out[2 * i + 1] = (i - first[lo]) * rows;
+    }
+  };
+  tiles(s16, max16, 16, pv.tiles16);
+  tiles(s128, max128, 128, pv.tiles128);
+}
+
+__global__ __launch_bounds__(kPlanSmall) void route_place_kernel(const int32_t* __restrict__ idx,
+                                                                 int routes, int k, int E,
+                                                                 PlanView pv) {
+  constexpr int NW = kPlanSmall / kWave;
+  __shared__ int32_t wc[NW][kMaxExperts];  // wave counts, then wave bases
+  __shared__ int32_t base[kMaxExperts];
+  int r0, r1;
+  plan_range(routes, r0, r1);
+  if ((int)threadIdx.x < E)
+    base[threadIdx.x] = pv.offsets[threadIdx.x] + pv.inverse[r0 + threadIdx.x];
+  __syncthreads();  // `inverse` is written below
+  for (int s = r0; s < r1; s += kPlanSmall) {
+    const int r = s + threadIdx.x, wave = threadIdx.x / kWave;
+    int e = -1;
+    if (r < r1) {
+      e = idx[r];
+      if (e < 0 || e >= E) {
+        pv.inverse[r] = -1;  // flagged route: combine skips it
+        e = -1;
+      }
+    }
+    const int rank = expert_rank(e, E, wc[wave]);
+    __syncthreads();
+    if ((int)threadIdx.x < E) {
+      int at = base[threadIdx.x];
+      for (int w = 0; w < NW; ++w) {
+        const int c = wc[w][threadIdx.x];
+        wc[w][threadIdx.x] = at;
+        at += c;
+      }
+      base[threadIdx.x] = at;
+    }
+    __syncthreads();
+    if (e >= 0) {
+      const int pos = wc[wave][e] + rank;
+      pv.order[pos] = r;
+      pv.inverse[r] = pos;
+      pv.src_rows[pos] = r / k;
+    }
+    __syncthreads();
+  }
+}
+
+void route_plan_large(const int32_t* idx, int routes, int k, int E, PlanView pv, int max16,
+                      int max128, int32_t* error, hipStream_t st) {
+  const int nb = routes / kPlanSmall;
+  route_count_kernel<<<nb, kPlanSmall, 0, st>>>(idx, routes, E, pv, error);
+  route_scan_kernel<<<1, kPlanSmall, 0, st>>>(nb, E, pv, max16, max128);
+  route_place_kernel<<<nb, kPlanSmall, 0, st>>>(idx, routes, k, E, pv);
 }
 
 // The same plan for at most kPlanSmall routes (decode batches): one thread per
@@ -291,9 +476,7 @@ __global__ __launch_bounds__(kPlanThreads) void route_plan_kernel(const int32_t*
 // and each route's rank among the wave's routes of that expert (lanes, like
 // waves, are in route order, so the sort stays stable); a 16-step pass per
 // expert turns the wave counts into wave bases, and one wave scans the
-// expert totals and tile counts with shuffles. Output identical to
-// route_plan_kernel.
-constexpr int kPlanSmall = 1024;
+// expert totals and tile counts with shuffles.
 constexpr size_t kPlanLogitsLds = 64 * 1024;  // logits route_plan_small_kernel stages
 
 // With logits (top-2 routing, k = 2): route r first takes the top-2 of its
@@ -328,13 +511,7 @@ __global__ __launch_bounds__(kPlanSmall) void route_plan_small_kernel(
       e = -1;
     }
   }
-  const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  int rank = 0;
-  for (int x = 0; x < E; ++x) {
-    const uint64_t m = __ballot(e == x);
-    if (e == x) rank = __popcll(m & below);
-    if (lane == 0) wc[wave][x] = __popcll(m);
-  }
+  const int rank = expert_rank(e, E, wc[wave]);
   __syncthreads();
   if (wave == 0) {
     // lane x: expert x's wave bases and total; then the exclusive scans of
@@ -396,22 +573,34 @@ __global__ void top2_from_logits_kernel(const float* __restrict__ logits, int64_
 }
 
 // x[t, c] += sum_j w[t, j] * routed[inverse[t*k + j], c]   (f32); routes the
-// plan flagged (inverse < 0) contribute nothing
-__global__ void combine_kernel(const float* __restrict__ routed, const float* __restrict__ w,
+// plan flagged (inverse < 0) contribute nothing. HBM-bound: T is four columns
+// where the rows allow (8192 x 2048: 69 us with one column per thread, 38 with
+// four; 65536 tokens 808 -> 384).
+template <typename T>
+__global__ void combine_kernel(const T* __restrict__ routed, const float* __restrict__ w,
                                const int32_t* __restrict__ inverse, int64_t tokens, int k, int d,
-                               float* __restrict__ x) {
+                               T* __restrict__ x) {
+  constexpr int NC = sizeof(T) / sizeof(float);
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= tokens * d) return;
+  if (i >= tokens * d) return;  // d in units of T
   const int64_t t = i / d;
   const int c = i % d;
   const int64_t routes = tokens * k;
-  float sum = 0.f;
+  float sum[NC] = {};
   for (int j = 0; j < k; ++j) {
     const int64_t route = t * k + j;
     const int p = inverse[route];
-    if (p >= 0 && p < routes) sum += routed[(int64_t)p * d + c] * w[route];
+    if (p >= 0 && p < routes) {
+      const T v = routed[(int64_t)p * d + c];
+      const float f = w[route];
+#pragma unroll
+      for (int e = 0; e < NC; ++e) sum[e] += reinterpret_cast<const float*>(&v)[e] * f;
+    }
   }
-  x[i] += sum;
+  T v = x[i];
+#pragma unroll
+  for (int e = 0; e < NC; ++e) reinterpret_cast<float*>(&v)[e] += sum[e];
+  x[i] = v;
 }
 
 // combine_kernel's sum for one token row (its routes in order, x += sum),
@@ -454,6 +643,8 @@ __global__ __launch_bounds__(64 * V) void combine_rmsnorm_kernel(
 
 using namespace sm;
 
+extern "C" int sm_moe_route_plan(const int32_t* top_idx, int64_t tokens, int64_t top_k,
+                                 int64_t experts, int32_t* plan, int32_t* error, void* stream);
 extern "C" int sm_rmsnorm(const float* x, const float* gamma, int64_t rows, int64_t d, float eps,
                           void* y, int out_dtype, void* stream);
 extern "C" int sm_moe_combine(const float* routed, const float* top_w, const int32_t* plan,
@@ -545,8 +736,8 @@ extern "C" int sm_moe_route_plan(const int32_t* top_idx, int64_t tokens, int64_t
     route_plan_small_kernel<<<1, kPlanSmall, 0, as_stream(stream)>>>(
         top_idx, (int)routes, (int)top_k, (int)experts, pv, max16, max128, error);
   else
-    route_plan_kernel<<<1, kPlanThreads, 0, as_stream(stream)>>>(
-        top_idx, (int)routes, (int)top_k, (int)experts, pv, max16, max128, error);
+    route_plan_large(top_idx, (int)routes, (int)top_k, (int)experts, pv, max16, max128, error,
+                     as_stream(stream));
   SM_LAUNCH_CHECK();
   return SM_OK;
 }
@@ -572,8 +763,8 @@ extern "C" int sm_moe_route_plan_logits(const float* logits, int64_t tokens, int
   } else {
     top2_from_logits_kernel<<<(unsigned)ceil_div(tokens, 256), 256, 0, st>>>(
         logits, tokens, (int)experts, top_idx, top_w);
-    route_plan_kernel<<<1, kPlanThreads, 0, st>>>(top_idx, (int)routes, 2, (int)experts, pv,
-                                                  max16, max128, error);
+    SM_LAUNCH_CHECK();
+    return sm_moe_route_plan(top_idx, tokens, 2, experts, plan, error, stream);
   }
   SM_LAUNCH_CHECK();
   return SM_OK;
@@ -586,8 +777,14 @@ extern "C" int sm_moe_combine(const float* routed, const float* top_w, const int
   SM_REQUIRE(tokens >= 0 && top_k >= 1 && d > 0, "sm_moe_combine: bad shape");
   if (tokens == 0) return SM_OK;
   PlanView pv = plan_view(const_cast<int32_t*>(plan), tokens * top_k, experts);
-  combine_kernel<<<(unsigned)ceil_div(tokens * d, 256), 256, 0, as_stream(stream)>>>(
-      routed, top_w, pv.inverse, tokens, (int)top_k, (int)d, x);
+  if (d % 4 == 0 && reinterpret_cast<uintptr_t>(routed) % 16 == 0 &&
+      reinterpret_cast<uintptr_t>(x) % 16 == 0)
+    combine_kernel<float4><<<(unsigned)ceil_div(tokens * (d / 4), 256), 256, 0, as_stream(stream)>>>(
+        reinterpret_cast<const float4*>(routed), top_w, pv.inverse, tokens, (int)top_k,
+        (int)(d / 4), reinterpret_cast<float4*>(x));
+  else
+    combine_kernel<float><<<(unsigned)ceil_div(tokens * d, 256), 256, 0, as_stream(stream)>>>(
+        routed, top_w, pv.inverse, tokens, (int)top_k, (int)d, x);
   SM_LAUNCH_CHECK();
   return SM_OK;
 }

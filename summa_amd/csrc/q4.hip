@@ -1606,6 +1606,16 @@ extern "C" int sm_q4_grouped_matmul(const uint8_t* codes, const uint16_t* scales
     if (is_swiglu(epilogue) || K < 4 * 128) return launch_q4<2, 1>(a, epilogue, xt, st, rt);
     return launch_q4<2, 4>(a, epilogue, xt, st, rt);
   }
+  // 256 x 256 tiles (q4_gemm_wide.hip, the same bits) once an expert has about
+  // a tile of rows and the launch half the chip (the two projections, us): 8192
+  // tokens, top-2 of 32 experts, d 2048, width 1408: 592 + 284 -> 482 + 238; 65536:
+  // 3736 + 1926 -> 2779 + 1439; 3072 (192 rows an expert) 256 + 131 -> 205 + 90;
+  // 2100 tokens, 8 experts, d and width 512 (80 and 40 workgroups): 32 + 26 -> 32 + 29.
+  const int64_t wide = (routes / 256 + experts / 2) * ceil_div(N, 256);
+  if ((xt == X_F16 || xt == X_F16X2) && routes >= 192 * experts && wide >= 128)
+    return q4_gemm_wide_grouped(codes, scales, (int)N, (int)K, x, xt, (int)routes, (int)experts,
+                                (int)ldx, y, (int)ldy, epilogue, (int)ncols, pv.offsets, rowidx,
+                                cstride, sstride, st);
   return q4_gemm_bl(codes, scales, (int)N, (int)K, x, xt, (int)routes, (int)ldx, y, (int)ldy,
                     epilogue, (int)ncols, st, pv.tiles128, pv.ntiles128,
                     moe_max_tiles(routes, experts, 128), pv.offsets, rowidx, cstride, sstride,

@@ -60,11 +60,17 @@ struct WideArgs {
   _Float16* q_out;
   _Float16* kc;
   _Float16* vc;
+  // grouped (MoE) mode: expert e's positions goff[e] .. goff[e+1]-1 in 256-row
+  // tiles; A row of position p = rowidx[p] (or p); weights cstride / sstride apart
+  const int32_t* goff;
+  const int32_t* rowidx;
+  int experts;
+  size_t cstride, sstride;
 };
 
 // EPI: 0 store f32, 1 store bf16, 2 add f32, 3 swiglu bf16, 4 swiglu f16,
 // 5 swiglu f16 pair, 6 qkv + RoPE + cache append (f16). NA: 1 f16 x, 2 pairs.
-template <int NA, int EPI>
+template <int NA, int EPI, bool GROUPED = false>
 __global__ __launch_bounds__(512, 1) void q4_gemm_wide_kernel(WideArgs a) {
   constexpr bool SWIGLU = (EPI >= 3 && EPI <= 5);
   constexpr int MT = 4, NB = 8;  // 16-row / 16-column blocks per wave
@@ -75,7 +81,25 @@ __global__ __launch_bounds__(512, 1) void q4_gemm_wide_kernel(WideArgs a) {
   //      one per XCD, take 8 row tiles of one column tile; each XCD sweeps
   //      the column tiles of its row tile back to back)
   int tn, tm;
-  if (a.mtiles >= 8) {
+  int m0, mlim = a.M;  // the tile's first row; rows from mlim on are not its own
+  const uint8_t* codes = a.codes;
+  const uint16_t* scales = a.scales;
+  if constexpr (GROUPED) {
+    // the same walk over the experts' row tiles, counted here from the offsets
+    const int w = blockIdx.x, xcd = w % 8, q = w / 8;
+    tn = q % a.ntiles;
+    tm = (q / a.ntiles) * 8 + xcd;
+    int e = 0, n = 0;
+    for (; e < a.experts; ++e, tm -= n) {
+      n = (a.goff[e + 1] - a.goff[e] + kWM - 1) / kWM;
+      if (tm < n) break;
+    }
+    if (e == a.experts) return;  // past the last tile (uniform per workgroup)
+    m0 = a.goff[e] + tm * kWM;
+    mlim = a.goff[e + 1];
+    codes += (size_t)e * a.cstride;
+    scales += (size_t)e * a.sstride;
+  } else if (a.mtiles >= 8) {
     const int w = blockIdx.x, xcd = w % 8, q = w / 8;
     tn = q % a.ntiles;
     tm = (q / a.ntiles) * 8 + xcd;
@@ -84,7 +108,7 @@ __global__ __launch_bounds__(512, 1) void q4_gemm_wide_kernel(WideArgs a) {
     tn = blockIdx.x % a.ntiles;
     tm = blockIdx.x / a.ntiles;
   }
-  const int m0 = tm * kWM;
+  if constexpr (!GROUPED) m0 = tm * kWM;
   const int t = threadIdx.x, wave = t / kWave, lane = t % kWave;
   const int j = lane % 16, g = lane / 16;
   const int wr = wave / 2, wc = wave % 2;
@@ -99,7 +123,10 @@ __global__ __launch_bounds__(512, 1) void q4_gemm_wide_kernel(WideArgs a) {
   for (int i = 0; i < 2; ++i) {
     const int c = i * 512 + t;
     aoff[i] = wsw(c / 4, c % 4);
-    xa[i] = a.x + (size_t)min(m0 + c / 4, a.M - 1) * a.ldx + (c % 4) * 8;
+    int row = min(m0 + c / 4, mlim - 1);
+    if constexpr (GROUPED)
+      if (a.rowidx) row = a.rowidx[row];
+    xa[i] = a.x + (size_t)row * a.ldx + (c % 4) * 8;
   }
   const int bcol = t / 2, bhalf = t & 1;
   int wrow;  // weight row staged into LDS column bcol (-1: zero column)
@@ -114,8 +141,8 @@ __global__ __launch_bounds__(512, 1) void q4_gemm_wide_kernel(WideArgs a) {
       wrow = col < a.N ? col : -1;
     }
   }
-  const uint8_t* cbase = a.codes + q4t_code_offset(max(wrow, 0), 0, ngroups) + bhalf * 8;
-  const uint16_t* sbase = a.scales + q4t_scale_index(max(wrow, 0), 0, ngroups);
+  const uint8_t* cbase = codes + q4t_code_offset(max(wrow, 0), 0, ngroups) + bhalf * 8;
+  const uint16_t* sbase = scales + q4t_scale_index(max(wrow, 0), 0, ngroups);
   const int boff0 = wsw(bcol, bhalf * 2), boff1 = wsw(bcol, bhalf * 2 + 1);
 
   u32x4 ra[NA][2];
@@ -262,7 +289,7 @@ __global__ __launch_bounds__(512, 1) void q4_gemm_wide_kernel(WideArgs a) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int row = m0 + wr * 64 + mt * 16 + 4 * g + r;
-      if (row >= a.M) continue;
+      if (row >= mlim) continue;
       if constexpr (SWIGLU) {
 #pragma unroll
         for (int b = 0; b < NB / 2; ++b) {
@@ -316,7 +343,57 @@ int launch_wide(const WideArgs& a, int epi, unsigned grid, hipStream_t st) {
   return SM_OK;
 }
 
+template <int NA>
+int launch_wide_grouped(const WideArgs& a, int epi, unsigned grid, hipStream_t st) {
+  switch (epi) {
+#define SM_WIDE(E) \
+    case E: q4_gemm_wide_kernel<NA, E, true><<<grid, 512, 0, st>>>(a); break;
+    SM_WIDE(0)
+    SM_WIDE(1)
+    SM_WIDE(3)
+    SM_WIDE(4)
+    SM_WIDE(5)
+#undef SM_WIDE
+    default: set_error("sm_q4_grouped_matmul: unknown epilogue %d", epi); return SM_ERR_INVALID;
+  }
+  SM_LAUNCH_CHECK();
+  return SM_OK;
+}
+
 }  // namespace
+
+int q4_gemm_wide_grouped(const uint8_t* codes, const uint16_t* scales, int N, int K, const void* x,
+                         int xt, int routes, int experts, int ldx, void* y, int ldy, int epi,
+                         int ncols, const int32_t* goff, const int32_t* rowidx, size_t cstride,
+                         size_t sstride, hipStream_t st) {
+  WideArgs a{};
+  a.codes = codes;
+  a.scales = scales;
+  a.x = static_cast<const _Float16*>(x);
+  a.y = y;
+  a.M = routes;
+  a.N = N;
+  a.K = K;
+  a.ldx = ldx;
+  a.ldy = ldy;
+  a.ncols = ncols;
+  a.goff = goff;
+  a.rowidx = rowidx;
+  a.experts = experts;
+  a.cstride = cstride;
+  a.sstride = sstride;
+  const bool swiglu = epi >= 3 && epi <= 5;
+  a.ntiles = (int)ceil_div(swiglu ? 2 * (int64_t)ncols : N, kWN);
+  // (at most one partial tile per expert)
+  const int64_t mtiles = routes / kWM + experts;
+  const int64_t blocks = ceil_div(mtiles, 8) * 8 * a.ntiles;
+  if (blocks > 0x7fffffff) {
+    set_error("sm_q4_grouped_matmul: problem too large");
+    return SM_ERR_UNSUPPORTED;
+  }
+  return xt == 2 ? launch_wide_grouped<2>(a, epi, (unsigned)blocks, st)
+                 : launch_wide_grouped<1>(a, epi, (unsigned)blocks, st);
+}
 
 int64_t q4_wide_tiles(int M, int N, int ncols, int epi) {
   const bool swiglu = epi >= 3 && epi <= 5;

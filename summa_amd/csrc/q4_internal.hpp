@@ -37,6 +37,12 @@ int splitk_reduce(const float* part, int ks, int M, int N, int ncols, void* y, i
 int q4_gemm_wide(const uint8_t* codes, const uint16_t* scales, int N, int K, const void* x,
                  int xt, int M, int ldx, void* y, int ldy, int epi, int ncols, hipStream_t st,
                  const QkvRope* qr);
+// The same kernel over a route plan's experts (offsets goff; gathered rows when
+// rowidx).
+int q4_gemm_wide_grouped(const uint8_t* codes, const uint16_t* scales, int N, int K, const void* x,
+                         int xt, int routes, int experts, int ldx, void* y, int ldy, int epi,
+                         int ncols, const int32_t* goff, const int32_t* rowidx, size_t cstride,
+                         size_t sstride, hipStream_t st);
 int64_t q4_wide_tiles(int M, int N, int ncols, int epi);
 
 }  // namespace sm
