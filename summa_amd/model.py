@@ -14,6 +14,7 @@ import torch
 
 from . import _lib
 from ._lib import call
+from .ops import _stream
 
 # tensor kinds (include/summa_amd.h SM_W_*)
 KIND = {"embed": 0, "attn_norm": 1, "qkv": 2, "o": 3, "ffn_norm": 4, "in": 5, "down": 6,
@@ -57,10 +58,6 @@ class ModelConfig:
         if self.experts:
             cfg.update(E=self.experts, Fe=self.expert_ffn)
         return cfg
-
-
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
 
 
 class Model:

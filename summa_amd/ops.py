@@ -17,7 +17,13 @@ _DTYPES = {torch.float32: SM_F32, torch.bfloat16: SM_BF16, torch.float16: SM_F16
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """Handle of the current device's current stream, as
+    ``torch.cuda.current_stream().cuda_stream`` gives it, without the Stream
+    object and the device look-ups behind it (7 us a call, as long as a small
+    kernel; four projections of a decoder layer at M 8 take 41 -> 31 us a pass)."""
+    if not torch.cuda.is_initialized():
+        torch.cuda.init()
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _dt(t: torch.Tensor) -> int:

@@ -23,6 +23,7 @@ import torch
 from . import ops
 from ._lib import SM_F32, call
 from .model import Model, ModelConfig
+from .ops import _stream as _st
 
 LAYER_KEYS = ("attn_norm", "qkv", "o", "ffn_norm", "in", "down")
 # per-layer tensors of an MoE policy (stacked experts, the f32 router)
@@ -31,10 +32,6 @@ MUON_MOMENTUM = 0.95                       # muon.rs:10
 NS_COEFFICIENTS = (3.4445, -4.775, 2.0315)  # muon.rs:11
 NS_STEPS = 5                               # muon.rs:12
 MUON_EPSILON = 1e-7                        # muon.rs:13
-
-
-def _st() -> int:
-    return torch.cuda.current_stream().cuda_stream
 
 
 def gemm(a, b, *, ta=False, tb=False, out=None, alpha=1.0, beta=0.0, entry="sm_gemm_ex"):
