@@ -445,6 +445,14 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_pairs_kernel(PairArgs g)
         if (!whole && col >= g.N) continue;
         const int sb = F16 ? scale_shift(bmax[col]) : 0;
         const float bias = g.bias ? g.bias[col] : 0.f;
+        float old[16];  // read together: a read behind a write of C waits for it
+        if (g.beta != 0.f && !(MODE == kPlain && g.splits > 1)) {
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            const int row = rb + 8 * (e / 4) + e % 4;
+            if (whole || row < M) old[e] = C[(int64_t)row * g.ldc + col];
+          }
+        }
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
           const int row = rb + 8 * (e / 4) + e % 4;
@@ -454,9 +462,8 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_pairs_kernel(PairArgs g)
             g.part[((int64_t)z * M + row) * g.N + col] = v;
             continue;
           }
-          float* o = C + (int64_t)row * g.ldc + col;
-          const float w = g.beta == 0.f ? g.alpha * v : fmaf(g.alpha, v, g.beta * *o);
-          *o = g.bias ? w + bias : w;
+          const float w = g.beta == 0.f ? g.alpha * v : fmaf(g.alpha, v, g.beta * old[e]);
+          C[(int64_t)row * g.ldc + col] = g.bias ? w + bias : w;
         }
       }
     }

@@ -249,12 +249,15 @@ __global__ __launch_bounds__(512, 1) void q4_gemm_wide_kernel(WideArgs a) {
     // RoPE pairs (2p, 2p+1) are adjacent columns, i.e. lanes j and j^1: every
     // lane takes part in the swap, even lanes store the rotated pair. Row
     // positions are computed here (once per tile, after the long K loop).
+    // Two rows at a time: each lane hands its neighbour the value it needs, so the
+    // even lane holds a whole pair of row r and the odd one of row r + 1.
     const int hd_shift = __builtin_ctz(a.hd);
+    const bool odd = j & 1;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = m0 + wr * 64 + mt * 16 + 4 * g + r;
+      for (int r = 0; r < 4; r += 2) {
+        const int row = m0 + wr * 64 + mt * 16 + 4 * g + r + (odd ? 1 : 0);
         const int rc = min(row, a.M - 1);
         const int sq = (a.rope_L == 1) ? rc : rc / a.rope_L;
         const int pos = a.pos0[sq] + (rc - sq * a.rope_L);
@@ -262,10 +265,11 @@ __global__ __launch_bounds__(512, 1) void q4_gemm_wide_kernel(WideArgs a) {
         const float2* rrow = a.rope + (size_t)(ok ? pos : 0) * (a.hd / 2);
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
-          const float va = acc[mt][b][r];
-          const float vb = __shfl_xor(va, 1, kWave);  // column e + 1
-          const int col = tn * kWN + wc * 128 + b * 16 + j;
-          if (!ok || (j & 1) || col >= a.N) continue;
+          const float got = dpp_f32<kDppXor1>(odd ? acc[mt][b][r] : acc[mt][b][r + 1]);
+          const float va = odd ? got : acc[mt][b][r];
+          const float vb = odd ? acc[mt][b][r + 1] : got;
+          const int col = tn * kWN + wc * 128 + b * 16 + (j & ~1);
+          if (!ok || col >= a.N) continue;
           const int slot = col >> hd_shift, e = col & (a.hd - 1);
           h2 out;
           _Float16* dst;
@@ -282,6 +286,30 @@ __global__ __launch_bounds__(512, 1) void q4_gemm_wide_kernel(WideArgs a) {
           *reinterpret_cast<h2*>(dst) = out;
         }
       }
+    return;
+  }
+  if constexpr (EPI == 2) {
+    // a row block's outputs are read together before any is written: a read
+    // after a write of the same array waits for its turn (49024 x 768 x 768 242 ->
+    // 194 us, x 3072 604 -> 515; 65408 x 2048 x 2048 1240 -> 1014)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      float* yp = static_cast<float*>(a.y);
+      float old[4][NB];
+      auto each = [&](auto f) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int row = m0 + wr * 64 + mt * 16 + 4 * g + r;
+#pragma unroll
+          for (int b = 0; b < NB; ++b) {
+            const int col = tn * kWN + wc * 128 + b * 16 + j;
+            if (row < mlim && col < a.N) f(r, b, yp + (size_t)row * a.ldy + col);
+          }
+        }
+      };
+      each([&](int r, int b, float* o) { old[r][b] = *o; });
+      each([&](int r, int b, float* o) { *o = old[r][b] + acc[mt][b][r]; });
+    }
     return;
   }
 #pragma unroll
@@ -317,7 +345,6 @@ __global__ __launch_bounds__(512, 1) void q4_gemm_wide_kernel(WideArgs a) {
           const float v = acc[mt][b][r];
           if constexpr (EPI == 0) static_cast<float*>(a.y)[o] = v;
           else if constexpr (EPI == 1) static_cast<uint16_t*>(a.y)[o] = f32_to_bf16(v);
-          else static_cast<float*>(a.y)[o] += v;
         }
       }
     }
