@@ -81,6 +81,14 @@ int sm_moe_combine(const float*, const float*, const int32_t*, int64_t, int64_t,
 }
 
 namespace sm {
+// gemm_f32.hip: fp32 decode projections with the step that follows them
+bool f32_fused_fits(int64_t M, int64_t N);
+int f32_swiglu(const float* w, const float* x, int64_t M, int64_t F, int64_t K, float* y,
+               hipStream_t st);
+int f32_qkv_rope(const float* w, const float* x, int64_t S, int64_t L, int64_t H, int64_t KVH,
+                 int64_t hd, int64_t K, const float* rope, const int32_t* pos0, int64_t cap,
+                 float* q, float* kc, float* vc, hipStream_t st);
+
 namespace {
 
 // A workspace buffer of the model: grow-only device memory the model
@@ -394,6 +402,8 @@ int linear_swiglu(sm_model* m, const Linear& L, const void* x, int64_t M, void* 
                   hipStream_t st) {
   if (m->cfg.quantized)
     return q4_linear(m, L, x, M, u, m->act_ld(L.N / 2), SM_EPI_SWIGLU_F16X2, st);
+  if (f32_fused_fits(M, L.N / 2))
+    return f32_swiglu(L.w, (const float*)x, M, L.N / 2, L.K, (float*)u, st);
   SM_TRY(ensure(m->gv, (size_t)M * L.N * 4));
   SM_TRY(sm_gemm_f32(L.w, L.N, L.K, (const float*)x, M, L.K, (float*)m->gv.p, L.N,
                      SM_EPI_STORE_F32, st));
@@ -527,6 +537,9 @@ int run_layers(sm_model* m, const int32_t* ids, int64_t S, int64_t L, const int3
       SM_TRY(sm_q4_qkv_rope(Ly.qkv.codes, Ly.qkv.scales, c.heads, c.kv_heads, c.head_dim, d,
                             m->h.p, m->act, S, L, m->act_ld(d), m->rope, pos0, cap, m->qb.p, kl,
                             vl, m->kvt, st));
+    } else if (f32_fused_fits(rows, m->qkv_n)) {
+      SM_TRY(f32_qkv_rope(Ly.qkv.w, (const float*)m->h.p, S, L, c.heads, c.kv_heads, c.head_dim, d,
+                          m->rope, pos0, cap, (float*)m->qb.p, (float*)kl, (float*)vl, st));
     } else {
       SM_TRY(linear_f32out(m, Ly.qkv, m->h.p, rows, (float*)m->qkv.p, false, st));
       SM_TRY(sm_rope_append((const float*)m->qkv.p, m->rope, pos0, S, L, c.heads, c.kv_heads,

@@ -64,3 +64,22 @@ def test_small_gemm_ex_matches_f64(dev, ta, tb, M, N, K, pad):
     want = 0.5 * (a64 @ b64) + 2.0 * c0
     mag = 0.5 * (np.abs(a64) @ np.abs(b64)) + 2.0 * np.abs(c0)
     assert (np.abs(got - want) <= (K + 3) * 2.0 ** -24 * mag).all()
+
+
+@pytest.mark.parametrize("d,heads,kv_heads,hd,ffn,vocab", [(256, 4, 2, 64, 1024, 1000),
+                                                           (132, 2, 1, 64, 200, 333)])
+def test_fp32_decode_batches_equal_larger_ones(dev, d, heads, kv_heads, hd, ffn, vocab):
+    """Few rows run SwiGLU, RoPE and the cache append inside their projections,
+    more rows the separate kernels: the log-probs of the same sequences are the
+    same bits."""
+    from summa_amd.model import Model, ModelConfig
+    cfg = ModelConfig(layers=2, d_model=d, heads=heads, kv_heads=kv_heads, head_dim=hd, ffn=ffn,
+                      vocab=vocab, max_seq=40, quantized=False)
+    m = Model(cfg)
+    m.init_random(3, std=0.05)
+    gen = torch.Generator().manual_seed(2)
+    prompts = torch.randint(0, vocab, (600, 5), generator=gen, dtype=torch.int32).to(dev)
+    tokens = torch.randint(0, vocab, (600, 20), generator=gen, dtype=torch.int32).to(dev)
+    many = m.logprobs(prompts, tokens)  # 14400 rows: more than 4096 8 x 8 tiles
+    few = torch.cat([m.logprobs(prompts[i:i + 1], tokens[i:i + 1]) for i in (0, 1, 599)])
+    assert torch.equal(few, many[[0, 1, 599]])
