@@ -11,8 +11,7 @@
 // ldexp per output. Three MFMAs per f32 product against the six of three
 // bf16 planes, and half as many f32 additions, which is where such a product's
 // error comes from: over K 512 to 32768 its distance to float64 is no larger
-// (measured beside each caller). Values of at most 11 bits (a 4-bit code times a
-// bf16 scale) need one plane: two MFMAs.
+// (measured beside each caller).
 // bf16 forms: one, two or three unscaled bf16 planes, the plane products of
 // gemm_mfma.hip in its order (the same bits) with the split taken out of the K
 // loop.
@@ -60,7 +59,7 @@ template <Split F>
 __device__ inline void store8(char* row, int64_t k, const float* v, int shift) {
   constexpr int P = F == Split::kBf16x3 ? 3 : F == Split::kPair || F == Split::kBf16x2 ? 2 : 1;
   u32x4 w[P];
-  if constexpr (F == Split::kF16 || F == Split::kPair) {
+  if constexpr (F == Split::kPair) {
     h8 h, l;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -69,7 +68,7 @@ __device__ inline void store8(char* row, int64_t k, const float* v, int shift) {
       l[i] = (_Float16)(x - (float)h[i]);
     }
     w[0] = __builtin_bit_cast(u32x4, h);
-    if constexpr (P > 1) w[1] = __builtin_bit_cast(u32x4, l);
+    w[1] = __builtin_bit_cast(u32x4, l);
   } else {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -126,7 +125,7 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict
       if (k < Kp) load8(k, v[i]);
     }
   }
-  if constexpr (F == Split::kF16 || F == Split::kPair) {
+  if constexpr (F == Split::kPair) {
     uint32_t m = 0;  // magnitudes as bits: NaN above infinity above all finite
     if (live) {
 #pragma unroll
@@ -224,7 +223,7 @@ __global__ __launch_bounds__(256) void split_cols_kernel(const float* __restrict
     float v[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = t[kl + e][rl];
-    const int shift = (F == Split::kF16 || F == Split::kPair) ? scale_shift(amax[r0 + rl]) : 0;
+    const int shift = F == Split::kPair ? scale_shift(amax[r0 + rl]) : 0;
     store8<F>(out + (r0 + rl) * row_bytes, kb * 64 + kl, v, shift);
   }
 }
@@ -271,7 +270,6 @@ template <> struct Products<3, 2> {
 template <> struct Products<2, 2> {
   static constexpr int n = 3, a[3] = {1, 0, 0}, b[3] = {0, 1, 0};
 };
-template <> struct Products<2, 1> { static constexpr int n = 2, a[2] = {1, 0}, b[2] = {0, 0}; };
 template <> struct Products<1, 1> { static constexpr int n = 1, a[1] = {0}, b[1] = {0}; };
 
 template <bool F16>
@@ -511,8 +509,7 @@ int launch(const SplitOperand& A, const SplitOperand& B, PairArgs& g, int64_t wg
   if constexpr (MODE == kPlain) {
     if (A.form == Split::kBf16x2) SM_GP(false, 2, 2, 32);
     else if (A.form == Split::kBf16) SM_GP(false, 1, 1, 64);
-    else if (A.form == Split::kPair && B.form == Split::kPair) SM_GP(true, 2, 2, 32);
-    else if (A.form == Split::kPair) SM_GP(true, 2, 1, 32);
+    else if (A.form == Split::kPair) SM_GP(true, 2, 2, 32);
   }
 #undef SM_GP
   SM_LAUNCH_CHECK();
@@ -534,7 +531,8 @@ PairArgs pair_args(const SplitOperand& A, const SplitOperand& B) {
 }
 
 // The tile and the K splits of an M x N x K product: rounds of workgroups over
-// the chip times the time of a round, ns per k measured at full rounds (`ns`;
+// the chip times the time of a round, ns per k measured at full rounds (`ns1` for
+// one product, `ns3` for three, more in proportion;
 // 1.05-1.2 PF/s of MFMA work, set by power rather than by the tile), less where
 // a round leaves CUs idle (0.6 of it for the large tiles with few busy, half for
 // the 128 x 128 ones, two of which share a CU). A split writes and reads its
@@ -544,17 +542,15 @@ PairArgs pair_args(const SplitOperand& A, const SplitOperand& B) {
 // 167. One bf16 product: 4096 x 2048 x 65536 1598, 1350, 1112.
 struct Tile {
   int bm, bn, slots;  // slots: workgroups the chip runs at once
-  double ns[3];       // 1, 2 and 3 products; more in proportion
+  double ns1, ns3;
 };
-constexpr Tile kTiles[] = {{256, 256, kCUs, {34, 57, 85}},
-                           {128, 256, kCUs, {20, 30.5, 46}},
-                           {128, 128, 2 * kCUs, {18.5, 33, 47.5}}};
+constexpr Tile kTiles[] = {
+    {256, 256, kCUs, 34, 85}, {128, 256, kCUs, 20, 46}, {128, 128, 2 * kCUs, 18.5, 47.5}};
 struct Plan {
   int tile, splits;
 };
 Plan pair_plan(Split a, Split b, int64_t M, int64_t N, int64_t K) {
   const bool three = a == Split::kBf16x3;
-  const int form = a == Split::kBf16 ? 0 : b == Split::kF16 ? 1 : 2;
   const double products = !three ? 1.0 : b == Split::kBf16x3 ? 2.0 : 5.0 / 3.0;
   Plan best{0, 1};
   double least = 0;
@@ -569,7 +565,7 @@ Plan pair_plan(Split a, Split b, int64_t M, int64_t N, int64_t K) {
       const double rounds = (double)ceil_div(tiles * s, slots);
       const double full = tiles * s / (rounds * slots);
       const double part = slots > kCUs ? std::max(0.53, 0.1 + 0.9 * full) : 0.6 + 0.4 * full;
-      const double ns = rounds * ((double)K / s * t.ns[form] * products / half * part + 4000) +
+      const double ns = rounds * ((double)K / s * (a == Split::kBf16 ? t.ns1 : t.ns3) * products / half * part + 4000) +
                         (s > 1 ? (double)s * M * N * 8 / 4000 + 5000 : 0);
       if (least == 0 || ns < 0.98 * least) {
         least = ns;
@@ -630,7 +626,6 @@ int split_operand(const SplitOperand& o, const float* X, int64_t ld, bool kc, in
   if (o.rows == 0 || o.kp == 0) return SM_OK;
   switch (o.form) {
     case Split::kBf16: return split_fill<Split::kBf16>(o, X, ld, kc, K, st, runs, batch);
-    case Split::kF16: return split_fill<Split::kF16>(o, X, ld, kc, K, st, runs, batch);
     case Split::kBf16x2: return split_fill<Split::kBf16x2>(o, X, ld, kc, K, st, runs, batch);
     case Split::kBf16x3: return split_fill<Split::kBf16x3>(o, X, ld, kc, K, st, runs, batch);
     default: return split_fill<Split::kPair>(o, X, ld, kc, K, st, runs, batch);

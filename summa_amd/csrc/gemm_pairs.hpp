@@ -10,15 +10,14 @@ namespace sm {
 
 // How a split operand holds its values.
 // kBf16: rounded to bf16, one plane (the one-plane policy's operands).
-// kF16: one f16 plane of x 2^s, s from the row's largest magnitude: exact for
-//   values of at most 11 significant bits (a 4-bit code times a bf16 scale).
-// kPair: x 2^s = hi + lo, two f16 planes, about 22 significant bits.
+// kPair: x 2^s = hi + lo, two f16 planes, about 22 significant bits; s from the
+//   row's largest magnitude.
 // kBf16x2, kBf16x3: the leading two or three bf16 planes of x (three: exact).
-enum class Split { kBf16, kF16, kPair, kBf16x2, kBf16x3 };
+enum class Split { kBf16, kPair, kBf16x2, kBf16x3 };
 inline int planes_of(Split f) {
   return f == Split::kBf16x3 ? 3 : f == Split::kPair || f == Split::kBf16x2 ? 2 : 1;
 }
-inline bool scaled(Split f) { return f == Split::kF16 || f == Split::kPair; }
+inline bool scaled(Split f) { return f == Split::kPair; }
 
 // Consecutive runs of the grouped forms: run i covers `cnt[i]` rows (or k)
 // from `off[i]` of the dense operand.
@@ -51,8 +50,8 @@ bool pairs_fit(int64_t K);
 int split_operand(const SplitOperand& o, const float* X, int64_t ld, bool kc, int64_t K,
                   hipStream_t st, const Runs* runs = nullptr, int64_t batch = 1);
 
-// C = alpha A B^T + beta C (+ bias along n) from split operands: kPair with kPair
-// or kF16, kBf16 with itself, kBf16x2 with itself, kBf16x3 with itself or kBf16x2.
+// C = alpha A B^T + beta C (+ bias along n) from split operands: each form with
+// itself, or kBf16x3 with kBf16x2.
 // part (nullable): room for split-K partial sums, part_floats floats; without
 // it, or where it is too small, K is not split.
 int gemm_pairs(const SplitOperand& A, const SplitOperand& B, int64_t M, int64_t N, float alpha,
