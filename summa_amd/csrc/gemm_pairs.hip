@@ -21,11 +21,12 @@
 // whole lines.
 //
 // gemm_pairs_kernel: a BM x BN tile per workgroup, 8 waves (4 for 128 x 128), 2
-// waves per SIMD; two LDS stages filled by global_load_lds (16 bytes a lane, no registers): the next
-// stage's copies are issued right after the barrier and land during the
-// current one's MFMAs. 16-byte chunk c of row r lies at c ^ f(r), f chosen so
-// that the 32-row fragment reads spread over all banks; the copy permutes its
-// global addresses instead, as its LDS side is always consecutive.
+// waves per SIMD; two LDS stages filled by global_load_lds (16 bytes a lane, no
+// registers): the next stage's copies are issued right after the barrier and
+// land during the current one's MFMAs. 16-byte chunk c of row r lies at
+// c ^ f(r), f chosen so that the 32-row fragment reads spread over all banks;
+// the copy permutes its global addresses instead, as its LDS side is always
+// consecutive.
 #include "gemm_pairs.hpp"
 
 #include <algorithm>
@@ -170,16 +171,33 @@ __global__ __launch_bounds__(256) void zero_u32_kernel(uint32_t* __restrict__ p,
   if (i < n) p[i] = 0;
 }
 
-// column maxima of X [K][ld] over 64-row slices; the atomic max of magnitude
-// bits does not depend on the order
+// The rows [k0, k1) of X behind 64-k block kb of the split operand, and their run.
+__device__ inline int block_rows(int64_t kb, int64_t K, int use_runs, const Runs& runs,
+                                 int64_t& k0, int64_t& k1) {
+  k0 = kb * 64;
+  k1 = K;
+  if (!use_runs) return 0;
+  int e = 0;
+  while (kb >= (runs.cnt[e] + 63) / 64) kb -= (runs.cnt[e++] + 63) / 64;
+  k0 = runs.off[e] + kb * 64;
+  k1 = runs.off[e] + runs.cnt[e];
+  return e;
+}
+
+// column maxima of X [K][ld], a 64-k block per workgroup; the atomic max of
+// magnitude bits does not depend on the order. Runs have their own maxima: one
+// expert's large or infinite values leave the others' precision alone.
 __global__ __launch_bounds__(256) void col_amax_kernel(const float* __restrict__ X, int64_t ld,
                                                        int64_t R, int64_t K,
-                                                       uint32_t* __restrict__ amax) {
+                                                       uint32_t* __restrict__ amax,
+                                                       int use_runs, Runs runs) {
   const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (r >= R) return;
   X += blockIdx.z * K * ld;
   amax += blockIdx.z * R;
-  const int64_t k0 = (int64_t)blockIdx.y * 64, k1 = min(k0 + 64, K);
+  int64_t k0, k1;
+  amax += block_rows(blockIdx.y, K, use_runs, runs, k0, k1) * R;
+  k1 = min(k0 + 64, k1);
   uint32_t m = 0;
 #pragma unroll 8
   for (int64_t k = k0; k < k1; ++k) m = max(m, __float_as_uint(X[k * ld + r]) & 0x7fffffffu);
@@ -201,14 +219,8 @@ __global__ __launch_bounds__(256) void split_cols_kernel(const float* __restrict
   X += blockIdx.z * K * ld;
   out += blockIdx.z * R * row_bytes;
   amax += blockIdx.z * R;
-  int64_t k0 = kb * 64, k1 = K;
-  if (use_runs) {
-    int64_t b = kb;
-    int e = 0;
-    while (b >= (runs.cnt[e] + 63) / 64) b -= (runs.cnt[e++] + 63) / 64;
-    k0 = runs.off[e] + b * 64;
-    k1 = runs.off[e] + runs.cnt[e];
-  }
+  int64_t k0, k1;
+  amax += block_rows(kb, K, use_runs, runs, k0, k1) * R;
   const int tx = threadIdx.x % 64, ty = threadIdx.x / 64;
 #pragma unroll 4
   for (int i = ty; i < 64; i += 4) {
@@ -299,7 +311,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_pairs_kernel(PairArgs g)
 
   int tm, tn, z = 0, M = g.M, s0 = 0, s1 = g.nst, arow0 = 0;
   const char* Bp = g.B;
-  const uint32_t* bmax = g.bmax;
+  const uint32_t *amax = g.amax, *bmax = g.bmax;
   float* C = g.C;
   if constexpr (MODE == kPlain) {
     const int per = g.ntm * g.ntn;
@@ -326,6 +338,8 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_pairs_kernel(PairArgs g)
     for (int i = 0; i < e; ++i) s0 += (g.runs.cnt[i] + 63) / 64 * (64 / BK);
     s1 = s0 + (g.runs.cnt[e] + 63) / 64 * (64 / BK);
     C += (int64_t)e * g.stride;
+    amax += (int64_t)e * g.M;
+    bmax += (int64_t)e * g.N;
   }
   const int m0 = tm * BM, n0 = tn * BN;
 
@@ -434,7 +448,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_pairs_kernel(PairArgs g)
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
           const int row = rb + 8 * (e / 4) + e % 4;
-          sa[e] = scale_shift(g.amax[arow0 + (whole ? row : min(row, M - 1))]);
+          sa[e] = scale_shift(amax[arow0 + (whole ? row : min(row, M - 1))]);
         }
       }
 #pragma unroll
@@ -565,7 +579,8 @@ Plan pair_plan(Split a, Split b, int64_t M, int64_t N, int64_t K) {
       const double rounds = (double)ceil_div(tiles * s, slots);
       const double full = tiles * s / (rounds * slots);
       const double part = slots > kCUs ? std::max(0.53, 0.1 + 0.9 * full) : 0.6 + 0.4 * full;
-      const double ns = rounds * ((double)K / s * (a == Split::kBf16 ? t.ns1 : t.ns3) * products / half * part + 4000) +
+      const double per_k = (a == Split::kBf16 ? t.ns1 : t.ns3) * products / half * part;
+      const double ns = rounds * ((double)K / s * per_k + 4000) +
                         (s > 1 ? (double)s * M * N * 8 / 4000 + 5000 : 0);
       if (least == 0 || ns < 0.98 * least) {
         least = ns;
@@ -580,10 +595,10 @@ Plan pair_plan(Split a, Split b, int64_t M, int64_t N, int64_t K) {
 
 bool pairs_fit(int64_t K) { return K <= ((int64_t)1 << 21); }
 
-int64_t split_bytes(Split form, int64_t rows, int64_t K) {
+int64_t split_bytes(Split form, int64_t rows, int64_t K, int64_t runs) {
   const SplitOperand o = split_place(form, rows, K, nullptr);
   const int64_t data = ceil_div(rows * o.row_bytes(), 256) * 256;
-  return data + (scaled(form) ? ceil_div(rows * 4, 256) * 256 : 0);
+  return data + (scaled(form) ? ceil_div(runs * rows * 4, 256) * 256 : 0);
 }
 
 SplitOperand split_place(Split form, int64_t rows, int64_t K, void* buf) {
@@ -608,9 +623,11 @@ int split_fill(const SplitOperand& o, const float* X, int64_t ld, bool kc, int64
                                                              o.amax, vec);
   } else {
     if (scaled(F)) {
-      zero_u32_kernel<<<(unsigned)ceil_div(o.rows, 256), 256, 0, st>>>(o.amax, o.rows);
-      const dim3 grid((unsigned)ceil_div(R, 256), (unsigned)ceil_div(K, 64), (unsigned)batch);
-      col_amax_kernel<<<grid, 256, 0, st>>>(X, ld, R, K, o.amax);
+      const int64_t n = (runs ? runs->n : 1) * o.rows;
+      zero_u32_kernel<<<(unsigned)ceil_div(n, 256), 256, 0, st>>>(o.amax, n);
+      const dim3 grid((unsigned)ceil_div(R, 256), (unsigned)(o.kp / 64), (unsigned)batch);
+      col_amax_kernel<<<grid, 256, 0, st>>>(X, ld, R, K, o.amax, runs ? 1 : 0,
+                                            runs ? *runs : Runs{});
     }
     const dim3 grid((unsigned)(o.kp / 64), (unsigned)ceil_div(R, 64), (unsigned)batch);
     split_cols_kernel<F><<<grid, 256, 0, st>>>(X, ld, R, K, o.data, rb, o.amax,

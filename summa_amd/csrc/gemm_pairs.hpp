@@ -33,11 +33,11 @@ struct Runs {
 struct SplitOperand {
   Split form;
   char* data;
-  uint32_t* amax;  // bits of each row's largest |x| (the scaled forms)
+  uint32_t* amax;  // bits of each row's largest |x| (the scaled forms; of runs: [run][row])
   int64_t rows, kp;
   int64_t row_bytes() const { return kp * 2 * planes_of(form); }
 };
-int64_t split_bytes(Split form, int64_t rows, int64_t K);
+int64_t split_bytes(Split form, int64_t rows, int64_t K, int64_t runs = 1);
 SplitOperand split_place(Split form, int64_t rows, int64_t K, void* buf);
 
 // Whether K is in the kernel's range (a tile's rows lie within 4 GB).
@@ -45,7 +45,7 @@ bool pairs_fit(int64_t K);
 
 // Fills `o` from X: element (r, k) at X[r * ld + k] (kc) or X[k * ld + r]. With
 // `runs` (not kc), the runs' k follow each other, each padded with zeros to whole
-// 64s (K: their sum). With `batch` > 1 (not kc), X holds that many matrices,
+// 64s and with its own row maxima. With `batch` > 1 (not kc), X holds that many matrices,
 // K * ld apart, whose rows / batch rows each follow each other.
 int split_operand(const SplitOperand& o, const float* X, int64_t ld, bool kc, int64_t K,
                   hipStream_t st, const Runs* runs = nullptr, int64_t batch = 1);

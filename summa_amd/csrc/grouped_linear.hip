@@ -95,9 +95,11 @@ int64_t forward_bytes(int64_t experts, int64_t routes, int64_t d_in, int64_t d_o
 int64_t backward_bytes(int64_t experts, int64_t routes, int64_t d_in, int64_t d_out) {
   if (!grouped_split_sizes(routes, d_in, d_out, experts)) return 0;
   const int64_t kp = routes + 64 * experts;  // every run padded to whole 64s
+  const int64_t runs = std::min<int64_t>(experts, kMaxRuns);
   return std::max(split_bytes(Split::kPair, routes, d_out) +
                       split_bytes(Split::kPair, experts * d_in, d_out),
-                  split_bytes(Split::kPair, d_in, kp) + split_bytes(Split::kPair, d_out, kp));
+                  split_bytes(Split::kPair, d_in, kp, runs) +
+                      split_bytes(Split::kPair, d_out, kp, runs));
 }
 
 bool use_split(const GroupedWs& ws, int64_t need) {
@@ -178,9 +180,7 @@ int grouped_backward_split(const float* x, const float* w, const float* grad,
       for (int i = 0; i < r.n; ++i) kp += ceil_div(r.cnt[i], 64) * 64;
       const SplitOperand a = split_place(Split::kPair, d_in, kp, at);
       const SplitOperand b =
-          split_place(Split::kPair, d_out, kp, at + split_bytes(Split::kPair, d_in, kp));
-      // (the runs are consecutive rows of x: their maxima are taken over rows
-      // r.off[0] on, which the shifted base and K give)
+          split_place(Split::kPair, d_out, kp, at + split_bytes(Split::kPair, d_in, kp, r.n));
       const int64_t rows = r.off[r.n - 1] + r.cnt[r.n - 1] - r.off[0];
       Runs local = r;
       for (int i = 0; i < r.n; ++i) local.off[i] -= r.off[0];

@@ -45,11 +45,29 @@ def test_grouped_linear_split_matches_f64(dev, counts, din, dout):
             continue
         assert ((ye - xe @ we).abs() <= _bound(din) * (xe.abs() @ we.abs())).all(), e
         assert ((gxe - de @ we.T).abs() <= _bound(dout) * (de.abs() @ we.abs().T)).all(), e
-        # a column of x or dy is scaled by its largest value over every expert's
+        # a column of x or dy is scaled by its largest value over the expert's
         # rows, 2^-39 of which bounds what the pairs drop of smaller ones
         mag = xe.abs().T @ de.abs()
-        floor = c * 2.0 ** -38 * (x.abs().amax(0).double()[:, None] * dy.abs().amax(0).double())
+        floor = c * 2.0 ** -38 * (xe.abs().amax(0)[:, None] * de.abs().amax(0))
         assert ((gw[e].double() - xe.T @ de).abs() <= _bound(c) * mag + floor).all(), e
+
+
+def test_grouped_weight_gradient_keeps_experts_apart(dev):
+    """An expert whose rows are infinite, and one whose rows are 2^40 larger,
+    change nothing in the other experts' weight gradients."""
+    counts, din, dout = [200, 130, 300, 64], 224, 260
+    assert sum(counts) * din * dout >= 1 << 25
+    g = torch.Generator(device=dev).manual_seed(7)
+    x = torch.randn(sum(counts), din, generator=g, device=dev)
+    w = torch.randn(len(counts), din, dout, generator=g, device=dev)
+    dy = torch.randn(sum(counts), dout, generator=g, device=dev)
+    want = ops.grouped_linear_backward(x, w, dy, counts)[1]
+    x[210] = float("inf")
+    x[330:630] *= 2.0 ** 40
+    got = ops.grouped_linear_backward(x, w, dy, counts)[1]
+    assert not torch.isfinite(got[1]).any()
+    assert torch.equal(got[2], want[2] * 2.0 ** 40)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[3], want[3])
 
 
 def test_grouped_swiglu_mlp_split_matches_small_problem_path(dev):
