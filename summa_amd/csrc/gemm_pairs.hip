@@ -2,28 +2,22 @@
 // large f32 products of training (the policy's forward, data and weight
 // gradients, the linear head + cross-entropy, the MoE expert projections).
 //
-// f32-grade form. A row of op(A) (a column of op(B)) is scaled by a power of two
-// that puts its largest magnitude into [2^14, 2^15) and written as two f16
-// planes, x 2^s = hi + lo: 22 significant bits for every element within 2^-18
-// of its row's largest, and an absolute error of 2^-39 of that largest for
-// the rest. A product is lo.hi + hi.lo + hi.hi in f32 (v_mfma_f32_32x32x16_f16,
-// smallest first; lo.lo is below 2^-22), the scales are undone by one exact
-// ldexp per output. Three MFMAs per f32 product against the six of three
-// bf16 planes, and half as many f32 additions, which is where such a product's
-// error comes from: over K 512 to 32768 its distance to float64 is no larger
-// (measured beside each caller).
-// bf16 forms: one, two or three unscaled bf16 planes, the plane products of
-// gemm_mfma.hip in its order (the same bits) with the split taken out of the K
-// loop.
+// Forms: one, two or three unscaled bf16 planes, the plane products of
+// gemm_mfma.hip with the split taken out of the K loop, in its order (the same bits)
+// unless the caller lets the sums be more exact. Three planes hold every f32 exactly,
+// whatever its row holds beside it. (Two f16 planes on a power-of-two scale of the row
+// or column took three products instead of six, and 0.7 of the time, but held 22 bits,
+// and fewer of values below 2^-18 of their row's largest: a row that a zero factor
+// took out of the sum erased the others.)
 //
 // Layout of a split operand: per row, one plane: its k in order; more: per 32 k
 // the planes' 64 bytes one after the other. A stage of the K loop then reads
 // whole lines.
 //
-// gemm_pairs_kernel: a BM x BN tile per workgroup, 8 waves (4 for 128 x 128), 2
-// waves per SIMD; two LDS stages filled by global_load_lds (16 bytes a lane, no
-// registers): the next stage's copies are issued right after the barrier and
-// land during the current one's MFMAs. 16-byte chunk c of row r lies at
+// gemm_pairs_kernel: a BM x BN tile per workgroup, 8 waves (4 for the dense 128 x 128,
+// two of which share a CU where their planes leave the LDS for it); two LDS stages
+// filled by global_load_lds (16 bytes a lane, no registers): the next stage's copies
+// are issued right after the barrier and land during the current one's MFMAs. 16-byte chunk c of row r lies at
 // c ^ f(r), f chosen so that the 32-row fragment reads spread over all banks;
 // the copy permutes its global addresses instead, as its LDS side is always
 // consecutive.
@@ -43,43 +37,21 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kCUs = 256;
 
-// The power of two that a row of largest magnitude `bits` is scaled by:
-// 2^(14 - floor(log2)); 1 for a zero row and for one with an infinity or a NaN
-// (whose outputs are NaN either way).
-__host__ __device__ inline int scale_shift(uint32_t bits) {
-  if (bits == 0 || bits >= 0x7f800000u) return 0;
-  const int e = (int)(bits >> 23);
-  if (e > 0) return 14 - (e - 127);
-  return 14 - (31 - __builtin_clz(bits) - 149);  // denormal: by its leading bit
-}
-
 // ------------------------------------------------------------------ split --
 
 // 8 consecutive values of a row at k (a multiple of 8) -> 16 bytes per plane
 template <Split F>
-__device__ inline void store8(char* row, int64_t k, const float* v, int shift) {
-  constexpr int P = F == Split::kBf16x3 ? 3 : F == Split::kPair || F == Split::kBf16x2 ? 2 : 1;
+__device__ inline void store8(char* row, int64_t k, const float* v) {
+  constexpr int P = planes_of(F);
   u32x4 w[P];
-  if constexpr (F == Split::kPair) {
-    h8 h, l;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float x = ldexpf(v[i], shift);
-      h[i] = (_Float16)x;
-      l[i] = (_Float16)(x - (float)h[i]);
-    }
-    w[0] = __builtin_bit_cast(u32x4, h);
-    w[1] = __builtin_bit_cast(u32x4, l);
-  } else {
+  for (int i = 0; i < 4; ++i) {
+    float a = v[2 * i], b = v[2 * i + 1];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      float a = v[2 * i], b = v[2 * i + 1];
-#pragma unroll
-      for (int p = 0; p < P; ++p) {
-        w[p][i] = pack_bf16x2(a, b);
-        a -= bf16lo(w[p][i]);
-        b -= bf16hi(w[p][i]);
-      }
+    for (int p = 0; p < P; ++p) {
+      w[p][i] = pack_bf16x2(a, b);
+      a -= bf16lo(w[p][i]);
+      b -= bf16hi(w[p][i]);
     }
   }
   char* o = row + (P == 1 ? k * 2 : k / 32 * (64 * P) + k % 32 * 2);
@@ -88,120 +60,55 @@ __device__ inline void store8(char* row, int64_t k, const float* v, int shift) {
 }
 
 // k contiguous: T threads per row (one wave, or the workgroup for long rows),
-// 8 k per thread and step; the first 4 steps stay in registers between the
-// row's maximum and its conversion, later ones are read twice. HBM-bound:
-// 4 bytes read and 2 per plane written a value.
+// 8 k per thread and step, 4 steps in flight. HBM-bound: 4 bytes read and 2 per
+// plane written a value.
 template <Split F, int T>
 __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ X, int64_t ld,
                                                          int64_t R, int64_t K, int64_t Kp,
                                                          char* __restrict__ out,
-                                                         int64_t row_bytes,
-                                                         uint32_t* __restrict__ amax, int vec) {
+                                                         int64_t row_bytes, int vec) {
   constexpr int NR = 4;
-  __shared__ float red[256 / kWave];
   const int64_t r = (int64_t)blockIdx.x * (256 / T) + threadIdx.x / T;
-  const int t = threadIdx.x % T;
-  const bool live = r < R;
-  const float* x = X + (live ? r : 0) * ld;
-  auto load8 = [&](int64_t k, float* v) {
-    if (vec && k + 8 <= K) {
-      const f32x4 a = *reinterpret_cast<const f32x4*>(x + k);
-      const f32x4 b = *reinterpret_cast<const f32x4*>(x + k + 4);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        v[e] = a[e];
-        v[4 + e] = b[e];
-      }
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = k + e < K ? x[k + e] : 0.f;
-    }
-  };
-  float v[NR][8];
-  int shift = 0;
-  if (live) {
+  if (r >= R) return;
+  const float* x = X + r * ld;
+  char* row = out + r * row_bytes;
+  for (int64_t k0 = 8 * (threadIdx.x % T); k0 < Kp; k0 += 8 * T * NR) {
+    float v[NR][8];
 #pragma unroll
     for (int i = 0; i < NR; ++i) {
-      const int64_t k = 8 * (t + (int64_t)T * i);
-      if (k < Kp) load8(k, v[i]);
-    }
-  }
-  if constexpr (F == Split::kPair) {
-    uint32_t m = 0;  // magnitudes as bits: NaN above infinity above all finite
-    if (live) {
+      const int64_t k = k0 + 8 * T * i;
+      if (k >= Kp) continue;
+      if (vec && k + 8 <= K) {
+        const f32x4 a = *reinterpret_cast<const f32x4*>(x + k);
+        const f32x4 b = *reinterpret_cast<const f32x4*>(x + k + 4);
 #pragma unroll
-      for (int i = 0; i < NR; ++i)
-        if (8 * (t + (int64_t)T * i) < Kp)
+        for (int e = 0; e < 4; ++e) {
+          v[i][e] = a[e];
+          v[i][4 + e] = b[e];
+        }
+      } else {
 #pragma unroll
-          for (int e = 0; e < 8; ++e) m = max(m, __float_as_uint(v[i][e]) & 0x7fffffffu);
-      for (int64_t k = 8 * (t + (int64_t)T * NR); k < Kp; k += 8 * T) {
-        float w[8];
-        load8(k, w);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) m = max(m, __float_as_uint(w[e]) & 0x7fffffffu);
+        for (int e = 0; e < 8; ++e) v[i][e] = k + e < K ? x[k + e] : 0.f;
       }
     }
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o, kWave));
-    if constexpr (T > kWave) {
-      if (threadIdx.x % kWave == 0) red[threadIdx.x / kWave] = __uint_as_float(m);
-      __syncthreads();
-#pragma unroll
-      for (int w = 0; w < 256 / kWave; ++w) m = max(m, __float_as_uint(red[w]));
+    for (int i = 0; i < NR; ++i) {
+      const int64_t k = k0 + 8 * T * i;
+      if (k < Kp) store8<F>(row, k, v[i]);
     }
-    if (live && t == 0) amax[r] = m;
-    shift = scale_shift(m);
-  }
-  if (!live) return;
-  char* row = out + r * row_bytes;
-#pragma unroll
-  for (int i = 0; i < NR; ++i) {
-    const int64_t k = 8 * (t + (int64_t)T * i);
-    if (k < Kp) store8<F>(row, k, v[i], shift);
-  }
-  for (int64_t k = 8 * (t + (int64_t)T * NR); k < Kp; k += 8 * T) {
-    float w[8];
-    load8(k, w);
-    store8<F>(row, k, w, shift);
   }
 }
 
-__global__ __launch_bounds__(256) void zero_u32_kernel(uint32_t* __restrict__ p, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i < n) p[i] = 0;
-}
-
-// The rows [k0, k1) of X behind 64-k block kb of the split operand, and their run.
-__device__ inline int block_rows(int64_t kb, int64_t K, int use_runs, const Runs& runs,
-                                 int64_t& k0, int64_t& k1) {
+// The rows [k0, k1) of X behind 64-k block kb of the split operand.
+__device__ inline void block_rows(int64_t kb, int64_t K, int use_runs, const Runs& runs,
+                                  int64_t& k0, int64_t& k1) {
   k0 = kb * 64;
   k1 = K;
-  if (!use_runs) return 0;
+  if (!use_runs) return;
   int e = 0;
   while (kb >= (runs.cnt[e] + 63) / 64) kb -= (runs.cnt[e++] + 63) / 64;
   k0 = runs.off[e] + kb * 64;
   k1 = runs.off[e] + runs.cnt[e];
-  return e;
-}
-
-// column maxima of X [K][ld], a 64-k block per workgroup; the atomic max of
-// magnitude bits does not depend on the order. Runs have their own maxima: one
-// expert's large or infinite values leave the others' precision alone.
-__global__ __launch_bounds__(256) void col_amax_kernel(const float* __restrict__ X, int64_t ld,
-                                                       int64_t R, int64_t K,
-                                                       uint32_t* __restrict__ amax,
-                                                       int use_runs, Runs runs) {
-  const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (r >= R) return;
-  X += blockIdx.z * K * ld;
-  amax += blockIdx.z * R;
-  int64_t k0, k1;
-  amax += block_rows(blockIdx.y, K, use_runs, runs, k0, k1) * R;
-  k1 = min(k0 + 64, k1);
-  uint32_t m = 0;
-#pragma unroll 8
-  for (int64_t k = k0; k < k1; ++k) m = max(m, __float_as_uint(X[k * ld + r]) & 0x7fffffffu);
-  if (m) atomicMax(amax + r, m);
 }
 
 // k across rows: 64 k x 64 r tiles through LDS; reads are 64 consecutive r a
@@ -211,16 +118,14 @@ template <Split F>
 __global__ __launch_bounds__(256) void split_cols_kernel(const float* __restrict__ X, int64_t ld,
                                                          int64_t R, int64_t K,
                                                          char* __restrict__ out,
-                                                         int64_t row_bytes,
-                                                         const uint32_t* __restrict__ amax,
-                                                         int use_runs, Runs runs) {
+                                                         int64_t row_bytes, int use_runs,
+                                                         Runs runs) {
   __shared__ float t[64][65];  // [k][r]
   const int64_t kb = blockIdx.x, r0 = (int64_t)blockIdx.y * 64;
   X += blockIdx.z * K * ld;
   out += blockIdx.z * R * row_bytes;
-  amax += blockIdx.z * R;
   int64_t k0, k1;
-  amax += block_rows(kb, K, use_runs, runs, k0, k1) * R;
+  block_rows(kb, K, use_runs, runs, k0, k1);
   const int tx = threadIdx.x % 64, ty = threadIdx.x / 64;
 #pragma unroll 4
   for (int i = ty; i < 64; i += 4) {
@@ -235,8 +140,7 @@ __global__ __launch_bounds__(256) void split_cols_kernel(const float* __restrict
     float v[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = t[kl + e][rl];
-    const int shift = F == Split::kPair ? scale_shift(amax[r0 + rl]) : 0;
-    store8<F>(out + (r0 + rl) * row_bytes, kb * 64 + kl, v, shift);
+    store8<F>(out + (r0 + rl) * row_bytes, kb * 64 + kl, v);
   }
 }
 
@@ -246,7 +150,6 @@ struct PairArgs {
   const char *A, *B;
   int64_t rowA, rowB;  // bytes
   int rowsA;
-  const uint32_t *amax, *bmax;
   float* C;
   int64_t ldc;
   int M, N, nst;  // nst: K stages
@@ -284,17 +187,17 @@ template <> struct Products<2, 2> {
 };
 template <> struct Products<1, 1> { static constexpr int n = 1, a[1] = {0}, b[1] = {0}; };
 
-template <bool F16>
 __device__ inline f32x16 mfma(u32x4 a, u32x4 b, f32x16 c) {
-  if constexpr (F16)
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8, a),
-                                                  __builtin_bit_cast(h8, b), c, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
-                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
+                                                 __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-template <bool F16, int PA, int PB, int BM, int BN, int BK, int WM, int WN, Mode MODE>
+// TWO: the products of lower planes, all but hi.hi, are summed apart and added last.
+// An addition rounds at the size of the sum, so five of three planes' six additions
+// then round at 2^-8 of it: at the same time, a third to two thirds of the error
+// against float64 (K 512, 768, 1536: 3.4e-7, 4.2e-7, 6.0e-7 -> 1.3e-7, 1.6e-7, 2.3e-7;
+// K 32768 in 10 splits 6.5e-7 -> 3.8e-7).
+template <int PA, int PB, int BM, int BN, int BK, int WM, int WN, Mode MODE, bool TWO>
 __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_pairs_kernel(PairArgs g) {
   static_assert((PA == 1 || BK == 32) && (PB == 1 || BK == 32), "");
   constexpr int NW = WM * WN;
@@ -311,7 +214,6 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_pairs_kernel(PairArgs g)
 
   int tm, tn, z = 0, M = g.M, s0 = 0, s1 = g.nst, arow0 = 0;
   const char* Bp = g.B;
-  const uint32_t *amax = g.amax, *bmax = g.bmax;
   float* C = g.C;
   if constexpr (MODE == kPlain) {
     const int per = g.ntm * g.ntn;
@@ -329,7 +231,6 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_pairs_kernel(PairArgs g)
     M = g.runs.cnt[e];
     arow0 = g.runs.off[e];
     Bp += (int64_t)e * g.stride * g.rowB;
-    if (F16) bmax += (int64_t)e * g.stride;
     C += (int64_t)arow0 * g.ldc;
   } else {
     const int per = g.ntm * g.ntn, e = blockIdx.x / per;
@@ -338,8 +239,6 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_pairs_kernel(PairArgs g)
     for (int i = 0; i < e; ++i) s0 += (g.runs.cnt[i] + 63) / 64 * (64 / BK);
     s1 = s0 + (g.runs.cnt[e] + 63) / 64 * (64 / BK);
     C += (int64_t)e * g.stride;
-    amax += (int64_t)e * g.M;
-    bmax += (int64_t)e * g.N;
   }
   const int m0 = tm * BM, n0 = tn * BN;
 
@@ -373,13 +272,16 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_pairs_kernel(PairArgs g)
     bt += BK * 2 * PB;
   };
 
-  f32x16 acc[MB][NBk];
+  f32x16 acc[MB][NBk], low[TWO ? MB : 1][TWO ? NBk : 1];
 #pragma unroll
   for (int i = 0; i < MB; ++i)
 #pragma unroll
     for (int j = 0; j < NBk; ++j)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+      for (int e = 0; e < 16; ++e) {
+        acc[i][j][e] = 0.f;
+        if constexpr (TWO) low[i][j][e] = 0.f;
+      }
   // fragment of lane l: row l % 32 of the block, chunk 2 ks + l / 32
   const int fr = lane % 32, fs = swz(fr);  // blocks start at multiples of 32
   const int fa = (wm * (BM / WM) + fr) * CR * 16, fb = (wn * (BN / WN) + fr) * CR * 16;
@@ -423,8 +325,10 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_pairs_kernel(PairArgs g)
 #pragma unroll
         for (int i = 0; i < MB; ++i)
 #pragma unroll
-          for (int j = 0; j < NBk; ++j)
-            acc[i][j] = mfma<F16>(a[ks & 1][Pr::a[q]][i], b[ks & 1][Pr::b[q]][j], acc[i][j]);
+          for (int j = 0; j < NBk; ++j) {
+            f32x16& c = TWO && q + 1 < Pr::n ? low[TWO ? i : 0][TWO ? j : 0] : acc[i][j];
+            c = mfma(a[ks & 1][Pr::a[q]][i], b[ks & 1][Pr::b[q]][j], c);
+          }
       if (ks + 1 < BK / 16) {
         constexpr int nr = PA * MB + PB * NBk, nm = Pr::n * MB * NBk;
 #pragma unroll
@@ -443,19 +347,10 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_pairs_kernel(PairArgs g)
 #pragma unroll
     for (int i = 0; i < MB; ++i) {
       const int rb = m0 + wm * (BM / WM) + i * 32 + 4 * (lane / 32);
-      int sa[16];
-      if constexpr (F16) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int row = rb + 8 * (e / 4) + e % 4;
-          sa[e] = scale_shift(amax[arow0 + (whole ? row : min(row, M - 1))]);
-        }
-      }
 #pragma unroll
       for (int j = 0; j < NBk; ++j) {
         const int col = n0 + wn * (BN / WN) + j * 32 + fr;
         if (!whole && col >= g.N) continue;
-        const int sb = F16 ? scale_shift(bmax[col]) : 0;
         const float bias = g.bias ? g.bias[col] : 0.f;
         float old[16];  // read together: a read behind a write of C waits for it
         if (g.beta != 0.f && !(MODE == kPlain && g.splits > 1)) {
@@ -469,7 +364,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_pairs_kernel(PairArgs g)
         for (int e = 0; e < 16; ++e) {
           const int row = rb + 8 * (e / 4) + e % 4;
           if (!whole && row >= M) continue;
-          const float v = F16 ? ldexpf(acc[i][j][e], -(sa[e] + sb)) : acc[i][j][e];
+          const float v = TWO ? acc[i][j][e] + low[TWO ? i : 0][TWO ? j : 0][e] : acc[i][j][e];
           if (MODE == kPlain && g.splits > 1) {
             g.part[((int64_t)z * M + row) * g.N + col] = v;
             continue;
@@ -501,29 +396,28 @@ __global__ __launch_bounds__(256) void pairs_reduce_kernel(const float* __restri
 
 // ---------------------------------------------------------------- dispatch --
 
-// (the grouped modes take f16 pairs only)
-template <Mode MODE, int BM, int BN, int WM, int WN>
+// (the grouped modes and TWO take three planes only)
+template <Mode MODE, int BM, int BN, int WM, int WN, bool TWO>
 int launch(const SplitOperand& A, const SplitOperand& B, PairArgs& g, int64_t wgs,
            hipStream_t st) {
   if (wgs == 0) return SM_OK;
   SM_REQUIRE(wgs * 512 < ((int64_t)1 << 32) && pairs_fit(A.kp) && A.kp == B.kp,
              "gemm_pairs: shape out of range");
-#define SM_GP(F16, PA, PB, BK) \
-  gemm_pairs_kernel<F16, PA, PB, BM, BN, BK, WM, WN, MODE>  \
+#define SM_GP(PA, PB, BK) \
+  gemm_pairs_kernel<PA, PB, BM, BN, BK, WM, WN, MODE, TWO>  \
       <<<(unsigned)wgs, WM * WN * 64, 0, st>>>(g)
   g.nst = (int)(A.kp / (A.form == Split::kBf16 ? 64 : 32));
-  if constexpr (MODE != kPlain) {
-    SM_GP(true, 2, 2, 32);
-  } else if constexpr (BM * BN <= 256 * 128) {  // (three planes of a larger tile overflow LDS)
-    if (A.form == Split::kBf16x3) {
-      if (B.form == Split::kBf16x3) SM_GP(false, 3, 3, 32);
-      else SM_GP(false, 3, 2, 32);
+  if constexpr (TWO) {
+    SM_GP(3, 3, 32);
+  } else {
+    if constexpr (BM * BN <= 256 * 128) {  // (three planes of a larger tile overflow LDS)
+      if (A.form == Split::kBf16x3) {
+        if (B.form == Split::kBf16x3) SM_GP(3, 3, 32);
+        else SM_GP(3, 2, 32);
+      }
     }
-  }
-  if constexpr (MODE == kPlain) {
-    if (A.form == Split::kBf16x2) SM_GP(false, 2, 2, 32);
-    else if (A.form == Split::kBf16) SM_GP(false, 1, 1, 64);
-    else if (A.form == Split::kPair) SM_GP(true, 2, 2, 32);
+    if (A.form == Split::kBf16x2) SM_GP(2, 2, 32);
+    else if (A.form == Split::kBf16) SM_GP(1, 1, 64);
   }
 #undef SM_GP
   SM_LAUNCH_CHECK();
@@ -537,8 +431,6 @@ PairArgs pair_args(const SplitOperand& A, const SplitOperand& B) {
   g.rowA = A.row_bytes();
   g.rowB = B.row_bytes();
   g.rowsA = (int)A.rows;
-  g.amax = A.amax;
-  g.bmax = B.amax;
   g.alpha = 1.f;
   g.splits = 1;
   return g;
@@ -551,9 +443,9 @@ PairArgs pair_args(const SplitOperand& A, const SplitOperand& B) {
 // a round leaves CUs idle (0.6 of it for the large tiles with few busy, half for
 // the 128 x 128 ones, two of which share a CU). A split writes and reads its
 // partial sums. Three products, us: 8192 x 8192 x 4096 256 x 256 1378, 128 x 256
-// 1493, 128 x 128 1558; 2048 x 2048 x 8184 500, 288, 208 (256 x 256 in 4 splits
-// 197); 1024 x 768 x 32768 128 x 256 in 10 splits 159, 256 x 256 in 8 259, in 21
-// 167. One bf16 product: 4096 x 2048 x 65536 1598, 1350, 1112.
+// 1493, 128 x 128 1558; 2048 x 2048 x 8184 500, 288, 208. Six: 1024 x 768 x 32768 (24
+// tiles of 128 x 256) in 10 splits 291. One bf16 product: 4096 x 2048 x 65536 1598,
+// 1350, 1112.
 struct Tile {
   int bm, bn, slots;  // slots: workgroups the chip runs at once
   double ns1, ns3;
@@ -563,7 +455,7 @@ constexpr Tile kTiles[] = {
 struct Plan {
   int tile, splits;
 };
-Plan pair_plan(Split a, Split b, int64_t M, int64_t N, int64_t K) {
+Plan pair_plan(Split a, Split b, int64_t M, int64_t N, int64_t K, bool split_k) {
   const bool three = a == Split::kBf16x3;
   const double products = !three ? 1.0 : b == Split::kBf16x3 ? 2.0 : 5.0 / 3.0;
   Plan best{0, 1};
@@ -574,8 +466,7 @@ Plan pair_plan(Split a, Split b, int64_t M, int64_t N, int64_t K) {
     const int slots = three ? kCUs : t.slots;  // (three planes: one workgroup's LDS per CU)
     const double half = t.slots / slots;
     for (int s = 1; s <= 32; ++s) {
-      // (bf16 planes: one accumulation chain per output, as in gemm_mfma.hip)
-      if (s > 1 && (!scaled(a) || K / s < 512 || tiles * s > 4 * slots)) break;
+      if (s > 1 && (!split_k || K / s < 512 || tiles * s > 4 * slots)) break;
       const double rounds = (double)ceil_div(tiles * s, slots);
       const double full = tiles * s / (rounds * slots);
       const double part = slots > kCUs ? std::max(0.53, 0.1 + 0.9 * full) : 0.6 + 0.4 * full;
@@ -595,17 +486,12 @@ Plan pair_plan(Split a, Split b, int64_t M, int64_t N, int64_t K) {
 
 bool pairs_fit(int64_t K) { return K <= ((int64_t)1 << 21); }
 
-int64_t split_bytes(Split form, int64_t rows, int64_t K, int64_t runs) {
-  const SplitOperand o = split_place(form, rows, K, nullptr);
-  const int64_t data = ceil_div(rows * o.row_bytes(), 256) * 256;
-  return data + (scaled(form) ? ceil_div(runs * rows * 4, 256) * 256 : 0);
+int64_t split_bytes(Split form, int64_t rows, int64_t K) {
+  return ceil_div(rows * split_place(form, rows, K, nullptr).row_bytes(), 256) * 256;
 }
 
 SplitOperand split_place(Split form, int64_t rows, int64_t K, void* buf) {
-  SplitOperand o{form, static_cast<char*>(buf), nullptr, rows, ceil_div(K, 64) * 64};
-  if (scaled(form))
-    o.amax = reinterpret_cast<uint32_t*>(o.data + ceil_div(rows * o.row_bytes(), 256) * 256);
-  return o;
+  return {form, static_cast<char*>(buf), rows, ceil_div(K, 64) * 64};
 }
 
 namespace {
@@ -617,20 +503,12 @@ int split_fill(const SplitOperand& o, const float* X, int64_t ld, bool kc, int64
     const int vec = ld % 4 == 0 && reinterpret_cast<uintptr_t>(X) % 16 == 0;
     if (o.kp <= 2048)
       split_rows_kernel<F, 64><<<(unsigned)ceil_div(R, 4), 256, 0, st>>>(X, ld, R, K, o.kp,
-                                                                         o.data, rb, o.amax, vec);
+                                                                         o.data, rb, vec);
     else
-      split_rows_kernel<F, 256><<<(unsigned)R, 256, 0, st>>>(X, ld, R, K, o.kp, o.data, rb,
-                                                             o.amax, vec);
+      split_rows_kernel<F, 256><<<(unsigned)R, 256, 0, st>>>(X, ld, R, K, o.kp, o.data, rb, vec);
   } else {
-    if (scaled(F)) {
-      const int64_t n = (runs ? runs->n : 1) * o.rows;
-      zero_u32_kernel<<<(unsigned)ceil_div(n, 256), 256, 0, st>>>(o.amax, n);
-      const dim3 grid((unsigned)ceil_div(R, 256), (unsigned)(o.kp / 64), (unsigned)batch);
-      col_amax_kernel<<<grid, 256, 0, st>>>(X, ld, R, K, o.amax, runs ? 1 : 0,
-                                            runs ? *runs : Runs{});
-    }
     const dim3 grid((unsigned)(o.kp / 64), (unsigned)ceil_div(R, 64), (unsigned)batch);
-    split_cols_kernel<F><<<grid, 256, 0, st>>>(X, ld, R, K, o.data, rb, o.amax,
+    split_cols_kernel<F><<<grid, 256, 0, st>>>(X, ld, R, K, o.data, rb,
                                                runs ? 1 : 0, runs ? *runs : Runs{});
   }
   SM_LAUNCH_CHECK();
@@ -644,13 +522,12 @@ int split_operand(const SplitOperand& o, const float* X, int64_t ld, bool kc, in
   switch (o.form) {
     case Split::kBf16: return split_fill<Split::kBf16>(o, X, ld, kc, K, st, runs, batch);
     case Split::kBf16x2: return split_fill<Split::kBf16x2>(o, X, ld, kc, K, st, runs, batch);
-    case Split::kBf16x3: return split_fill<Split::kBf16x3>(o, X, ld, kc, K, st, runs, batch);
-    default: return split_fill<Split::kPair>(o, X, ld, kc, K, st, runs, batch);
+    default: return split_fill<Split::kBf16x3>(o, X, ld, kc, K, st, runs, batch);
   }
 }
 
 int64_t gemm_pairs_part_floats(Split a, Split b, int64_t M, int64_t N, int64_t K) {
-  const Plan p = pair_plan(a, b, M, N, ceil_div(K, 64) * 64);  // as gemm_pairs sees it
+  const Plan p = pair_plan(a, b, M, N, ceil_div(K, 64) * 64, true);  // as gemm_pairs sees it
   return p.splits == 1 ? 0 : p.splits * M * N;
 }
 
@@ -659,8 +536,8 @@ int gemm_pairs(const SplitOperand& A, const SplitOperand& B, int64_t M, int64_t 
                int64_t part_floats, hipStream_t st) {
   if (M == 0 || N == 0) return SM_OK;
   PairArgs g = pair_args(A, B);
-  Plan p = pair_plan(A.form, B.form, M, N, A.kp);
-  if (!part || p.splits * M * N > part_floats) p.splits = 1;
+  Plan p = pair_plan(A.form, B.form, M, N, A.kp, part != nullptr);
+  if (p.splits * M * N > part_floats) p.splits = 1;
   g.C = C;
   g.ldc = ldc;
   g.M = (int)M;
@@ -673,9 +550,16 @@ int gemm_pairs(const SplitOperand& A, const SplitOperand& B, int64_t M, int64_t 
   g.ntm = (int)ceil_div(M, kTiles[p.tile].bm);
   g.ntn = (int)ceil_div(N, kTiles[p.tile].bn);
   const int64_t wgs = (int64_t)g.ntm * g.ntn * p.splits;
-  if (p.tile == 0) SM_TRY((launch<kPlain, 256, 256, 2, 4>(A, B, g, wgs, st)));
-  else if (p.tile == 1) SM_TRY((launch<kPlain, 128, 256, 2, 4>(A, B, g, wgs, st)));
-  else SM_TRY((launch<kPlain, 128, 128, 2, 2>(A, B, g, wgs, st)));
+  if (part && B.form == Split::kBf16x3) {
+    if (p.tile == 1) SM_TRY((launch<kPlain, 128, 256, 2, 4, true>(A, B, g, wgs, st)));
+    else SM_TRY((launch<kPlain, 128, 128, 2, 4, true>(A, B, g, wgs, st)));
+  } else if (p.tile == 0) {
+    SM_TRY((launch<kPlain, 256, 256, 2, 4, false>(A, B, g, wgs, st)));
+  } else if (p.tile == 1) {
+    SM_TRY((launch<kPlain, 128, 256, 2, 4, false>(A, B, g, wgs, st)));
+  } else {
+    SM_TRY((launch<kPlain, 128, 128, 2, 2, false>(A, B, g, wgs, st)));
+  }
   if (p.splits > 1) {
     pairs_reduce_kernel<<<(unsigned)ceil_div(M * N, 256), 256, 0, st>>>(part, p.splits, M, N, alpha,
                                                                         beta, bias, C, ldc);
@@ -684,11 +568,10 @@ int gemm_pairs(const SplitOperand& A, const SplitOperand& B, int64_t M, int64_t 
   return SM_OK;
 }
 
-namespace {
-// The grouped forms' column tile: 256 from two rounds of workgroups on.
-bool wide_tiles(int64_t tm, int64_t N) { return tm * ceil_div(N, 256) >= 2 * kCUs; }
-}  // namespace
-
+// The grouped forms' tile is 128 x 128 with eight waves: three planes of it fill the
+// CU's LDS, so four waves would be one per SIMD (8 experts of 512 rows, 512 x 1536,
+// forward / backward: 79 / 176 us, with eight 71 / 163; 128 x 256 tiles are within 4 %
+// of it either way from two rounds on).
 int gemm_pairs_rows(const SplitOperand& A, const SplitOperand& B, int64_t bstride, int64_t N,
                     const Runs& runs, float* C, int64_t ldc, hipStream_t st) {
   PairArgs g = pair_args(A, B);
@@ -699,10 +582,8 @@ int gemm_pairs_rows(const SplitOperand& A, const SplitOperand& B, int64_t bstrid
   g.runs = runs;
   int64_t tm = 0;
   for (int i = 0; i < runs.n; ++i) tm += ceil_div(runs.cnt[i], 128);
-  const bool wide = wide_tiles(tm, N);
-  g.ntn = (int)ceil_div(N, wide ? 256 : 128);
-  if (wide) return launch<kRows, 128, 256, 2, 4>(A, B, g, tm * g.ntn, st);
-  return launch<kRows, 128, 128, 2, 2>(A, B, g, tm * g.ntn, st);
+  g.ntn = (int)ceil_div(N, 128);
+  return launch<kRows, 128, 128, 2, 4, true>(A, B, g, tm * g.ntn, st);
 }
 
 int gemm_pairs_ks(const SplitOperand& A, const SplitOperand& B, int64_t M, int64_t N,
@@ -715,11 +596,8 @@ int gemm_pairs_ks(const SplitOperand& A, const SplitOperand& B, int64_t M, int64
   g.stride = cstride;
   g.runs = runs;
   g.ntm = (int)ceil_div(M, 128);
-  const bool wide = wide_tiles(g.ntm * runs.n, N);
-  g.ntn = (int)ceil_div(N, wide ? 256 : 128);
-  const int64_t wgs = (int64_t)runs.n * g.ntm * g.ntn;
-  if (wide) return launch<kKs, 128, 256, 2, 4>(A, B, g, wgs, st);
-  return launch<kKs, 128, 128, 2, 2>(A, B, g, wgs, st);
+  g.ntn = (int)ceil_div(N, 128);
+  return launch<kKs, 128, 128, 2, 4, true>(A, B, g, (int64_t)runs.n * g.ntm * g.ntn, st);
 }
 
 }  // namespace sm

@@ -8,16 +8,12 @@
 
 namespace sm {
 
-// How a split operand holds its values.
-// kBf16: rounded to bf16, one plane (the one-plane policy's operands).
-// kPair: x 2^s = hi + lo, two f16 planes, about 22 significant bits; s from the
-//   row's largest magnitude.
-// kBf16x2, kBf16x3: the leading two or three bf16 planes of x (three: exact).
-enum class Split { kBf16, kPair, kBf16x2, kBf16x3 };
-inline int planes_of(Split f) {
-  return f == Split::kBf16x3 ? 3 : f == Split::kPair || f == Split::kBf16x2 ? 2 : 1;
+// How a split operand holds its values: the leading one, two or three bf16 planes
+// of x (one: rounded to bf16; three: exact).
+enum class Split { kBf16, kBf16x2, kBf16x3 };
+constexpr int planes_of(Split f) {
+  return f == Split::kBf16x3 ? 3 : f == Split::kBf16x2 ? 2 : 1;
 }
-inline bool scaled(Split f) { return f == Split::kPair; }
 
 // Consecutive runs of the grouped forms: run i covers `cnt[i]` rows (or k)
 // from `off[i]` of the dense operand.
@@ -28,16 +24,14 @@ struct Runs {
 };
 
 // op(X) of `rows` rows and K columns in split form, k padded with zeros to whole
-// 64s. `data` and the row maxima live in the caller's buffer of split_bytes()
-// (16-byte aligned).
+// 64s, in the caller's buffer of split_bytes() (16-byte aligned).
 struct SplitOperand {
   Split form;
   char* data;
-  uint32_t* amax;  // bits of each row's largest |x| (the scaled forms; of runs: [run][row])
   int64_t rows, kp;
   int64_t row_bytes() const { return kp * 2 * planes_of(form); }
 };
-int64_t split_bytes(Split form, int64_t rows, int64_t K, int64_t runs = 1);
+int64_t split_bytes(Split form, int64_t rows, int64_t K);
 SplitOperand split_place(Split form, int64_t rows, int64_t K, void* buf);
 
 // Whether K is in the kernel's range (a tile's rows lie within 4 GB).
@@ -45,15 +39,15 @@ bool pairs_fit(int64_t K);
 
 // Fills `o` from X: element (r, k) at X[r * ld + k] (kc) or X[k * ld + r]. With
 // `runs` (not kc), the runs' k follow each other, each padded with zeros to whole
-// 64s and with its own row maxima. With `batch` > 1 (not kc), X holds that many matrices,
+// 64s. With `batch` > 1 (not kc), X holds that many matrices,
 // K * ld apart, whose rows / batch rows each follow each other.
 int split_operand(const SplitOperand& o, const float* X, int64_t ld, bool kc, int64_t K,
                   hipStream_t st, const Runs* runs = nullptr, int64_t batch = 1);
 
 // C = alpha A B^T + beta C (+ bias along n) from split operands: each form with
-// itself, or kBf16x3 with kBf16x2.
-// part (nullable): room for split-K partial sums, part_floats floats; without
-// it, or where it is too small, K is not split.
+// itself, or kBf16x3 with kBf16x2. Without `part`, gemm_planes' sums bit for bit. With
+// it, three planes' sums as exact as they come: the lower planes' products apart from
+// hi.hi, and K split where the plan says so and part_floats are room for the parts.
 int gemm_pairs(const SplitOperand& A, const SplitOperand& B, int64_t M, int64_t N, float alpha,
                float beta, const float* bias, float* C, int64_t ldc, float* part,
                int64_t part_floats, hipStream_t st);

@@ -20,11 +20,11 @@
 // grouped_linear.rs:787).
 //
 // With a workspace (the _ws entries) a projection is one f32-grade launch over
-// all experts on operands split once into scaled f16 pairs (gemm_pairs.hip): a
+// all experts on operands split once into three exact bf16 planes (gemm_pairs.hip): a
 // launch per expert left the chip with one expert's few tiles at a time (24 to
 // 100 workgroups on 256 CUs; the weight gradients, K = an expert's rows, ran on
 // 24-48). 8192 tokens, top-2 of 8 experts, d 512, width 768, forward and
-// backward: 4.81 -> 0.96 ms. Without one, or for products under 2^25 multiply-adds
+// backward: 4.81 -> 1.25 ms. Without one, or for products under 2^25 multiply-adds
 // in all, each expert with rows is one sm_gemm_ex, in expert order.
 #include <algorithm>
 
@@ -75,7 +75,10 @@ int check_counts(const int64_t* counts, int64_t experts, int64_t routes, const c
 }
 
 // The workspace of a projection: the rows, the weights and, in the backward, the
-// two run-padded transposes, all as f16 pairs.
+// two run-padded transposes, all as three exact bf16 planes: a row whose factor in a
+// sum is zero may hold any finite values. (f16 pairs on one power-of-two scale per
+// row or column took half the products but lost the small rows to a large one.)
+constexpr Split kForm = Split::kBf16x3;
 struct GroupedWs {
   void* p;
   int64_t bytes;
@@ -89,17 +92,14 @@ bool grouped_split_sizes(int64_t routes, int64_t d_in, int64_t d_out, int64_t ex
 
 int64_t forward_bytes(int64_t experts, int64_t routes, int64_t d_in, int64_t d_out) {
   if (!grouped_split_sizes(routes, d_in, d_out, experts)) return 0;
-  return split_bytes(Split::kPair, routes, d_in) + split_bytes(Split::kPair, experts * d_out, d_in);
+  return split_bytes(kForm, routes, d_in) + split_bytes(kForm, experts * d_out, d_in);
 }
 
 int64_t backward_bytes(int64_t experts, int64_t routes, int64_t d_in, int64_t d_out) {
   if (!grouped_split_sizes(routes, d_in, d_out, experts)) return 0;
   const int64_t kp = routes + 64 * experts;  // every run padded to whole 64s
-  const int64_t runs = std::min<int64_t>(experts, kMaxRuns);
-  return std::max(split_bytes(Split::kPair, routes, d_out) +
-                      split_bytes(Split::kPair, experts * d_in, d_out),
-                  split_bytes(Split::kPair, d_in, kp, runs) +
-                      split_bytes(Split::kPair, d_out, kp, runs));
+  return std::max(split_bytes(kForm, routes, d_out) + split_bytes(kForm, experts * d_in, d_out),
+                  split_bytes(kForm, d_in, kp) + split_bytes(kForm, d_out, kp));
 }
 
 bool use_split(const GroupedWs& ws, int64_t need) {
@@ -126,7 +126,6 @@ int grouped_rows(const SplitOperand& x, const SplitOperand& w, const int64_t* co
     const Runs r = runs_of(counts, experts, e0, off);
     SplitOperand b = w;
     b.data += e0 * n * w.row_bytes();
-    b.amax += e0 * n;
     SM_TRY(gemm_pairs_rows(x, b, n, n, r, y, n, st));
     off = r.off[r.n - 1] + r.cnt[r.n - 1];
   }
@@ -139,10 +138,10 @@ int grouped_forward(const float* x, const float* w, const int64_t* counts, int64
                     void* stream) {
   if (use_split(ws, forward_bytes(experts, routes, d_in, d_out))) {
     hipStream_t st = as_stream(stream);
-    const SplitOperand a = split_place(Split::kPair, routes, d_in, ws.p);
+    const SplitOperand a = split_place(kForm, routes, d_in, ws.p);
     const SplitOperand b =
-        split_place(Split::kPair, experts * d_out, d_in,
-                    static_cast<char*>(ws.p) + split_bytes(Split::kPair, routes, d_in));
+        split_place(kForm, experts * d_out, d_in,
+                    static_cast<char*>(ws.p) + split_bytes(kForm, routes, d_in));
     SM_TRY(split_operand(a, x, d_in, true, d_in, st));
     SM_TRY(split_operand(b, w, d_out, false, d_in, st, nullptr, experts));
     return grouped_rows(a, b, counts, experts, d_out, y, st);
@@ -165,9 +164,9 @@ int grouped_backward_split(const float* x, const float* w, const float* grad,
                            hipStream_t st) {
   char* at = static_cast<char*>(ws);
   if (grad_x) {
-    const SplitOperand g = split_place(Split::kPair, routes, d_out, at);
-    const SplitOperand b = split_place(Split::kPair, experts * d_in, d_out,
-                                       at + split_bytes(Split::kPair, routes, d_out));
+    const SplitOperand g = split_place(kForm, routes, d_out, at);
+    const SplitOperand b = split_place(kForm, experts * d_in, d_out,
+                                       at + split_bytes(kForm, routes, d_out));
     SM_TRY(split_operand(g, grad, d_out, true, d_out, st));
     SM_TRY(split_operand(b, w, d_out, true, d_out, st));
     SM_TRY(grouped_rows(g, b, counts, experts, d_in, grad_x, st));
@@ -178,9 +177,9 @@ int grouped_backward_split(const float* x, const float* w, const float* grad,
       const Runs r = runs_of(counts, experts, e0, off);
       int64_t kp = 0;
       for (int i = 0; i < r.n; ++i) kp += ceil_div(r.cnt[i], 64) * 64;
-      const SplitOperand a = split_place(Split::kPair, d_in, kp, at);
+      const SplitOperand a = split_place(kForm, d_in, kp, at);
       const SplitOperand b =
-          split_place(Split::kPair, d_out, kp, at + split_bytes(Split::kPair, d_in, kp, r.n));
+          split_place(kForm, d_out, kp, at + split_bytes(kForm, d_in, kp));
       const int64_t rows = r.off[r.n - 1] + r.cnt[r.n - 1] - r.off[0];
       Runs local = r;
       for (int i = 0; i < r.n; ++i) local.off[i] -= r.off[0];

@@ -10,11 +10,11 @@
 // and db (+)= column sums of G, so padded rows of dW and db stay exactly 0.
 // The GEMMs are f32-grade. Small problems, and calls whose workspace holds no
 // more than the chunk's buffers, run sm_gemm_ex. The others split every operand
-// once into scaled f16 pairs (gemm_pairs.hip): the weight and the hidden rows
+// once into its bf16 planes (gemm_pairs.hip): the weight and the hidden rows
 // once per call in each orientation a product reads them, G once per chunk and
 // orientation; dhidden, whose few tiles have K = V, splits K over the chip.
 // MFMA-bound then. Forward and backward at 4096 x 768 x 32768, chunk 1024, with
-// bias: 13.6 -> 4.3 ms, and the gradients' error against float64 2.3e-6 -> 4.8e-7
+// bias: 13.6 -> 5.7 ms, and the gradients' error against float64 2.3e-6 -> 3.8e-7
 // (dhidden, whose sums over V are the longest).
 //
 // Reference: LinearCrossEntropyBackend (summa-llm/src/model/linear_cross_entropy/mod.rs:33-57),
@@ -52,6 +52,12 @@ LceLayout lce_layout(int64_t tokens, int64_t stored, int64_t chunk, bool use_bia
 
 // The split operands and the split-K partial sums behind the chunk's buffers:
 // W [V, d] and W^T [d, V], hidden [tokens, d], and per chunk hidden^T, G and G^T.
+// Three exact bf16 planes each: a vocabulary row or a token whose factor in a sum
+// is zero (padding, a softmax saturated on its target) may hold any finite values,
+// and planes of every element's own leave the others' bits alone. (f16 pairs on one
+// power-of-two scale per row took half the products but lost the small rows to a
+// large one.)
+constexpr Split kForm = Split::kBf16x3;
 struct LceSplit {
   SplitOperand w, wt, h, ht, g, gt;
   float* part;
@@ -72,8 +78,8 @@ LceSplit lce_split(int64_t tokens, int64_t d, int64_t stored, int64_t chunk, siz
   LceSplit l{};
   size_t at = start;
   auto place = [&](int64_t r, int64_t k) {
-    const SplitOperand o = split_place(Split::kPair, r, k, ws + at);
-    at += (size_t)split_bytes(Split::kPair, r, k);
+    const SplitOperand o = split_place(kForm, r, k, ws + at);
+    at += (size_t)split_bytes(kForm, r, k);
     return o;
   };
   l.w = place(stored, d);
@@ -83,13 +89,12 @@ LceSplit lce_split(int64_t tokens, int64_t d, int64_t stored, int64_t chunk, siz
   l.g = place(rows, stored);
   l.gt = place(stored, rows);
   auto parts = [](int64_t m, int64_t n, int64_t k) {
-    return gemm_pairs_part_floats(Split::kPair, Split::kPair, m, n, k);
+    return gemm_pairs_part_floats(kForm, kForm, m, n, k);
   };
   const int64_t last = tokens % rows;  // the last chunk may choose other splits
   for (int64_t r : {rows, last})
     if (r > 0)
-      l.part_floats = std::max({l.part_floats, parts(r, stored, d), parts(r, d, stored),
-                                parts(stored, d, r)});
+      l.part_floats = std::max({l.part_floats, parts(r, d, stored), parts(stored, d, r)});
   l.part = reinterpret_cast<float*>(ws + at);
   l.total = at + lce_align((size_t)l.part_floats * 4);
   return l;
@@ -98,7 +103,6 @@ LceSplit lce_split(int64_t tokens, int64_t d, int64_t stored, int64_t chunk, siz
 // rows [start, start + n) of a row-split operand
 SplitOperand lce_rows(SplitOperand o, int64_t start, int64_t n) {
   o.data += start * o.row_bytes();
-  o.amax += start;
   o.rows = n;
   return o;
 }
@@ -203,7 +207,7 @@ bool lce_use_split(int64_t tokens, int64_t d, int64_t stored, int64_t chunk, siz
 int lce_split_logits(const LceSplit& l, int64_t start, int64_t rows, int64_t stored,
                      const float* bias, float* logits, hipStream_t st) {
   return gemm_pairs(lce_rows(l.h, start, rows), l.w, rows, stored, 1.f, 0.f, bias, logits, stored,
-                    l.part, l.part_floats, st);
+                    nullptr, 0, st);
 }
 
 }  // namespace
@@ -297,9 +301,9 @@ extern "C" int sm_linear_cross_entropy_backward(
     // dhidden[rows] = G . W          ([rows, Vs] x [Vs, d])
     // dW (+)= G^T . hidden[rows]     ([Vs, rows] x [rows, d])
     if (split) {
-      const SplitOperand g = split_place(Split::kPair, rows, stored_vocab, sp.g.data);
-      const SplitOperand gt = split_place(Split::kPair, stored_vocab, rows, sp.gt.data);
-      const SplitOperand ht = split_place(Split::kPair, d, rows, sp.ht.data);
+      const SplitOperand g = split_place(kForm, rows, stored_vocab, sp.g.data);
+      const SplitOperand gt = split_place(kForm, stored_vocab, rows, sp.gt.data);
+      const SplitOperand ht = split_place(kForm, d, rows, sp.ht.data);
       SM_TRY(split_operand(g, logits, stored_vocab, true, stored_vocab, st));
       SM_TRY(split_operand(gt, logits, stored_vocab, false, rows, st));
       SM_TRY(split_operand(ht, hidden + s0 * d, d, false, rows, st));

@@ -1,5 +1,5 @@
-"""The linear head + cross-entropy on split operands (scaled f16 pairs on the
-matrix cores), at the sizes its tiles and K splits meet edges, against float64."""
+"""The linear head + cross-entropy on split operands (three exact bf16 planes on
+the matrix cores), at the sizes its tiles and K splits meet edges, against float64."""
 import pytest
 import torch
 import torch.nn.functional as F
@@ -11,8 +11,8 @@ pytestmark = pytest.mark.gpu
 
 
 def _bound(K):
-    """Relative to sum |a||b|: the pairs' products (2^-22 a factor, lo.lo
-    dropped) and 3 K / 16 f32 additions."""
+    """Relative to sum |a||b|: the plane products left out (below 3 x 2^-24) and
+    half of the 6 K / 16 f32 additions, whose errors have either sign."""
     return 2.0 ** -21 + 2.0 ** -22 + (3 * K / 16 + 2) * 2.0 ** -24
 
 
@@ -56,7 +56,8 @@ def test_split_linear_ce_matches_f64(dev, T, d, V, logical, chunk, bias):
 
 def test_small_workspace_keeps_the_unsplit_path(dev):
     """A workspace with room for the chunk's buffers alone is accepted, and the
-    two paths agree to f32 rounding."""
+    two paths agree: the same plane products in the same order, split once per
+    call or in the K loop (at this K no sum is split)."""
     T, d, V, chunk = 512, 512, 2048, 512
     g = torch.Generator(device=dev).manual_seed(3)
     h = torch.randn(T, d, generator=g, device=dev)
@@ -74,8 +75,7 @@ def test_small_workspace_keeps_the_unsplit_path(dev):
         call("sm_linear_cross_entropy", h.data_ptr(), w.data_ptr(), None, t.data_ptr(), T, d, V, V,
              chunk, 0, loss.data_ptr(), lp.data_ptr(), base, nbytes, st)
         out.append(lp)
-    torch.testing.assert_close(out[0], out[1], rtol=1e-5, atol=1e-5)
-    assert not torch.equal(out[0], out[1])  # two paths ran
+    assert torch.equal(out[0], out[1])
 
 
 def test_split_linear_ce_infinity_and_zero_rows(dev):
@@ -93,3 +93,48 @@ def test_split_linear_ce_infinity_and_zero_rows(dev):
     keep = torch.ones(T, dtype=torch.bool, device=dev)
     keep[[7, 9]] = False
     assert torch.equal(lp[keep], clean[keep])
+
+
+def _f64_grads(h, w, t, logical):
+    logits = (h.double() @ w.double().T)[:, :logical]
+    G = torch.softmax(logits, 1)
+    G[torch.arange(len(t), device=h.device), t.long()] -= 1
+    G /= len(t)
+    return G, G @ w[:logical].double(), G.T @ h.double()
+
+
+@pytest.mark.parametrize("case", ["padded rows", "saturated token", "unlikely row"])
+def test_split_linear_ce_large_values_without_a_gradient(dev, case):
+    """Finite values whose factor in a sum is exactly zero change nothing, however
+    large: vocabulary rows past the logical size, the hidden row of a token whose
+    softmax is saturated on its target, a vocabulary row that no token gives any
+    probability. Against float64, as far as f32 sums of the other terms are off."""
+    T, d, V, logical = 300, 512, 4096, 4000
+    print(f"case split linear ce {case}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(11)
+    h = torch.randn(T, d, generator=g, device=dev)
+    w = torch.randn(V, d, generator=g, device=dev) * 0.02
+    t = torch.randint(0, logical - 1, (T,), generator=g, device=dev, dtype=torch.int32)
+    big = 2.0 ** 40
+    if case == "padded rows":
+        w[logical:] *= big
+    elif case == "saturated token":
+        w[:, :2], w[t[7].long(), 1] = 0.0, 1.0
+        h[7], h[7, 0], h[7, 1] = 0.0, big, 256.0  # its logit 256, the others 0
+    else:  # every token's logit of row logical - 1 is about -2^39
+        h[:, 0] = h[:, 0].abs() + 0.5
+        w[logical - 1] = 0.0
+        w[logical - 1, 0] = -big
+    G, want_h, want_w = _f64_grads(h, w, t, logical)
+    quiet = G.abs() > 0  # the terms with a gradient
+    gh, gw, _ = ops.linear_cross_entropy_backward(h, w, None, t, torch.ones(1, device=dev), logical)
+    # G's own error: that of a logit, doubled (the saturated and unlikely ones are exact)
+    live = torch.where((h.abs().amax(1) < big / 2 ** 20)[:, None], h.double(), 0.0).abs()
+    rows = torch.where((w[:logical].abs().amax(1) < big / 2 ** 20)[:, None],
+                       w[:logical].double(), 0.0).abs()
+    el = 2 * _bound(d) * float((live @ rows.T).amax()) + 2e-6
+    A = G.abs() + torch.nn.functional.one_hot(t.long(), logical) * quiet / T
+    for name, got, want, mag, K in (("hidden", gh, want_h, A @ w[:logical].double().abs(), V),
+                                    ("weight", gw[:logical], want_w, A.T @ h.double().abs(), T)):
+        err = (got.double() - want).abs()
+        assert (err <= (_bound(K) + el) * mag).all(), (name, float((err / (mag + 1e-300)).max()))
