@@ -1078,8 +1078,8 @@ def bench_policy_gemms(args) -> dict:
     """The policy update's largest GEMM shapes at config[2] (one GRPO group:
     8 x 1023 positions, d 2048, F 5632, V 65536; the last group's 4096 scored
     rows for the LM head) through sm_gemm_planes_ws as the prepare runs them
-    (operands whose k is not contiguous transposed into the scratch first,
-    transposes inside the timing; the forward and data-gradient shapes with a
+    (both operands split into their bf16 planes in the scratch first, the
+    splits inside the timing; the forward and data-gradient shapes with a
     fake-quantized B, exact in two bf16 planes, as in the quantized prepare),
     for 3, 2 and 1 bf16 planes. Per shape: the
     event-timed average of 5 calls, algorithmic f32 TF/s (2 M N K) and the
@@ -1103,8 +1103,8 @@ def bench_policy_gemms(args) -> dict:
         "dW_o": (1, 0, d, d, M), "dX_o": (0, 0, M, d, d),
         "fwd_lm_head": (0, 1, R, V, d), "dW_lm_head": (1, 0, V, d, R),
         "dX_lm_head": (0, 0, R, d, V)}
-    need = max(int(L.sm_gemm_planes_scratch_bytes(ta, tb, m, n, k))
-               for ta, tb, m, n, k in shapes.values())
+    need = max(int(L.sm_gemm_planes_split_bytes(3, 0, m, n, k))
+               for _, _, m, n, k in shapes.values())
     scratch = torch.empty(max(need, 16) // 4, device=dev)
     products = {3: 6, 2: 3, 1: 1}  # per f32 product (three planes with a two-plane B: 5)
     res = {}

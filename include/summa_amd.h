@@ -633,18 +633,22 @@ int sm_gemm_mfma(int trans_a, int trans_b, int64_t M, int64_t N, int64_t K, floa
 int sm_gemm_planes(int planes, int trans_a, int trans_b, int64_t M, int64_t N, int64_t K,
                    float alpha, const float* A, int64_t lda, const float* B, int64_t ldb,
                    float beta, float* C, int64_t ldc, void* stream);
-/* sm_gemm_planes with a scratch (16-byte aligned) of at least
- * sm_gemm_planes_scratch_bytes(trans_a, trans_b, M, N, K) bytes: an operand
- * whose k is not contiguous (op(A) of a transposed A, op(B) of an
- * untransposed B) is transposed into it first, so that both operands stream
- * along k (at one plane both operands are converted once into bf16 copies
- * there instead); the result is sm_gemm_planes' bit for bit. A smaller
- * scratch runs sm_gemm_planes as is. b_planes 2 (with planes 3) declares every B value
+/* sm_gemm_planes with a scratch (16-byte aligned); the result is
+ * sm_gemm_planes' bit for bit, whatever its size:
+ * sm_gemm_planes_split_bytes(planes, b_planes, M, N, K) bytes (-1 for a bad
+ *   count): each operand is split once into its bf16 planes, the fastest form
+ *   and the one the policy update runs;
+ * sm_gemm_planes_scratch_bytes(trans_a, trans_b, M, N, K) bytes: at one plane
+ *   the same; at more, an operand whose k is not contiguous (op(A) of a
+ *   transposed A, op(B) of an untransposed B) is transposed first, so that both
+ *   stream along k;
+ * less: sm_gemm_planes as is. b_planes 2 (with planes 3) declares every B value
  * exact in two bf16 planes (value - bf16(value) is itself a bf16, as for a
  * bf16 scale times a 4-bit code): the zero third plane of B is then not
  * multiplied (five plane products instead of six, the same bits); 0 or 3:
  * no such claim. (The policy update's GEMMs run this way.) */
 int64_t sm_gemm_planes_scratch_bytes(int trans_a, int trans_b, int64_t M, int64_t N, int64_t K);
+int64_t sm_gemm_planes_split_bytes(int planes, int b_planes, int64_t M, int64_t N, int64_t K);
 int sm_gemm_planes_ws(int planes, int b_planes, int trans_a, int trans_b, int64_t M, int64_t N,
                       int64_t K, float alpha, const float* A, int64_t lda, const float* B,
                       int64_t ldb, float beta, float* C, int64_t ldc, void* scratch,

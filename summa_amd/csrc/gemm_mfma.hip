@@ -321,15 +321,15 @@ int64_t transpose_scratch_floats(bool ta, bool tb, int64_t M, int64_t N, int64_t
   return (ta ? M * kp : 0) + (tb ? 0 : N * kp);
 }
 
-// scratch for both operands converted once to bf16 (floats; rows rounded up to
-// whole 128-row tiles, the size callers of sm_gemm_planes_ws were told)
+// scratch for both operands converted once to one bf16 plane (floats; rows rounded
+// up to whole 128-row tiles, the size callers of sm_gemm_planes_ws were told)
 int64_t split_scratch_floats(int64_t M, int64_t N, int64_t K) {
   const int64_t Mp = ceil_div(M, kBM) * kBM, Np = ceil_div(N, kBM) * kBM;
   const int64_t Kp = ceil_div(K, 64) * 64;
   return (Mp * Kp + Np * Kp + 1) / 2;
 }
 
-// the most any call needs (the pre-split path runs at one plane)
+// room for the split operands at one plane and for the transposes at any count
 int64_t gemm_planes_scratch_floats(bool ta, bool tb, int64_t M, int64_t N, int64_t K) {
   return std::max(split_scratch_floats(M, N, K), transpose_scratch_floats(ta, tb, M, N, K));
 }
@@ -469,6 +469,13 @@ extern "C" int64_t sm_gemm_planes_scratch_bytes(int trans_a, int trans_b, int64_
                                                 int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   return 4 * sm::gemm_planes_scratch_floats(trans_a != 0, trans_b != 0, M, N, K);
+}
+
+extern "C" int64_t sm_gemm_planes_split_bytes(int planes, int b_planes, int64_t M, int64_t N,
+                                              int64_t K) {
+  if (planes < 1 || planes > 3 || (b_planes != 0 && b_planes != 2 && b_planes != 3)) return -1;
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  return sm::gemm_presplit_scratch_bytes(planes, b_planes, M, N, K);
 }
 
 extern "C" int sm_gemm_planes_ws(int planes, int b_planes, int trans_a, int trans_b, int64_t M,

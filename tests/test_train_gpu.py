@@ -127,11 +127,11 @@ def test_gemm_planes_reduced(dev, planes, ta, tb, M, N, K, pad):
 def test_gemm_planes_scratch_is_bit_exact(dev, planes, ta, tb, M, N, K):
     """sm_gemm_planes_ws equals sm_gemm_planes (the kernel's own plane split
     and transposed loads) bit for bit, with alpha and beta, on each of its
-    paths: a scratch of sm_gemm_planes_scratch_bytes (one plane: both operands
-    converted once into zero-padded bf16 copies, transposed where k is not
-    contiguous; more planes: the transposes below); one only big enough for
-    the transposes of the operands whose k is not contiguous (rows padded to
-    4 floats); none."""
+    paths: a scratch of sm_gemm_planes_split_bytes (both operands split once
+    into their zero-padded planes, transposed where k is not contiguous); one of
+    sm_gemm_planes_scratch_bytes (the same at one plane; more planes: the
+    transposes below); one only big enough for the transposes of the operands
+    whose k is not contiguous (rows padded to 4 floats); none."""
     print(f"case gemm_planes_ws planes={planes} ta={ta} tb={tb} M={M} N={N} K={K}", flush=True)
     g = torch.Generator(device=dev).manual_seed(M + N + K + 4 * ta + 2 * tb)
     a = torch.randn((K, M) if ta else (M, K), generator=g, device=dev)
@@ -143,11 +143,13 @@ def test_gemm_planes_scratch_is_bit_exact(dev, planes, ta, tb, M, N, K):
     trans = 4 * ((M * kp4 if ta else 0) + (0 if tb else N * kp4))
     mp, np_, kp = -(-M // 128) * 128, -(-N // 128) * 128, -(-K // 64) * 64
     assert need == max(4 * ((mp * kp + np_ * kp + 1) // 2), trans)
+    split = int(_lib.lib().sm_gemm_planes_split_bytes(planes, 0, M, N, K))
+    assert split >= 2 * planes * (M + N) * kp
     ref = c0.clone()
     call("sm_gemm_planes", planes, ta, tb, M, N, K, 0.75, a.data_ptr(), a.stride(0), b.data_ptr(),
          b.stride(0), 0.5, ref.data_ptr(), N, st)
-    for nbytes in (need, trans, 0):
-        scratch = torch.full((max(need, 16) // 4,), float("nan"), device=dev)
+    for nbytes in (split, need, trans, 0):
+        scratch = torch.full((max(split, need, 16) // 4,), float("nan"), device=dev)
         out = c0.clone()
         call("sm_gemm_planes_ws", planes, 0, ta, tb, M, N, K, 0.75, a.data_ptr(), a.stride(0),
              b.data_ptr(), b.stride(0), 0.5, out.data_ptr(), N, scratch.data_ptr(), nbytes, st)
@@ -171,7 +173,8 @@ def test_gemm_planes_two_plane_b_is_bit_exact(dev, ta, tb):
     bq = codes * scale  # a bf16 scale times a 4-bit code, exact in f32
     bf = torch.randn(bshape, generator=g, device=dev)
     st = torch.cuda.current_stream().cuda_stream
-    need = int(_lib.lib().sm_gemm_planes_scratch_bytes(ta, tb, M, N, K))
+    need = int(_lib.lib().sm_gemm_planes_split_bytes(3, 3, M, N, K))
+    assert need > int(_lib.lib().sm_gemm_planes_split_bytes(3, 2, M, N, K))
     scratch = torch.empty(max(need, 16) // 4, device=dev)
 
     def run(b, bp, nbytes=need):
@@ -182,9 +185,37 @@ def test_gemm_planes_two_plane_b_is_bit_exact(dev, ta, tb):
     ref = run(bq, 3)
     assert torch.equal(run(bq, 2), ref)  # pre-split planes
     assert torch.equal(run(bq, 2, 0), ref)  # the kernel's own split
+    assert torch.equal(run(bq, 3, 0), ref)
     assert not torch.equal(run(bf, 2), run(bf, 3))
     with pytest.raises(_lib.SummaError, match="b_planes must be"):
         run(bq, 1)
+
+
+# Sizes whose plan takes each tile (gemm_pairs.hip: 256 x 256 at one and two planes,
+# 128 x 256, 128 x 128), ragged in every direction.
+@pytest.mark.parametrize("planes,bp", [(1, 0), (2, 0), (3, 2), (3, 0)])
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0)])
+@pytest.mark.parametrize("M,N,K", [(2000, 2070, 330), (700, 900, 650), (4090, 4070, 270)])
+def test_gemm_planes_split_tiles_are_bit_exact(dev, planes, bp, ta, tb, M, N, K):
+    """The operands split once give the in-loop split's bits on every tile."""
+    print(f"case gemm_planes split planes={planes} bp={bp} ta={ta} tb={tb} {M}x{N}x{K}",
+          flush=True)
+    g = torch.Generator(device=dev).manual_seed(M + planes + bp + ta)
+    a = torch.randn((K, M) if ta else (M, K), generator=g, device=dev)
+    b = torch.randn((N, K) if tb else (K, N), generator=g, device=dev)
+    if bp == 2:  # exact in two planes
+        hi = b.bfloat16().float()
+        b = hi + (b - hi).bfloat16().float()
+    st = torch.cuda.current_stream().cuda_stream
+    nbytes = int(_lib.lib().sm_gemm_planes_split_bytes(planes, bp, M, N, K))
+    scratch = torch.empty(nbytes // 4, device=dev)
+    out = []
+    for n in (0, nbytes):
+        c = torch.zeros(M, N, device=dev)
+        call("sm_gemm_planes_ws", planes, bp, ta, tb, M, N, K, 1.0, a.data_ptr(), a.stride(0),
+             b.data_ptr(), b.stride(0), 0.0, c.data_ptr(), N, scratch.data_ptr(), n, st)
+        out.append(c)
+    assert torch.equal(out[0], out[1])
 
 
 def test_gemm_planes_rejects_bad_count(dev):
