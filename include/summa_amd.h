@@ -70,8 +70,10 @@ int sm_ce_rows(const void* logits, int dtype, const int32_t* targets, int64_t ro
  * Dispatch::linear_cross_entropy_inner calls (mod.rs:73), with the chunked
  * semantics of chunked_loss / chunked_backward (reference.rs:42-159) and
  * fused_loss / fused_backward (gpu.rs:264-426). f32 operands, f32-grade
- * GEMMs (sm_gemm_ex), so [chunk, stored_vocab] f32 logits exist only in the
- * workspace.
+ * GEMMs: sm_gemm_ex or, where that is faster and the workspace has room, the
+ * same plane products over operands split once into three exact bf16 planes
+ * (the backward's dhidden with K split over the chip). [chunk, stored_vocab]
+ * f32 logits exist only in the workspace.
  *
  * hidden [tokens, d] f32, weight [stored_vocab, d] f32 (Burn's [vocab,
  *   hidden] head weight), bias [stored_vocab] f32 (read only when use_bias),
@@ -86,14 +88,25 @@ int sm_ce_rows(const void* logits, int dtype, const int32_t* targets, int64_t ro
  *   [stored_vocab, d] =, grad_bias [stored_vocab] = (when use_bias) the
  *   three gradients of linear_cross_entropy_backward; rows >= logical_vocab
  *   of grad_weight / grad_bias are exactly 0.
- * workspace: sm_linear_cross_entropy_workspace_bytes(...) bytes, 256-byte
- *   aligned (-1 for a bad shape); no call allocates.
+ * workspace: 256-byte aligned, sm_linear_cross_entropy_workspace_bytes(...)
+ *   bytes (-1 for a bad shape) for either call, or
+ *   sm_linear_cross_entropy_forward_workspace_bytes(...) for the loss alone; no
+ *   call allocates. The least that is accepted is 4 (chunk (stored_vocab + 1) +
+ *   tokens) bytes, each of the three parts rounded up to 256, and 256
+ *   stored_vocab more with a bias: the products then run on sm_gemm_ex alone. The
+ *   rest holds the split operands, 6 bytes a value: W^T, hidden^T and G of a
+ *   chunk, W and hidden where the logits read them split, and the partial sums of
+ *   a split K (4096 x 768 x 32768, chunk 1024, bias: 143 MB, 313 for the loss
+ *   alone, 701 for both).
  * Errors (no panic across the ABI): chunk <= 0 ("linear cross-entropy chunk
  *   size must be positive"), tokens == 0 ("linear cross-entropy requires at
  *   least one token"), logical_vocab outside 1..=stored_vocab.
  */
 int64_t sm_linear_cross_entropy_workspace_bytes(int64_t tokens, int64_t d, int64_t stored_vocab,
                                                 int64_t chunk, int use_bias);
+int64_t sm_linear_cross_entropy_forward_workspace_bytes(int64_t tokens, int64_t d,
+                                                        int64_t stored_vocab, int64_t chunk,
+                                                        int use_bias);
 int sm_linear_cross_entropy(const float* hidden, const float* weight, const float* bias,
                             const int32_t* targets, int64_t tokens, int64_t d,
                             int64_t stored_vocab, int64_t logical_vocab, int64_t chunk,

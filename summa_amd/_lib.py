@@ -37,6 +37,7 @@ SIGNATURES: dict[str, tuple] = {
     "sm_last_error": (C.c_char_p, []),
     "sm_ce_rows": (i32, [vp, i32, vp, i64, i64, i64, vp, vp, vp, f32, vp, vp, vp]),
     "sm_linear_cross_entropy_workspace_bytes": (i64, [i64, i64, i64, i64, i32]),
+    "sm_linear_cross_entropy_forward_workspace_bytes": (i64, [i64, i64, i64, i64, i32]),
     "sm_linear_cross_entropy": (i32, [vp, vp, vp, vp, i64, i64, i64, i64, i64, i32, vp, vp, vp,
                                       i64, vp]),
     "sm_linear_cross_entropy_backward": (i32, [vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i32,

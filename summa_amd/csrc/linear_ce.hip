@@ -8,14 +8,13 @@
 // chunk, the row kernel's gradient in place scaled by grad_output / tokens
 // (read on the device), then dhidden[rows] = G . W, dW (+)= G^T . hidden[rows]
 // and db (+)= column sums of G, so padded rows of dW and db stay exactly 0.
-// The GEMMs are f32-grade. Small problems, and calls whose workspace holds no
-// more than the chunk's buffers, run sm_gemm_ex. The others split every operand
-// once into its bf16 planes (gemm_pairs.hip): the weight and the hidden rows
-// once per call in each orientation a product reads them, G once per chunk and
-// orientation; dhidden, whose few tiles have K = V, splits K over the chip.
-// MFMA-bound then. Forward and backward at 4096 x 768 x 32768, chunk 1024, with
-// bias: 13.6 -> 5.7 ms, and the gradients' error against float64 2.3e-6 -> 3.8e-7
-// (dhidden, whose sums over V are the longest).
+// The GEMMs are f32-grade: sm_gemm_ex, or the same plane products over operands that
+// were split once into their bf16 planes (gemm_pairs.hip), where that is the faster
+// one and the workspace has room. The backward's dhidden and dW always are at
+// matrix-core sizes: dhidden's few tiles have K = V, which is split over the chip
+// (4096 x 768 x 32768, chunk 1024, with bias: backward 11.98 -> 4.45 ms, dhidden's
+// error against float64 2.3e-6 -> 3.8e-7). The logits are where their bias then needs
+// no pass of its own or the weight is large (lce_split).
 //
 // Reference: LinearCrossEntropyBackend (summa-llm/src/model/linear_cross_entropy/mod.rs:33-57),
 // chunked_loss / chunked_backward (reference.rs:42-159), fused_loss /
@@ -59,10 +58,12 @@ LceLayout lce_layout(int64_t tokens, int64_t stored, int64_t chunk, bool use_bia
 // large one.)
 constexpr Split kForm = Split::kBf16x3;
 struct LceSplit {
-  SplitOperand w, wt, h, ht, g, gt;
+  bool logits, grads;  // which products run on split operands
+  SplitOperand w, h;   // the logits'
+  SplitOperand wt, ht, g, gt;
   float* part;
   int64_t part_floats;
-  size_t total;
+  size_t forward, total;  // bytes with which the forward, the backward does so
 };
 
 // the products sm_gemm_ex would run on the matrix cores
@@ -72,8 +73,8 @@ bool lce_split_sizes(int64_t rows, int64_t d, int64_t stored) {
          rows * stored * d >= ((int64_t)1 << 27);
 }
 
-LceSplit lce_split(int64_t tokens, int64_t d, int64_t stored, int64_t chunk, size_t start,
-                   char* ws) {
+LceSplit lce_split(int64_t tokens, int64_t d, int64_t stored, int64_t chunk, bool use_bias,
+                   size_t start, char* ws) {
   const int64_t rows = std::min(chunk, tokens);
   LceSplit l{};
   size_t at = start;
@@ -82,12 +83,26 @@ LceSplit lce_split(int64_t tokens, int64_t d, int64_t stored, int64_t chunk, siz
     at += (size_t)split_bytes(kForm, r, k);
     return o;
   };
-  l.w = place(stored, d);
+  l.grads = lce_split_sizes(rows, d, stored);
+  // The split of W pays from about 1024 tokens on, and then through the bias (added
+  // in the epilogue, not by a pass over the logits) or a weight of some 2^27
+  // elements. Forward, split against in-loop, us: with bias 1024 x 768 x 32768 332 /
+  // 355, 4096 x 768 x 32768 1206 / 1413, 4096 x 256 x 4096 134 / 178, but 512 x 1024 x
+  // 32768 252 / 226; without 4096 x 768 x 32768 1192 / 1221, 2048 x 1024 x 32768 812 /
+  // 779, 1024 x 2048 x 65536 1582 / 1638, 4096 x 2048 x 65536 5753 / 6546, but 128 x
+  // 2048 x 65536 481 / 213.
+  l.logits = l.grads && tokens >= 1024 && (use_bias || d * stored >= ((int64_t)1 << 27));
+  if (l.logits) {
+    l.w = place(stored, d);
+    l.h = place(tokens, d);
+  }
+  l.forward = l.total = at;
+  if (!l.grads) return l;
   l.wt = place(d, stored);
-  l.h = place(tokens, d);
   l.ht = place(d, rows);
-  l.g = place(rows, stored);
-  l.gt = place(stored, rows);
+  l.g = split_place(kForm, rows, stored, ws + at);  // G, then G^T in its place
+  l.gt = split_place(kForm, stored, rows, ws + at);
+  at += (size_t)std::max(split_bytes(kForm, rows, stored), split_bytes(kForm, stored, rows));
   auto parts = [](int64_t m, int64_t n, int64_t k) {
     return gemm_pairs_part_floats(kForm, kForm, m, n, k);
   };
@@ -180,10 +195,15 @@ int lce_check(const float* hidden, const float* weight, const float* bias,
   return SM_OK;
 }
 
-// logits of rows [start, start + rows) into the workspace slab (+ bias).
-int lce_logits(const float* hidden, const float* weight, const float* bias, int64_t start,
-               int64_t rows, int64_t d, int64_t stored, int use_bias, float* logits,
-               hipStream_t st) {
+// logits of rows [start, start + rows) into the workspace slab (+ bias), from the
+// split operands where `l` says so (K is not split: where sm_gemm_ex is on the matrix
+// cores, the same bits).
+int lce_logits(const LceSplit& l, const float* hidden, const float* weight, const float* bias,
+               int64_t start, int64_t rows, int64_t d, int64_t stored, int use_bias,
+               float* logits, hipStream_t st) {
+  if (l.logits)
+    return gemm_pairs(lce_rows(l.h, start, rows), l.w, rows, stored, 1.f, 0.f,
+                      use_bias ? bias : nullptr, logits, stored, nullptr, 0, st);
   SM_TRY(sm_gemm_ex(0, 1, rows, stored, d, 1.0f, hidden + start * d, d, weight, d, 0.0f, logits,
                     stored, st));
   if (use_bias) {
@@ -192,22 +212,6 @@ int lce_logits(const float* hidden, const float* weight, const float* bias, int6
     SM_LAUNCH_CHECK();
   }
   return SM_OK;
-}
-
-// Whether the call runs on split operands (placed in `l`): matrix-core sizes
-// and a workspace with room for them.
-bool lce_use_split(int64_t tokens, int64_t d, int64_t stored, int64_t chunk, size_t start,
-                   char* ws, int64_t ws_bytes, LceSplit& l) {
-  if (!lce_split_sizes(std::min(chunk, tokens), d, stored)) return false;
-  l = lce_split(tokens, d, stored, chunk, start, ws);
-  return (size_t)ws_bytes >= l.total;
-}
-
-// The same logits from the split operands.
-int lce_split_logits(const LceSplit& l, int64_t start, int64_t rows, int64_t stored,
-                     const float* bias, float* logits, hipStream_t st) {
-  return gemm_pairs(lce_rows(l.h, start, rows), l.w, rows, stored, 1.f, 0.f, bias, logits, stored,
-                    nullptr, 0, st);
 }
 
 }  // namespace
@@ -220,8 +224,15 @@ extern "C" int64_t sm_linear_cross_entropy_workspace_bytes(int64_t tokens, int64
                                                            int use_bias) {
   if (tokens <= 0 || d <= 0 || stored_vocab <= 0 || chunk <= 0) return -1;
   const size_t n = lce_layout(tokens, stored_vocab, chunk, use_bias != 0).total;
-  if (!lce_split_sizes(std::min(chunk, tokens), d, stored_vocab)) return (int64_t)n;
-  return (int64_t)lce_split(tokens, d, stored_vocab, chunk, n, nullptr).total;
+  return (int64_t)lce_split(tokens, d, stored_vocab, chunk, use_bias != 0, n, nullptr).total;
+}
+
+extern "C" int64_t sm_linear_cross_entropy_forward_workspace_bytes(int64_t tokens, int64_t d,
+                                                                   int64_t stored_vocab,
+                                                                   int64_t chunk, int use_bias) {
+  if (tokens <= 0 || d <= 0 || stored_vocab <= 0 || chunk <= 0) return -1;
+  const size_t n = lce_layout(tokens, stored_vocab, chunk, use_bias != 0).total;
+  return (int64_t)lce_split(tokens, d, stored_vocab, chunk, use_bias != 0, n, nullptr).forward;
 }
 
 extern "C" int sm_linear_cross_entropy(const float* hidden, const float* weight,
@@ -238,19 +249,15 @@ extern "C" int sm_linear_cross_entropy(const float* hidden, const float* weight,
   char* ws = static_cast<char*>(workspace);
   float* logits = reinterpret_cast<float*>(ws + l.logits);
   float* lp = token_logprob ? token_logprob : reinterpret_cast<float*>(ws + l.lp);
-  LceSplit sp{};
-  const bool split = lce_use_split(tokens, d, stored_vocab, chunk, l.total, ws, workspace_bytes,
-                                   sp);
-  if (split) {
+  LceSplit sp = lce_split(tokens, d, stored_vocab, chunk, use_bias != 0, l.total, ws);
+  if ((size_t)workspace_bytes < sp.forward) sp = {};
+  if (sp.logits) {
     SM_TRY(split_operand(sp.w, weight, d, true, d, st));
     SM_TRY(split_operand(sp.h, hidden, d, true, d, st));
   }
   for (int64_t s0 = 0; s0 < tokens; s0 += chunk) {
     const int64_t rows = std::min(chunk, tokens - s0);
-    if (split)
-      SM_TRY(lce_split_logits(sp, s0, rows, stored_vocab, use_bias ? bias : nullptr, logits, st));
-    else
-      SM_TRY(lce_logits(hidden, weight, bias, s0, rows, d, stored_vocab, use_bias, logits, st));
+    SM_TRY(lce_logits(sp, hidden, weight, bias, s0, rows, d, stored_vocab, use_bias, logits, st));
     SM_TRY(sm_ce_rows(logits, SM_F32, targets + s0, rows, stored_vocab, logical_vocab, lp + s0,
                       nullptr, nullptr, 1.0f, nullptr, nullptr, st));
   }
@@ -277,21 +284,17 @@ extern "C" int sm_linear_cross_entropy_backward(
   float* rscale = reinterpret_cast<float*>(ws + l.rscale);
   float* parts = reinterpret_cast<float*>(ws + l.parts);
   const float inv_tokens = (float)(1.0 / (double)tokens);
-  LceSplit sp{};
-  const bool split = lce_use_split(tokens, d, stored_vocab, chunk, l.total, ws, workspace_bytes,
-                                   sp);
-  if (split) {
+  LceSplit sp = lce_split(tokens, d, stored_vocab, chunk, use_bias != 0, l.total, ws);
+  if ((size_t)workspace_bytes < sp.total) sp = {};
+  if (sp.logits) {
     SM_TRY(split_operand(sp.w, weight, d, true, d, st));
-    SM_TRY(split_operand(sp.wt, weight, d, false, stored_vocab, st));
     SM_TRY(split_operand(sp.h, hidden, d, true, d, st));
   }
+  if (sp.grads) SM_TRY(split_operand(sp.wt, weight, d, false, stored_vocab, st));
   for (int64_t s0 = 0; s0 < tokens; s0 += chunk) {
     const int64_t rows = std::min(chunk, tokens - s0);
     const bool first = s0 == 0;
-    if (split)
-      SM_TRY(lce_split_logits(sp, s0, rows, stored_vocab, use_bias ? bias : nullptr, logits, st));
-    else
-      SM_TRY(lce_logits(hidden, weight, bias, s0, rows, d, stored_vocab, use_bias, logits, st));
+    SM_TRY(lce_logits(sp, hidden, weight, bias, s0, rows, d, stored_vocab, use_bias, logits, st));
     fill_scale_kernel<<<(unsigned)ceil_div(rows, 256), 256, 0, st>>>(rscale, rows, grad_output,
                                                                      inv_tokens);
     SM_LAUNCH_CHECK();
@@ -300,15 +303,15 @@ extern "C" int sm_linear_cross_entropy_backward(
                       nullptr, logits, 1.0f, rscale, nullptr, st));
     // dhidden[rows] = G . W          ([rows, Vs] x [Vs, d])
     // dW (+)= G^T . hidden[rows]     ([Vs, rows] x [rows, d])
-    if (split) {
+    if (sp.grads) {
       const SplitOperand g = split_place(kForm, rows, stored_vocab, sp.g.data);
       const SplitOperand gt = split_place(kForm, stored_vocab, rows, sp.gt.data);
       const SplitOperand ht = split_place(kForm, d, rows, sp.ht.data);
       SM_TRY(split_operand(g, logits, stored_vocab, true, stored_vocab, st));
-      SM_TRY(split_operand(gt, logits, stored_vocab, false, rows, st));
-      SM_TRY(split_operand(ht, hidden + s0 * d, d, false, rows, st));
       SM_TRY(gemm_pairs(g, sp.wt, rows, d, 1.f, 0.f, nullptr, grad_hidden + s0 * d, d, sp.part,
                         sp.part_floats, st));
+      SM_TRY(split_operand(gt, logits, stored_vocab, false, rows, st));
+      SM_TRY(split_operand(ht, hidden + s0 * d, d, false, rows, st));
       SM_TRY(gemm_pairs(gt, ht, stored_vocab, d, 1.f, first ? 0.f : 1.f, nullptr, grad_weight, d,
                         sp.part, sp.part_floats, st));
     } else {

@@ -76,7 +76,7 @@ def ce_rows(logits: torch.Tensor, targets: torch.Tensor, logical_vocab: int | No
     return lp, loss, lse
 
 
-def _lce_args(hidden, weight, bias, targets, logical_vocab, chunk_size):
+def _lce_args(hidden, weight, bias, targets, logical_vocab, chunk_size, workspace):
     for t, name in ((hidden, "hidden"), (weight, "weight"), (targets, "targets")):
         _dev(t, name)
     if hidden.dtype != torch.float32 or weight.dtype != torch.float32:
@@ -92,7 +92,7 @@ def _lce_args(hidden, weight, bias, targets, logical_vocab, chunk_size):
         if bias.dtype != torch.float32 or bias.shape != (stored,):
             raise ValueError("bias must be float32 [V]")
     lv = stored if logical_vocab is None else int(logical_vocab)
-    nbytes = int(_lib.lib().sm_linear_cross_entropy_workspace_bytes(
+    nbytes = int(getattr(_lib.lib(), workspace)(
         tokens, d, stored, int(chunk_size), int(bias is not None)))
     ws = torch.empty(max(nbytes, 0) + 256, dtype=torch.uint8, device=hidden.device)
     base = (ws.data_ptr() + 255) // 256 * 256
@@ -108,8 +108,9 @@ def linear_cross_entropy(hidden: torch.Tensor, weight: torch.Tensor, bias, targe
     (linear_cross_entropy_inner, summa-llm/src/model/linear_cross_entropy/mod.rs:33-43,
     reference.rs:42-92). Returns ``loss [1]`` (and the per-token log-probs with
     ``want_logprob``)."""
-    tokens, d, stored, lv, ws, base, nbytes = _lce_args(hidden, weight, bias, targets,
-                                                        logical_vocab, chunk_size)
+    tokens, d, stored, lv, ws, base, nbytes = _lce_args(
+        hidden, weight, bias, targets, logical_vocab, chunk_size,
+        "sm_linear_cross_entropy_forward_workspace_bytes")
     loss = torch.empty(1, dtype=torch.float32, device=hidden.device)
     lp = torch.empty(tokens, dtype=torch.float32, device=hidden.device) if want_logprob else None
     call("sm_linear_cross_entropy", hidden.data_ptr(), weight.data_ptr(), _p(bias),
@@ -125,8 +126,9 @@ def linear_cross_entropy_backward(hidden: torch.Tensor, weight: torch.Tensor, bi
     ``linear_cross_entropy`` for the upstream gradient ``grad_output`` [1]
     (``sm_linear_cross_entropy_backward``; linear_cross_entropy_backward,
     mod.rs:45-57, reference.rs:94-159, gpu.rs:313-426)."""
-    tokens, d, stored, lv, ws, base, nbytes = _lce_args(hidden, weight, bias, targets,
-                                                        logical_vocab, chunk_size)
+    tokens, d, stored, lv, ws, base, nbytes = _lce_args(
+        hidden, weight, bias, targets, logical_vocab, chunk_size,
+        "sm_linear_cross_entropy_workspace_bytes")
     _dev(grad_output, "grad_output")
     go = grad_output.reshape(1).to(torch.float32).contiguous()
     gh = torch.empty_like(hidden)

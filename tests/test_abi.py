@@ -119,6 +119,15 @@ def test_linear_cross_entropy_host_checks():
     assert L.sm_linear_cross_entropy_workspace_bytes(0, 8, 16, 4, 0) == -1
     assert L.sm_linear_cross_entropy_workspace_bytes(4, 8, 16, 4, 1) > 4 * 16 * 4
     ws = 1 << 20
+    # the loss alone: the chunk's buffers, with W and hidden split (6 bytes a value)
+    # for many tokens with a bias; the backward's operands behind them
+    fwd, both = (getattr(L, f"sm_linear_cross_entropy_{n}") for n in
+                 ("forward_workspace_bytes", "workspace_bytes"))
+    assert fwd(0, 8, 16, 4, 0) == -1 and fwd(4, 8, 16, 4, 1) == both(4, 8, 16, 4, 1)
+    least = 1024 * 32768 * 4 + 4096 * 4 + 1024 * 4
+    assert fwd(4096, 768, 32768, 1024, 0) == least
+    assert fwd(4096, 768, 32768, 1024, 1) == least + 64 * 32768 * 4 + 6 * 768 * (32768 + 4096)
+    assert both(4096, 768, 32768, 1024, 0) > least + 6 * 32768 * (768 + 1024)
     st = L.sm_linear_cross_entropy(16, 16, None, 16, 4, 8, 16, 16, 0, 0, 16, None, ws, 1 << 20,
                                    None)
     assert st == -1 and L.sm_last_error().decode() == \

@@ -57,37 +57,42 @@ def test_split_linear_ce_matches_f64(dev, T, d, V, logical, chunk, bias):
 def test_small_workspace_keeps_the_unsplit_path(dev):
     """A workspace with room for the chunk's buffers alone is accepted, and the
     two paths agree: the same plane products in the same order, split once per
-    call or in the K loop (at this K no sum is split)."""
-    T, d, V, chunk = 512, 512, 2048, 512
+    call or in the K loop. The loss alone needs no more than its own query's bytes:
+    the chunk's buffers, and W and hidden in split form where they are read so."""
+    T, d, V, chunk = 1536, 512, 2048, 512
     g = torch.Generator(device=dev).manual_seed(3)
     h = torch.randn(T, d, generator=g, device=dev)
     w = torch.randn(V, d, generator=g, device=dev) * 0.05
+    b = torch.randn(V, generator=g, device=dev) * 0.1
     t = torch.randint(0, V, (T,), generator=g, device=dev, dtype=torch.int32)
     st = torch.cuda.current_stream().cuda_stream
-    full = int(_lib.lib().sm_linear_cross_entropy_workspace_bytes(T, d, V, chunk, 0))
-    least = chunk * V * 4 + 2 * T * 4  # logits, log-probs, row scales: each 256-byte aligned
-    assert full > least
+    full = int(_lib.lib().sm_linear_cross_entropy_workspace_bytes(T, d, V, chunk, 1))
+    loss_only = int(_lib.lib().sm_linear_cross_entropy_forward_workspace_bytes(T, d, V, chunk, 1))
+    # logits, log-probs, row scales, bias-gradient parts: each 256-byte aligned
+    least = chunk * V * 4 + T * 4 + chunk * 4 + 64 * V * 4
+    assert loss_only == least + 6 * d * (V + T) and full > loss_only
     ws = torch.empty(full + 256, dtype=torch.uint8, device=dev)
     base = (ws.data_ptr() + 255) // 256 * 256
     out = []
-    for nbytes in (least, full):
+    for nbytes in (least, loss_only, full):
         loss, lp = torch.empty(1, device=dev), torch.empty(T, device=dev)
-        call("sm_linear_cross_entropy", h.data_ptr(), w.data_ptr(), None, t.data_ptr(), T, d, V, V,
-             chunk, 0, loss.data_ptr(), lp.data_ptr(), base, nbytes, st)
+        call("sm_linear_cross_entropy", h.data_ptr(), w.data_ptr(), b.data_ptr(), t.data_ptr(), T,
+             d, V, V, chunk, 1, loss.data_ptr(), lp.data_ptr(), base, nbytes, st)
         out.append(lp)
-    assert torch.equal(out[0], out[1])
+    assert torch.equal(out[0], out[1]) and torch.equal(out[1], out[2])
 
 
 def test_split_linear_ce_infinity_and_zero_rows(dev):
     """An infinity spoils its own token only; a zero row is exact."""
-    T, d, V = 512, 512, 2048
+    T, d, V = 1024, 512, 2048
     g = torch.Generator(device=dev).manual_seed(4)
     h = torch.randn(T, d, generator=g, device=dev)
     w = torch.randn(V, d, generator=g, device=dev) * 0.05
+    b = torch.zeros(V, device=dev)
     t = torch.randint(0, V, (T,), generator=g, device=dev, dtype=torch.int32)
-    _, clean = ops.linear_cross_entropy(h, w, None, t, want_logprob=True)
+    _, clean = ops.linear_cross_entropy(h, w, b, t, want_logprob=True)
     h[7, 3], h[9] = float("inf"), 0.0
-    _, lp = ops.linear_cross_entropy(h, w, None, t, want_logprob=True)
+    _, lp = ops.linear_cross_entropy(h, w, b, t, want_logprob=True)
     assert not torch.isfinite(lp[7])
     assert abs(float(lp[9]) + torch.log(torch.tensor(float(V)))) < 1e-5
     keep = torch.ones(T, dtype=torch.bool, device=dev)
