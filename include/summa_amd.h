@@ -533,9 +533,11 @@ int sm_swiglu_backward(const void* gate_value, const void* grad, int dtype, int6
  * reference's dispatch seam (GroupedLinearBackend, grouped_linear.rs:23-60;
  * RowPermutationBackend, row_permute.rs:33-41). All f32, f32-grade products
  * (sm_gemm_ex per expert with rows, in expert order; no allocation). The _ws
- * forms take a 16-byte aligned workspace of the queried bytes (0: none is used)
- * and run each projection as one launch over all experts; with a smaller one
- * they are the plain forms.
+ * forms take a 16-byte aligned workspace of the queried bytes and run each
+ * projection as one launch over all experts, on operands split once into three
+ * exact bf16 planes there (6 bytes a value); with a smaller one, and where the
+ * query gives 0 (few experts and small products, which are faster so), they are
+ * the plain forms.
  * counts: HOST array [experts] of the rows per expert, as
  *   grouped_linear_inner takes them (Vec<usize>); they must sum to routes.
  * sm_row_permute: out[i] = input[order[i]] over rows of `cols` elements

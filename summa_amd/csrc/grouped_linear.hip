@@ -24,8 +24,8 @@
 // launch per expert left the chip with one expert's few tiles at a time (24 to
 // 100 workgroups on 256 CUs; the weight gradients, K = an expert's rows, ran on
 // 24-48). 8192 tokens, top-2 of 8 experts, d 512, width 768, forward and
-// backward: 4.81 -> 1.25 ms. Without one, or for products under 2^25 multiply-adds
-// in all, each expert with rows is one sm_gemm_ex, in expert order.
+// backward: 4.81 -> 1.25 ms. Without one, or for few experts and small products
+// (grouped_split_sizes), each expert with rows is one sm_gemm_ex, in expert order.
 #include <algorithm>
 
 #include "common.hpp"
@@ -84,10 +84,23 @@ struct GroupedWs {
   int64_t bytes;
 };
 
+// Whether a projection is one launch over all experts on split operands, or a launch
+// per expert. One launch costs 20 to 30 us forward and 35 to 60 backward however little
+// it does (the splits, and one tile's serial K); the others 4 to 8 us an expert and then
+// their arithmetic, on the FMA units below 2^27 multiply-adds. Forward / backward us,
+// one launch against one per expert: 8 experts of 64 rows, 256 x 256 25 / 35 against 42 /
+// 61, of 2048 rows, 512 x 1536 222 / 501 against 357 / 2107; 6 of 128 rows, 256 x 256 25 /
+// 47 against 28 / 51 (2^25.6 in all); 4 of 512 rows, 256 x 512 28 / 82 against 39 / 87
+// (2^28), of 256 rows 27 / 64 against 26 / 61; 1 of 1024 rows, 512 x 512 32 / 80 against
+// 39 / 122, of 256 rows, 256 x 512 21 / 48 against 7 / 16. Few experts with narrow sides
+// have few tiles for long sums: 4 of 16384 rows, 64 x 128 47 / 812 against 43 / 689.
 bool grouped_split_sizes(int64_t routes, int64_t d_in, int64_t d_out, int64_t experts) {
-  return std::min(d_in, d_out) >= 32 && routes * d_in * d_out >= ((int64_t)1 << 25) &&
-         pairs_fit(d_in) && pairs_fit(d_out) && pairs_fit(routes + 64 * experts) &&
-         experts * std::max(d_in, d_out) < (1 << 30) && experts < (1 << 16);
+  const int64_t narrow = std::min(d_in, d_out), madds = routes * d_in * d_out;
+  if (!pairs_fit(d_in) || !pairs_fit(d_out) || !pairs_fit(routes + 64 * experts) ||
+      experts * std::max(d_in, d_out) >= (1 << 30) || experts >= (1 << 16))
+    return false;
+  return experts >= 6 ? narrow >= 32 && madds >= ((int64_t)1 << 25)
+                      : narrow >= 128 && madds >= ((int64_t)1 << 28);
 }
 
 int64_t forward_bytes(int64_t experts, int64_t routes, int64_t d_in, int64_t d_out) {

@@ -172,3 +172,19 @@ def test_grouped_linear_and_row_permute_host_checks():
     st = L.sm_row_permute(dummy, 0, 4, 8, dummy + 64, dummy, None)
     assert st == -1 and b"must not alias" in L.sm_last_error()
     assert L.sm_row_permute(dummy, 0, 0, 8, dummy + 64, dummy + 4096, None) == 0
+
+
+def test_grouped_linear_workspace_queries():
+    """No workspace where a launch per expert is the faster form (few experts and
+    small products or narrow sides), and three bf16 planes of every operand where
+    one launch is; -1 for a bad shape."""
+    q = _lib.lib().sm_grouped_linear_workspace_bytes
+    assert q(0, 64, 64, 64, 0) == -1 and q(4, 64, 0, 64, 1) == -1
+    for shape in ((1, 32, 1024, 1024), (4, 512, 256, 512), (4, 65536, 64, 128), (8, 64, 64, 128),
+                  (64, 65536, 16, 1024)):
+        assert q(*shape, 0) == 0 and q(*shape, 1) == 0, shape
+    for E, R, i, o in ((8, 512, 256, 256), (1, 9000, 128, 2304), (64, 4096, 64, 128)):
+        assert q(E, R, i, o, 0) == 6 * i * (R + E * o)
+        k = R + 64 * E  # every expert's rows rounded up to whole 64s
+        k = (k + 63) // 64 * 64
+        assert q(E, R, i, o, 1) == max(6 * o * (R + E * i), 6 * k * (i + o))
