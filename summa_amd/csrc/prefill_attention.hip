@@ -31,7 +31,7 @@
 //                Lane (j, h) accumulates dims 8 i + 4 h + 0..3 of query j, so
 //                rescaling needs no cross-lane traffic and stores are 8 bytes.
 // The workgroups that share K and V (a KV head's query heads and row tiles) are
-// consecutive on one XCD, so its L2 reads them from memory once.
+// consecutive on one XCD where there are KV heads for all of them (prefill_map.hpp).
 // 16-query waves on the 16 x 16 x 32 form read every K and V fragment for half as
 // many queries and passed P through LDS: bf16, 32 x 512, 16 / 4 heads of 128: 130 ->
 // 94 us; 64 x 1024 974 -> 644; 128 x 383, 12 heads of 64 137 -> 105.
@@ -43,10 +43,12 @@
 // tensors. The f16 pair keeps P.V at fp32-like precision, so the prefill path
 // matches the decode path's fp32 probabilities; a single bf16 or f16 P costs
 // measurable log-prob accuracy.
+#include <algorithm>
 #include <cmath>
 
 #include "attn_common.hpp"
 #include "common.hpp"
+#include "prefill_map.hpp"
 
 namespace sm {
 namespace {
@@ -80,14 +82,13 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(
   __shared__ __attribute__((aligned(16))) uint16_t ks[2][64 * KP];
   __shared__ __attribute__((aligned(16))) _Float16 vts[2][HD * VP];
 
-  // workgroup -> (KV head of a sequence, its query head and row tile); the row
-  // tiles with the most keys first
-  const int rep = H / KVH, per = rep * nqt;
-  const int xcd = blockIdx.x % 8, wi = blockIdx.x / 8;
-  const int64_t grp = (int64_t)(wi / per) * 8 + xcd;
-  if (grp >= (int64_t)S * KVH) return;  // (uniform per workgroup)
+  // the row tiles with the most keys first
+  const int rep = H / KVH;
+  const PrefillMap map((uint32_t)S * KVH, (uint32_t)rep * nqt);
+  uint32_t grp, place;
+  if (!map.at(blockIdx.y * gridDim.x + blockIdx.x, grp, place)) return;  // (uniform)
   const int s = (int)(grp / KVH), kvh = (int)(grp % KVH);
-  const int qt = nqt - 1 - wi % per / rep, h = kvh * rep + wi % rep;
+  const int qt = nqt - 1 - (int)(place / rep), h = kvh * rep + (int)(place % rep);
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   const int j = lane % 32, hf = lane / 32;
   const int p0 = pos0 ? pos0[s] : 0;
@@ -293,12 +294,17 @@ int attn_prefill_16(const uint16_t* q, const uint16_t* kc, const uint16_t* vc,
     return SM_ERR_UNSUPPORTED;
   }
   const int64_t nqt = ceil_div(L, kRows);
-  const int64_t wgs = ceil_div((int64_t)S * KVH, 8) * 8 * (H / KVH) * nqt;
-  if (wgs >= (int64_t)1 << 24) {
+  const int64_t most = (int64_t)1 << 31;
+  int64_t wgs = most;
+  if ((int64_t)S * KVH < most && (H / KVH) * nqt < most)
+    wgs = PrefillMap((uint32_t)S * KVH, (uint32_t)(H / KVH) * nqt).workgroups();
+  // (a grid dimension holds less than 2^24 workgroups of 256 threads)
+  const int64_t wide = std::min<int64_t>(wgs, (int64_t)1 << 23), tall = ceil_div(wgs, wide);
+  if (wgs >= most) {
     set_error("sm_attn_prefill: problem too large");
     return SM_ERR_UNSUPPORTED;
   }
-  const unsigned grid = (unsigned)wgs;
+  const dim3 grid((unsigned)wide, (unsigned)tall);
   const float scale = 1.0f / sqrtf((float)hd);
   const AttnStrides rows = AttnStrides::rows(L, H, hd);  // [S, L, H, hd]
   const AttnStrides qs = qs_in ? *qs_in : rows, os = os_in ? *os_in : rows;
