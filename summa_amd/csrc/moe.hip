@@ -49,16 +49,16 @@ namespace {
 
 constexpr int kRouterThreads = 512;  // 8 waves: four experts each at E = 32
 constexpr int kRouterLds = 64 * 1024;  // dynamic LDS budget (h rows + logits)
-constexpr int kRouterMaxE = 64;
 
 // One workgroup per TT tokens: their h rows go to LDS (f32), then each of the
 // 8 waves takes experts e = wave, wave + 8, ...: its lanes stream W_r[e] once
-// (coalesced, c = lane + 64 u; for d = 768 and 2048 all of the expert's loads
-// in flight together, else eight) and accumulate the dot products of all TT
-// tokens, reduced across the wave in a fixed order; the router weights are
-// read once per TT tokens instead of once per token. (Four waves walking the
-// experts with eight loads in flight waited one L2 round trip per 512 weights:
-// 31 us per call at config[4].) One
+// (coalesced, c = lane + 64 u, eight loads in flight) and accumulate the dot
+// products of all TT tokens, reduced across the wave in a fixed order; the router
+// weights are read once per TT tokens instead of once per token. 32 experts, d
+// 2048, a call: 14 us at 1024 tokens, 29 at 4096, 51 at 8192, 180 at 32768. (All of an
+// expert's loads in flight at once, for d 768 and 2048, cost the occupancy more than
+// the round trips: 15, 54, 106, 406. The weights staged through LDS for 32 tokens in
+// registers were 43, 50, 183 from 4096 tokens on.) One
 // thread per token then does the strict top-2 scan and the softmax over the
 // pair. Rows past the last token repeat the last token (their results are
 // not stored), so the inner loops carry no per-token branches.
@@ -80,7 +80,7 @@ __device__ inline void top2_of(const float* l, int E, int& i0, int& i1, float& w
   w1 = e1 / (1.f + e1);
 }
 
-template <typename TH, bool PAIR, int TT, bool VEC, int CH = 0>
+template <typename TH, bool PAIR, int TT, bool VEC>
 __global__ __launch_bounds__(kRouterThreads) void router_top2_kernel(
     const TH* __restrict__ h, const float* __restrict__ wr, int64_t tokens, int d, int E,
     float* __restrict__ logits_out, int32_t* __restrict__ top_idx, float* __restrict__ top_w) {
@@ -115,17 +115,7 @@ __global__ __launch_bounds__(kRouterThreads) void router_top2_kernel(
 #pragma unroll
     for (int t = 0; t < TT; ++t) acc[t] = 0.f;
     const float* we = wr + (size_t)e * d;
-    if constexpr (CH > 0) {
-      // d = 64 * CH: every weight load of the expert in flight at once (one
-      // L2 round trip per expert), then the same FMA order as below
-      float w[CH];
-#pragma unroll
-      for (int ch = 0; ch < CH; ++ch) w[ch] = we[ch * kWave + lane];
-#pragma unroll
-      for (int ch = 0; ch < CH; ++ch)
-#pragma unroll
-        for (int t = 0; t < TT; ++t) acc[t] = fmaf(hs[t * d + ch * kWave + lane], w[ch], acc[t]);
-    } else if constexpr (VEC) {
+    if constexpr (VEC) {
       const int chunks = d / kWave;
       int ch = 0;
       for (; ch + 8 <= chunks; ch += 8) {
@@ -175,112 +165,13 @@ __global__ __launch_bounds__(kRouterThreads) void router_top2_kernel(
   }
 }
 
-// The same for many tokens (d = 64 CH): 32 tokens per workgroup, each wave's four
-// rows held in registers (lane: columns 64 u + lane) and every expert's weights
-// staged through LDS once for all of them, two experts deep. With the rows in LDS
-// each FMA needed its own LDS read, and every four tokens re-read all the
-// router weights from L2: 32 experts, 8192 tokens 109 -> 54 us, 65536 861 -> 380. The
-// sums are those of the kernel above, bit for bit.
-constexpr int kRouterRows = 32;
-template <typename TH, bool PAIR, int CH>
-__global__ __launch_bounds__(kRouterThreads) void router_rows_kernel(
-    const TH* __restrict__ h, const float* __restrict__ wr, int64_t tokens, int E,
-    float* __restrict__ logits_out, int32_t* __restrict__ top_idx, float* __restrict__ top_w) {
-  constexpr int D = CH * kWave, TT = 4, NV = (D / 4 + kRouterThreads - 1) / kRouterThreads;
-  __shared__ __attribute__((aligned(16))) float ws[2][D];
-  __shared__ float lg[kRouterRows][kRouterMaxE + 1];
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int64_t t0 = (int64_t)blockIdx.x * kRouterRows;
-  float hv[TT][CH];
-#pragma unroll
-  for (int t = 0; t < TT; ++t) {
-    const int64_t r = min<int64_t>(t0 + wave * TT + t, tokens - 1);
-    const TH* row = h + r * (PAIR ? 2 * D : D) + lane;
-#pragma unroll
-    for (int u = 0; u < CH; ++u) {
-      float v = (float)row[u * kWave];
-      if constexpr (PAIR) v += (float)row[D + u * kWave];
-      hv[t][u] = v;
-    }
-  }
-  float4 next[NV];
-  auto fetch = [&](int e) {
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int c = threadIdx.x + i * kRouterThreads;
-      if (c < D / 4) next[i] = reinterpret_cast<const float4*>(wr + (size_t)e * D)[c];
-    }
-  };
-  auto stage = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int c = threadIdx.x + i * kRouterThreads;
-      if (c < D / 4) reinterpret_cast<float4*>(ws[buf])[c] = next[i];
-    }
-  };
-  fetch(0);
-  stage(0);
-  __syncthreads();
-  for (int e = 0; e < E; ++e) {
-    if (e + 1 < E) fetch(e + 1);
-    float acc[TT] = {};
-#pragma unroll
-    for (int u = 0; u < CH; ++u) {
-      const float w = ws[e & 1][u * kWave + lane];
-#pragma unroll
-      for (int t = 0; t < TT; ++t) acc[t] = fmaf(hv[t][u], w, acc[t]);
-    }
-#pragma unroll
-    for (int t = 0; t < TT; ++t) {
-      const float v = wave_sum(acc[t]);
-      if (lane == 0) lg[wave * TT + t][e] = v;
-    }
-    if (e + 1 < E) stage((e + 1) & 1);  // last read before the previous barrier
-    __syncthreads();
-  }
-  const int n = (int)min<int64_t>(kRouterRows, tokens - t0);
-  if ((int)threadIdx.x < n && top_idx) {
-    const int64_t r = t0 + threadIdx.x;
-    int i0, i1;
-    float w0, w1;
-    top2_of(lg[threadIdx.x], E, i0, i1, w0, w1);
-    top_idx[r * 2] = i0;
-    top_idx[r * 2 + 1] = i1;
-    top_w[r * 2] = w0;
-    top_w[r * 2 + 1] = w1;
-  }
-  if (logits_out)
-    for (int i = threadIdx.x; i < n * E; i += kRouterThreads)
-      logits_out[t0 * E + i] = lg[i / E][i % E];
-}
-
-// Runs router_rows_kernel where it is the faster one: rows that fill its registers
-// and enough tokens for half the chip (one workgroup takes 32 tokens through
-// every expert, 41 us however few there are: 3072 tokens 39 us with the kernel
-// above, 4096 56). At d 1024 it gains nothing (8192 tokens 35 -> 32, 4000 14 -> 18).
-template <typename TH, bool PAIR>
-bool launch_router_rows(const void* h, const float* wr, int64_t tokens, int d, int E, float* lo,
-                        int32_t* idx, float* w, hipStream_t st) {
-  if (tokens < 4096 || d != 32 * kWave || reinterpret_cast<uintptr_t>(wr) % 16 != 0) return false;
-  router_rows_kernel<TH, PAIR, 32><<<(unsigned)ceil_div(tokens, kRouterRows), kRouterThreads, 0,
-                                     st>>>(static_cast<const TH*>(h), wr, tokens, E, lo, idx, w);
-  return true;
-}
-
 template <typename TH, bool PAIR, int TT>
 void launch_router(const void* h, const float* wr, int64_t tokens, int d, int E, float* lo,
                    int32_t* idx, float* w, hipStream_t st) {
   const size_t shmem = (size_t)TT * (d + E) * sizeof(float);
   const unsigned grid = (unsigned)ceil_div(tokens, TT);
   const bool vec = d % kWave == 0 && reinterpret_cast<uintptr_t>(h) % 16 == 0;
-  // (d = 2048 rows hold at most four tokens in the LDS budget: TT <= 4 there)
-  if (TT <= 4 && vec && d == 32 * kWave)
-    router_top2_kernel<TH, PAIR, TT, true, (TT <= 4 ? 32 : 0)><<<grid, kRouterThreads, shmem, st>>>(
-        static_cast<const TH*>(h), wr, tokens, d, E, lo, idx, w);
-  else if (vec && d == 12 * kWave)
-    router_top2_kernel<TH, PAIR, TT, true, 12><<<grid, kRouterThreads, shmem, st>>>(
-        static_cast<const TH*>(h), wr, tokens, d, E, lo, idx, w);
-  else if (vec)
+  if (vec)
     router_top2_kernel<TH, PAIR, TT, true><<<grid, kRouterThreads, shmem, st>>>(
         static_cast<const TH*>(h), wr, tokens, d, E, lo, idx, w);
   else
@@ -291,7 +182,6 @@ void launch_router(const void* h, const float* wr, int64_t tokens, int d, int E,
 template <typename TH, bool PAIR>
 void launch_router_tt(const void* h, const float* wr, int64_t tokens, int d, int E, float* lo,
                       int32_t* idx, float* w, hipStream_t st) {
-  if (launch_router_rows<TH, PAIR>(h, wr, tokens, d, E, lo, idx, w, st)) return;
   // tokens per workgroup: the largest of 8 / 4 / 2 / 1 whose rows fit the LDS budget
   const int64_t row = (int64_t)(d + E) * sizeof(float);
   if (8 * row <= kRouterLds) launch_router<TH, PAIR, 8>(h, wr, tokens, d, E, lo, idx, w, st);
@@ -304,7 +194,6 @@ void launch_router_tt(const void* h, const float* wr, int64_t tokens, int d, int
 // equals the reference's host plan (experts ascending, route ids ascending
 // within one), with the 16- and 128-row tile lists beside it.
 constexpr int kMaxExperts = 64;
-static_assert(kRouterMaxE == kMaxExperts, "");
 constexpr int kPlanSmall = 1024;  // routes per workgroup pass
 
 // Rank of this thread's route among its wave's routes of the same expert (lanes,

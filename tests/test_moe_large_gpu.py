@@ -1,5 +1,5 @@
-"""The MoE layer at prefill and recompute sizes (many tokens): the router over
-staged weights, the three-launch route plan and the grouped projections on the
+"""The MoE layer at prefill and recompute sizes (many tokens): the router, the
+three-launch route plan and the grouped projections on the
 256-row tiles, against the small-batch kernels on slices and numpy."""
 import numpy as np
 import pytest
