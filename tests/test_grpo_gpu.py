@@ -83,3 +83,30 @@ def test_rejections(dev, case, msg):
     with pytest.raises(ops.GrpoValidationError, match=msg):
         ops.grpo_loss_tensor(_t(r, dev), _t(cur, dev), _t(beh, dev), None, _t(mask, dev),
                              0.2, 1e-6, 0.0)
+
+
+# Rollouts longer than the 512 tokens a lane requests at once, ending on either side of
+# them, and more rollouts than waves (a wave's second rollout).
+@pytest.mark.parametrize("B,G,T", [(2, 4, 513), (1, 16, 700), (3, 9, 1024), (1, 2, 1537)])
+@pytest.mark.parametrize("masked,kl", [(True, True), (False, False)])
+def test_matches_oracle_long_rollouts(dev, B, G, T, masked, kl):
+    print(f"case long B={B} G={G} T={T} masked={masked} kl={kl}", flush=True)
+    rng = np.random.default_rng(B * 100 + G + T)
+    cur = rng.normal(-3, 1, (B, G, T)).astype(np.float32)
+    beh = (cur + rng.normal(0, 0.3, (B, G, T))).astype(np.float32)
+    ref = (cur + rng.normal(0, 0.2, (B, G, T))).astype(np.float32) if kl else None
+    r = rng.uniform(0, 1, (B, G)).astype(np.float32)
+    mask = None
+    if masked:
+        ends = rng.integers(1, T + 1, (B, G))
+        ends[0, :2] = 511, 513
+        mask = (np.arange(T) < ends[..., None]).astype(np.float32)
+    c = 0.04 if kl else 0.0
+    out = ops.grpo_loss_batched(_t(r, dev), _t(cur, dev), _t(beh, dev),
+                                None if ref is None else _t(ref, dev),
+                                None if mask is None else _t(mask, dev), 0.2, 1e-6, c)
+    stats, adv, dlp, err = oracle.grpo_loss(r, cur, beh, ref, mask, 0.2, 1e-6, c)
+    assert err == 0
+    np.testing.assert_allclose(out["advantages"].cpu().numpy(), adv, rtol=1e-4, atol=1e-6)
+    np.testing.assert_allclose(out["stats"].cpu().numpy(), stats, rtol=1e-4, atol=1e-7)
+    np.testing.assert_allclose(out["dlp"].cpu().numpy(), dlp, rtol=1e-4, atol=1e-9)
